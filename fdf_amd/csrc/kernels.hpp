@@ -83,11 +83,27 @@ __global__ __launch_bounds__(kBlock) void k_reset_advect(int64_t n, double *__re
 // its 64 lanes busy: a lane whose walk ends takes the next unassigned
 // particle of the chunk (ballot + prefix count), so long and short walks are
 // regrouped instead of idling until the wave's longest walk ends.
+//
+// A walk is a chain of dependent record loads, so its time is iterations times
+// the latency of one load and its evaluation, and a large launch's is the
+// record lines it touches.  In FP64 the steps of a walk are therefore decided
+// on the 128-byte FP32 record (a.filter): where the filter certifies every
+// face (planes_fp32_distances), the reference's FP64 distances have those
+// signs and lie outside the zero band, so the step is the reference's.  The
+// 304-byte FP64 record (3 or 4 lines) is read where the filter certifies the
+// owner, for the weights, and where it certifies nothing.  Lanes wait for that
+// evaluation (ph 2) until kExactGroup of them can make it together: walks end
+// at different iterations, and a wavefront would otherwise pay for the FP64
+// path in nearly every one (groups of 8, 24 and 48 measure alike).
+// 8,388,608 particles moved by up to 1.5 cells an axis in 128x128x256 cells, in
+// random order, FP64: 2.60 -> 1.33 ms (about 9.1 -> 6.3 GB of record lines);
+// 10,000 particles from cell (0,0,0) of 20x20x280: 2.12 -> 0.33 ms.
 // ---------------------------------------------------------------------------
 template <typename R>
 struct LocateArgs {
   GridView g;
   const void *planes;  // CellPlanes64 (FP64) or CellPlanes32 (FP32) per cell
+  const CellPlanes32 *filter;  // FP64: the FP32 records (null: every evaluation is made in FP64)
   int64_t n;
   int64_t chunk;
   const double *pos;
@@ -105,44 +121,85 @@ struct LocateArgs {
   int skip_lost;
 };
 
+// Particles per wavefront: few where the launch would otherwise leave SIMDs
+// idle (each SIMD holds 4 of its wavefronts, 4096 on the chip), 256 where
+// there are enough, so that a wavefront's last, long walks weigh little.
+// 3,000 particles, FP32, call and wait: 63 us at 256 a wavefront, 42 us at 16.
+constexpr int64_t kLocateWaves = 4096;
+inline int64_t locate_chunk(int64_t n) {
+  const int64_t c = (n + kLocateWaves - 1) / kLocateWaves;
+  return c < 16 ? 16 : c > 256 ? 256 : c;
+}
+inline int64_t locate_blocks(int64_t n, int64_t chunk) {
+  const int64_t waves = (n + chunk - 1) / chunk;
+  return (waves * 64 + kBlock - 1) / kBlock;
+}
+constexpr int kExactGroup = 24;
+
 template <typename R, bool EXACT>
-__global__ __launch_bounds__(kBlock) void k_locate(LocateArgs<R> a) {
+__global__ __launch_bounds__(kBlock, 4) void k_locate(LocateArgs<R> a) {
+  __shared__ int32_t shist[64];
+  if (threadIdx.x < 64) shist[threadIdx.x] = 0;
+  __syncthreads();
   const int lane = threadIdx.x & 63;
   const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   const int64_t base = wave * a.chunk;
-  if (base >= a.n) return;
   const int64_t end = base + a.chunk < a.n ? base + a.chunk : a.n;
   int64_t cursor = base;
-  int64_t p = -1;
+  int32_t p = 0;  // n < 2^31
+  int ph = 0;  // 0: no particle, 1: walking, 2: waiting for the FP64 evaluation of its cell
   int ci = 0, cj = 0, ck = 0, steps = 0;
+  int32_t lc = 0;  // ci + IM (cj + JM ck); used only inside the grid
+  const int32_t sj = a.g.IM, sk = a.g.IM * a.g.JM;
   CycleGuard cyc;
   double x[3] = {0.0, 0.0, 0.0};
-  unsigned long long my_iters = 0, my_max = 0, my_fb = 0, my_loc = 0, my_lost = 0;
+  unsigned long long my_iters = 0;
+  unsigned long long my_fb = 0;
+  unsigned my_max = 0, my_loc = 0, my_lost = 0;
   int my_err = 0;
   const unsigned long long lane_mask_lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  // the step of walkingsearch.c:919-946 on certified or FP64 distances
+  auto step = [&](const auto d[6]) {
+    if (d[F_FRONT] < 0) {
+      ck += 1;
+      lc += sk;
+    } else if (d[F_BACK] < 0) {
+      ck -= 1;
+      lc -= sk;
+    }
+    if (d[F_LEFT] < 0) {
+      ci -= 1;
+      lc -= 1;
+    } else if (d[F_RIGHT] < 0) {
+      ci += 1;
+      lc += 1;
+    }
+    if (d[F_BOTTOM] < 0) {
+      cj -= 1;
+      lc -= sj;
+    } else if (d[F_TOP] < 0) {
+      cj += 1;
+      lc += sj;
+    }
+  };
   while (true) {
-    unsigned long long idle = __ballot(p < 0);
+    const unsigned long long idle = __ballot(ph == 0);
     if (idle != 0ull && cursor < end) {
-      if (p < 0) {
-        int64_t q = cursor + __popcll(idle & lane_mask_lt);
+      if (ph == 0) {
+        const int64_t q = cursor + __popcll(idle & lane_mask_lt);
         if (q < end) {
-          const int64_t pq = a.order ? (int64_t)a.order[q] : q;
-          int32_t st = a.status[pq];
-          bool skip = (st == ST_LOCATED) || (a.skip_lost && st == ST_LOST);
-          if (!skip) {
+          const int32_t pq = a.order ? a.order[q] : (int32_t)q;
+          const int32_t st = a.status[pq];
+          int32_t c = a.cell[pq];
+#pragma unroll
+          for (int t = 0; t < 3; ++t) x[t] = a.pos[3 * (int64_t)pq + t];
+          if (!(st == ST_LOCATED || (a.skip_lost && st == ST_LOST))) {
             p = pq;
-            x[0] = a.pos[3 * pq];
-            x[1] = a.pos[3 * pq + 1];
-            x[2] = a.pos[3 * pq + 2];
-            int32_t c = a.cell[pq];
+            ph = 1;
             if (c < 0 && a.guess) c = a.guess[pq];
-            if (c >= 0) {
-              unpack_cell(c, cell_idx(a.g), ci, cj, ck);
-            } else {
-              ci = 0;  // (info.xs, info.ys, info.zs) on one rank, walkingsearch.c:611-616
-              cj = 0;
-              ck = 0;
-            }
+            ci = cj = ck = 0;  // (info.xs, info.ys, info.zs) on one rank, walkingsearch.c:611-616
+            if (c >= 0) unpack_cell(c, cell_idx(a.g), ci, cj, ck);
+            lc = c >= 0 ? c : 0;
             steps = 0;
             cyc = CycleGuard();
           } else if (a.steps_out) {
@@ -152,41 +209,77 @@ __global__ __launch_bounds__(kBlock) void k_locate(LocateArgs<R> a) {
       }
       cursor += __popcll(idle);
     }
-    if (__ballot(p >= 0) == 0ull) {
+    const unsigned long long walking = __ballot(ph == 1);
+    unsigned long long waiting = 0ull;
+    if constexpr (EXACT) waiting = __ballot(ph == 2);
+    if ((walking | waiting) == 0ull) {
       if (cursor >= end) break;
       continue;
     }
-    if (p < 0) continue;
-    // ---- one iteration of the walk (walkingsearch.c:1123-1203) ----
-    steps++;
     bool done = false, located = false;
-    if (ci < 0 || ci >= a.g.IM || cj < 0 || cj >= a.g.JM || ck < 0 || ck >= a.g.KM) {
-      done = true;  // walked outside the global domain: LOST (:1127-1132)
-    } else if (cyc.revisit(pack_cell(ci, cj, ck, a.g.IM, a.g.JM))) {
-      done = true;  // periodic walk: LOST at MAX_TRAVERSAL (:1206-1212)
-      steps = a.max_traversal;
-    } else {
-      R d[6];
-      const bool degenerate = !eval_cell_planes<R, EXACT>(a.planes, a.g, ci, cj, ck, x, a.thresh_scale, d, my_fb);
-      if (degenerate) {
-        my_err = 1;
-        done = true;
-      } else if (point_accepted<R>(d)) {
-        R wv[3];
-        weights_from_distances<R>(d, a.clamp, wv);
-        a.w[3 * p] = wv[0];
-        a.w[3 * p + 1] = wv[1];
-        a.w[3 * p + 2] = wv[2];
-        located = true;
-        done = true;
+    const bool exact_turn = EXACT && (walking == 0ull || __popcll(waiting) >= kExactGroup);
+    if (exact_turn) {
+      if constexpr (EXACT) {
+        if (ph == 2) {
+          ph = 1;
+          R d[6];
+          if (!eval_planes_exact(static_cast<const CellPlanes64 *>(a.planes)[lc], x, d)) {
+            my_err = 1;
+            done = true;
+          } else if (point_accepted<R>(d)) {
+            R wv[3];
+            weights_from_distances<R>(d, a.clamp, wv);
+#pragma unroll
+            for (int t = 0; t < 3; ++t) a.w[3 * (int64_t)p + t] = wv[t];
+            located = true;
+            done = true;
+          } else {
+            step(d);
+            if (steps >= a.max_traversal) done = true;  // MAX_TRAVERSAL (:1206-1212)
+          }
+        }
+      }
+    } else if (ph == 1) {
+      // ---- one iteration of the walk (walkingsearch.c:1123-1203) ----
+      steps++;
+      if (ci < 0 || ci >= a.g.IM || cj < 0 || cj >= a.g.JM || ck < 0 || ck >= a.g.KM) {
+        done = true;  // walked outside the global domain: LOST (:1127-1132)
+      } else if (cyc.revisit(lc)) {
+        done = true;  // periodic walk: LOST at MAX_TRAVERSAL (:1206-1212)
+        steps = a.max_traversal;
+      } else if constexpr (EXACT) {
+        float d[6];
+        // certified: no distance is zero, so the point is inside or beyond a face
+        if (a.filter && planes_fp32_distances(a.filter[lc], x, d) == 0u && !point_accepted<float>(d)) {
+          step(d);
+          if (steps >= a.max_traversal) done = true;
+        } else {
+          ph = 2;
+        }
       } else {
-        step_indices<R>(d, ci, cj, ck);
-        if (steps >= a.max_traversal) done = true;  // MAX_TRAVERSAL (:1206-1212)
+        R d[6];
+        const FilterResult fr = eval_planes_fp32(static_cast<const CellPlanes32 *>(a.planes)[lc], a.g, ci, cj, ck, x,
+                                                 a.thresh_scale, d);
+        my_fb += fr.fallbacks;
+        if (fr.degenerate) {
+          my_err = 1;
+          done = true;
+        } else if (point_accepted<R>(d)) {
+          R wv[3];
+          weights_from_distances<R>(d, a.clamp, wv);
+#pragma unroll
+          for (int t = 0; t < 3; ++t) a.w[3 * (int64_t)p + t] = wv[t];
+          located = true;
+          done = true;
+        } else {
+          step(d);
+          if (steps >= a.max_traversal) done = true;
+        }
       }
     }
     if (done) {
       if (located) {
-        a.cell[p] = pack_cell(ci, cj, ck, a.g.IM, a.g.JM);
+        a.cell[p] = lc;
         a.status[p] = ST_LOCATED;
         my_loc++;
       } else if (!my_err) {
@@ -195,31 +288,38 @@ __global__ __launch_bounds__(kBlock) void k_locate(LocateArgs<R> a) {
         my_lost++;
       }
       if (a.steps_out) a.steps_out[p] = steps;
-      if (a.walk_hist)
-        atomicAdd(&a.walk_hist[(blockIdx.x & (kCounterStripes - 1)) * 64 + (steps < 63 ? steps : 63)], 1ull);
+      if (a.walk_hist) atomicAdd(&shist[steps < 63 ? steps : 63], 1);
       my_iters += steps;
-      my_max = my_max > (unsigned long long)steps ? my_max : (unsigned long long)steps;
-      p = -1;
+      my_max = my_max > (unsigned)steps ? my_max : (unsigned)steps;
+      ph = 0;
     }
   }
   // wave-level reduction of the statistics, one atomic per wave
-  for (int off = 32; off > 0; off >>= 1) {
-    my_iters += __shfl_xor(my_iters, off);
-    unsigned long long om = __shfl_xor(my_max, off);
-    my_max = my_max > om ? my_max : om;
-    my_fb += __shfl_xor(my_fb, off);
-    my_loc += __shfl_xor(my_loc, off);
-    my_lost += __shfl_xor(my_lost, off);
-    my_err |= __shfl_xor(my_err, off);
+  if (base < a.n) {
+    for (int off = 32; off > 0; off >>= 1) {
+      my_iters += __shfl_xor(my_iters, off);
+      const unsigned om = __shfl_xor(my_max, off);
+      my_max = my_max > om ? my_max : om;
+      my_fb += __shfl_xor(my_fb, off);
+      my_loc += __shfl_xor(my_loc, off);
+      my_lost += __shfl_xor(my_lost, off);
+      my_err |= __shfl_xor(my_err, off);
+    }
+    if (lane == 0) {
+      unsigned long long *ctr = counter_stripe(a.counters);
+      atomicAdd(&ctr[C_WALK_ITERS], my_iters);
+      atomicMax(&ctr[C_WALK_MAX], (unsigned long long)my_max);
+      if (my_fb) atomicAdd(&ctr[C_FALLBACKS], my_fb);
+      if (my_loc) atomicAdd(&ctr[C_LOCATED], (unsigned long long)my_loc);
+      if (my_lost) atomicAdd(&ctr[C_LOST], (unsigned long long)my_lost);
+      if (my_err) atomicOr(&ctr[C_ERROR], 1ull);
+    }
   }
-  if (lane == 0) {
-    unsigned long long *ctr = counter_stripe(a.counters);
-    atomicAdd(&ctr[C_WALK_ITERS], my_iters);
-    atomicMax(&ctr[C_WALK_MAX], my_max);
-    atomicAdd(&ctr[C_FALLBACKS], my_fb);
-    atomicAdd(&ctr[C_LOCATED], my_loc);
-    atomicAdd(&ctr[C_LOST], my_lost);
-    if (my_err) atomicOr(&ctr[C_ERROR], 1ull);
+  if (a.walk_hist) {
+    __syncthreads();
+    if (threadIdx.x < 64 && shist[threadIdx.x] > 0)
+      atomicAdd(&a.walk_hist[(blockIdx.x & (kCounterStripes - 1)) * 64 + threadIdx.x],
+                (unsigned long long)shist[threadIdx.x]);
   }
 }
 

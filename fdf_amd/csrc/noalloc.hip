@@ -90,14 +90,13 @@ extern "C" int picgpu_locate_device_noalloc(picgpu_ctx *c, int64_t n, const doub
                      ptr, (int64_t)kScratchWords);
   PG_HIP(hipGetLastError());
   if (n > 0) {
-    const int64_t chunk = 256;  // particles per wavefront, as picgpu_locate
-    const int64_t waves = (n + chunk - 1) / chunk;
-    const int64_t blocks = (waves * 64 + kBlock - 1) / kBlock;
+    const int64_t chunk = locate_chunk(n), blocks = locate_blocks(n, chunk);
     auto launch = [&](auto *tag) -> int {
       using R = std::remove_pointer_t<decltype(tag)>;
       LocateArgs<R> a;
       a.g = GridView{c->coor.as<double>(), c->IM, c->JM, c->KM, 1.0 / c->IM, 1.0 / ((double)c->IM * (double)c->JM)};
       a.planes = c->planes.ptr;
+      a.filter = c->have_filter ? c->filter.as<CellPlanes32>() : nullptr;
       a.n = n;
       a.chunk = chunk;
       a.pos = d_pos;

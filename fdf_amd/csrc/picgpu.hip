@@ -184,7 +184,7 @@ static int finish_grid(picgpu_ctx *c) {
     c->bmax[a] = c->bmax[a] + c->opt.bbox_tolerance;
   }
   c->have_grid = true;
-  c->have_planes = false;
+  c->have_planes = c->have_filter = c->filter_no_memory = false;
   c->have_ucat = false;
   c->eul.have_metrics = c->eul.have_bc = false;
   c->sorted = c->keyed = c->key_ordered = c->compact_pending = false;
@@ -275,7 +275,7 @@ int picgpu_destroy(picgpu_ctx *c) {
                     &c->vel0, &c->cell_count, &c->cell_start, &c->pavg, &c->face[0], &c->face[1], &c->face[2],
                     &c->scan_tmp, &c->counters, &c->mlp_master, &c->mlp_bf16, &c->mlp_adam_m, &c->mlp_adam_v,
                     &c->mlp_grad, &c->mlp_partial, &c->mlp_x, &c->mlp_t, &c->mlp_y, &c->kcount,
-                    &c->kstart[0], &c->kstart[1], &c->kidx[0], &c->kidx[1], &c->kslot, &c->kbase, &c->planes,
+                    &c->kstart[0], &c->kstart[1], &c->kidx[0], &c->kidx[1], &c->kslot, &c->kbase, &c->planes, &c->filter,
                     &c->defer, &c->walk_hist};
   for (DevBuf *b : bufs) b->release();
   c->step_counters.release();
@@ -565,6 +565,21 @@ static int ensure_planes(picgpu_ctx *c) {
   return PICGPU_OK;
 }
 
+// FP64: the FP32 records on which a locate decides the steps of its walks
+// (128 B per cell beside the FP64 records' 304), once per grid.  Without
+// memory for them every evaluation is made in FP64.
+static int ensure_filter(picgpu_ctx *c) {
+  if (c->opt.precision == PICGPU_FP32 || c->have_filter || c->filter_no_memory || c->ncell == 0) return PICGPU_OK;
+  if (c->filter.ensure(sizeof(CellPlanes32) * (size_t)c->ncell) != PICGPU_OK) {
+    c->filter_no_memory = true;
+    return PICGPU_OK;
+  }
+  PG_LAUNCH(c, "cell_filter", nblocks(c->ncell), kBlock, k_cell_planes32, grid_view(c), c->opt.distance_threshold,
+            c->filter.as<CellPlanes32>());
+  c->have_filter = true;
+  return PICGPU_OK;
+}
+
 static int build_key_index(picgpu_ctx *c, const int32_t *guess = nullptr);
 
 // An FP64 locate of at least this many particles from guessed start cells
@@ -581,6 +596,7 @@ static int do_locate(picgpu_ctx *c, int skip_lost) {
   PG_CHECK(need_grid(c));
   PG_CHECK(settle_swarm(c));
   PG_CHECK(ensure_planes(c));
+  PG_CHECK(ensure_filter(c));
   PG_CHECK(counters_reset(c));
   const int64_t n = c->n;
   if (n > 0) {
@@ -608,14 +624,13 @@ static int do_locate(picgpu_ctx *c, int skip_lost) {
       if (c->n_live == n) order = c->kidx[c->kcur].as<int32_t>();
     }
     unsigned long long *hist = hist_reset(c);
-    const int64_t chunk = 256;  // particles per wavefront
-    const int64_t waves = (n + chunk - 1) / chunk;
-    const int64_t blocks = (waves * 64 + kBlock - 1) / kBlock;
+    const int64_t chunk = locate_chunk(n), blocks = locate_blocks(n, chunk);
     int r = dispatch_real(c, [&](auto *tag) -> int {
       using R = std::remove_pointer_t<decltype(tag)>;
       LocateArgs<R> a;
       a.g = grid_view(c);
       a.planes = c->planes.ptr;
+      a.filter = c->have_filter ? c->filter.as<CellPlanes32>() : nullptr;
       a.n = n;
       a.chunk = chunk;
       a.pos = c->sw.pos.as<double>();

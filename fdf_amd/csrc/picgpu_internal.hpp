@@ -113,6 +113,8 @@ struct picgpu_ctx {
   double bmin[3] = {0, 0, 0}, bmax[3] = {0, 0, 0};
   picgpu::DevBuf planes;  // [ncell] CellPlanes64 (FP64) or CellPlanes32 (FP32)
   bool have_planes = false;
+  picgpu::DevBuf filter;  // FP64: [ncell] CellPlanes32 for the walk steps of a locate
+  bool have_filter = false, filter_no_memory = false;
 
   // Eulerian fields
   bool have_ucat = false;
