@@ -1289,24 +1289,27 @@ __global__ __launch_bounds__(kBlock) void k_step_finish(StepArgs<R> a, const int
 // Faces between two tiles: the lower cell's sum (hi) plus the upper cell's
 // (lo).  Entries are numbered i-seams, then j-seams, then k-seams; there are
 // fewer than half as many as cells, so 32-bit indices (and divisions) hold.
+struct SeamCounts {
+  int32_t ni, nj, nk;
+  __host__ __device__ int64_t total() const { return (int64_t)ni + nj + nk; }
+};
 template <typename R>
-__global__ __launch_bounds__(kBlock) void k_face_seams(int IM, int JM, int KM, int32_t ni, int32_t nj, int32_t nk,
-                                                       FaceOut<R> fo) {
-  int32_t q = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
+__device__ __forceinline__ void face_seam(int IM, int JM, int KM, const SeamCounts &sc, const FaceOut<R> &fo,
+                                          int32_t q) {
   int d, i, j, k;
-  if (q < ni) {
+  if (q < sc.ni) {
     d = 0;
     j = q % JM;
     const int32_t r = q / JM;
     k = r % KM;
     i = (r / KM + 1) * TX;
-  } else if ((q -= ni) < nj) {
+  } else if ((q -= sc.ni) < sc.nj) {
     d = 1;
     i = q % IM;
     const int32_t r = q / IM;
     k = r % KM;
     j = (r / KM + 1) * TY;
-  } else if ((q -= nj) < nk) {
+  } else if ((q -= sc.nj) < sc.nk) {
     d = 2;
     i = q % IM;
     const int32_t r = q / IM;
@@ -1321,15 +1324,35 @@ __global__ __launch_bounds__(kBlock) void k_face_seams(int IM, int JM, int KM, i
   const auto vh = load4<R>(hi), vl = load4<R>(lo);
   store4<R>(face + 4 * f, vh.x + vl.x, vh.y + vl.y, vh.z + vl.z, vh.w + vl.w);
 }
+template <typename R>
+__global__ __launch_bounds__(kBlock) void k_face_seams(int IM, int JM, int KM, SeamCounts sc, FaceOut<R> fo) {
+  face_seam<R>(IM, JM, KM, sc, fo, (int32_t)(blockIdx.x * blockDim.x + threadIdx.x));
+}
 
 // Particles deferred by k_step_tiled, stepped from their start state with the
-// FP64 routine for uncertified faces (a grid-stride loop over the list).
+// FP64 routine for uncertified faces: workgroups [0, dblocks), whose W
+// wavefronts take entry w, w + W, ... of the list in lane 0, 1, ....  A few
+// thousand entries among 4096 wavefronts leave one or two busy lanes in each:
+// a wavefront pays for every face that any of its lanes recomputes and for
+// its longest walk, one after another.  The workgroups after those add the
+// seam halves of a step that deposits: the deferred particles are a chain of
+// cache misses that leaves the chip idle, the seams a stream of memory, and
+// neither reads what the other writes.
+// 16.8M particles in 128x128x512 cells, FP32: 75 us in 64-lane order and 59
+// for the seams in a launch of their own, 64 us together; 262,144 particles:
+// 21.7 and 5.2 us, 16.4 together.
 template <typename R, bool EXACT, bool RK2>
-__global__ __launch_bounds__(kBlock) void k_step_deferred(StepArgs<R> a) {
-  const int64_t nd = *a.defer_count;
+__global__ __launch_bounds__(kBlock) void k_step_deferred(StepArgs<R> a, int dblocks, SeamCounts sc) {
+  if ((int)blockIdx.x >= dblocks) {
+    face_seam<R>(a.g.IM, a.g.JM, a.g.KM, sc, a.fo, (int32_t)((blockIdx.x - dblocks) * blockDim.x + threadIdx.x));
+    return;
+  }
+  const int32_t nd = *a.defer_count;
+  const int32_t waves = dblocks * (kBlock / 64), w = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+  if (w >= nd) return;
   StepTally tally;
   const PlaneSrc<R, false> src{a.g, a.corner, (const typename PlanesOf<R>::type *)a.planes, nullptr, 0, 0, 0};
-  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < nd; q += (int64_t)gridDim.x * blockDim.x) {
+  for (int64_t q = w + (int64_t)waves * (threadIdx.x & 63); q < nd; q += (int64_t)waves * 64) {
     const int64_t p = a.defer_list[q];
     PState<R> ps;
     load_state(a, p, ps);
@@ -1456,23 +1479,44 @@ __global__ __launch_bounds__(kBlock) void k_iota(int64_t n, const int32_t *__res
 // cell, are insertion-sorted in place.  The PIDs are read as T: the 32-bit
 // copy pid32 when every PID lies in [0, 2^31) (*wide == 0; the same order,
 // half the bytes), the 64-bit pid otherwise.
-template <typename T>
+//
+// With CELLS the thread also averages P over its bucket, in that order, into
+// its cell's pavg (interpolation.c:1838-2036): the bucket's entries are in
+// registers, and a pass over the cells of its own would read the index again.
+// FP64: 10 + 7.5 us in two launches, 15 in one at 400,000 particles in
+// 48x48x250 cells; 9.0 + 6.1, 13.3 at 500,000 in 64x64x96.
+template <typename T, typename R, bool CELLS>
 __device__ __forceinline__ void bucket_pid_order(int32_t s, int32_t e, int32_t *__restrict__ idx,
-                                                 const T *__restrict__ pid) {
+                                                 const T *__restrict__ pid, const R *__restrict__ P, Acc<R> &acc) {
   const int32_t L = e - s;
   if (L <= 8) {
-    int32_t q[8];
+    int32_t q[8], rank[8];
     T v[8];
+    R val[8];
 #pragma unroll
     for (int t = 0; t < 8; ++t) q[t] = t < L ? idx[s + t] : 0;
 #pragma unroll
-    for (int t = 0; t < 8; ++t) v[t] = t < L ? pid[q[t]] : (sizeof(T) == 4 ? (T)INT32_MAX : (T)INT64_MAX);
+    for (int t = 0; t < 8; ++t) {
+      v[t] = t < L ? pid[q[t]] : (sizeof(T) == 4 ? (T)INT32_MAX : (T)INT64_MAX);
+      if constexpr (CELLS) val[t] = t < L ? P[q[t]] : (R)0;
+    }
 #pragma unroll
     for (int a = 0; a < 8; ++a) {
       int r = 0;
 #pragma unroll
       for (int b = 0; b < 8; ++b) r += (v[b] < v[a] || (v[b] == v[a] && b < a)) ? 1 : 0;
+      rank[a] = r;
       if (a < L && r != a) idx[s + r] = q[a];  // entries already in place are not rewritten
+    }
+    if constexpr (CELLS) {
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        if (t >= L) break;
+        R x = val[0];
+#pragma unroll
+        for (int a = 1; a < 8; ++a) x = rank[a] == t ? val[a] : x;
+        acc.add(x);
+      }
     }
     return;
   }
@@ -1486,20 +1530,38 @@ __device__ __forceinline__ void bucket_pid_order(int32_t s, int32_t e, int32_t *
     }
     idx[u + 1] = x;
   }
+  if constexpr (CELLS)
+    for (int32_t t = s; t < e; ++t) acc.add(P[idx[t]]);
 }
+template <typename R, bool CELLS>
 __global__ __launch_bounds__(kBlock) void k_bucket_pid_order(int64_t nkeys, const int32_t *__restrict__ kstart,
                                                              int32_t *__restrict__ idx,
                                                              const int64_t *__restrict__ pid,
                                                              const int32_t *__restrict__ pid32,
-                                                             const int32_t *__restrict__ wide) {
+                                                             const int32_t *__restrict__ wide, int IM, int JM, int KM,
+                                                             TileMap tm, const R *__restrict__ P,
+                                                             R *__restrict__ avg) {
   const int64_t key = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (key >= nkeys) return;
   const int32_t s = kstart[key], e = kstart[key + 1];
-  if (e - s < 2) return;
-  if (*wide == 0)
-    bucket_pid_order<int32_t>(s, e, idx, pid32);
-  else
-    bucket_pid_order<int64_t>(s, e, idx, pid);
+  Acc<R> acc;
+  if (e - s == 1) {
+    if constexpr (CELLS) acc.add(P[idx[s]]);
+  } else if (e - s > 1) {
+    if (*wide == 0)
+      bucket_pid_order<int32_t, R, CELLS>(s, e, idx, pid32, P, acc);
+    else
+      bucket_pid_order<int64_t, R, CELLS>(s, e, idx, pid, P, acc);
+  }
+  if constexpr (CELLS) {
+    const int t = (int)(key / TS), l = (int)(key % TS);
+    const int i = t % tm.NTI * TX + l % TX, j = t / tm.NTI % tm.NTJ * TY + l / TX % TY,
+              k = t / (tm.NTI * tm.NTJ) * TZ + l / (TX * TY);
+    if (i < IM && j < JM && k < KM) {
+      const R cnt = (R)(e - s);
+      avg[(int64_t)i + (int64_t)IM * (j + (int64_t)JM * k)] = cnt > (R)0.5 ? acc.value() / cnt : (R)0;
+    }
+  }
 }
 
 // Face deposition (no reference counterpart).  A particle in cell (i,j,k)
@@ -1694,24 +1756,6 @@ __global__ __launch_bounds__(kBlock, sizeof(R) == 4 ? 6 : 1) void k_deposit_tile
 #pragma unroll
     for (int v = 0; v < 4; ++v) out[d][v] = lower[d][v] + acc[d][v].value();
   }
-}
-
-// P average per cell through the keyed index (buckets in PID order)
-template <typename R>
-__global__ __launch_bounds__(kBlock) void k_scatter_P_keyed(int IM, int JM, int KM, TileMap tm,
-                                                            const int32_t *__restrict__ kstart,
-                                                            const int32_t *__restrict__ idx, const R *__restrict__ P,
-                                                            R *__restrict__ avg) {
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= (int64_t)IM * JM * KM) return;
-  int i, j, k;
-  unpack_cell((int32_t)c, IM, JM, i, j, k);
-  const int32_t key = cell_key(tm, i, j, k);
-  const int32_t s = kstart[key], e = kstart[key + 1];
-  Acc<R> acc;
-  for (int32_t t = s; t < e; ++t) acc.add(P[idx[t]]);
-  const R cnt = (R)(e - s);
-  avg[c] = cnt > (R)0.5 ? acc.value() / cnt : (R)0;
 }
 
 // per-cell counts from the keyed histogram

@@ -328,14 +328,30 @@ __global__ __launch_bounds__(kBlock, 4) void k_locate(LocateArgs<R> a) {
 // valid cells (i-1..i, j-1..j, k-1..k), summed dk, dj, di in that nesting.
 // ucat is compact [KM][JM][IM][3].
 //
-// A thread takes the node column (i, j) over kC2CChunk consecutive k (grid:
-// x over columns, y over chunks of k).  The four cells of plane k that node k
-// sums last are the four that node k+1 sums first, so each node loads four
-// cells, not eight; the next plane is requested while a node is summed.
+// A thread takes the node column (i, j) over `chunk` consecutive k (grid: x
+// over columns, y over chunks of k).  The four cells of plane k that node k
+// sums last are the four that node k+1 sums first, so a long chunk loads four
+// cells a node, not eight; the next plane is requested while a node is summed.
 // Neighbouring threads take neighbouring i, so loads and stores are
-// contiguous.
+// contiguous.  A chunk is a serial chain of loads, so its length is cut
+// (c2c_chunk) until the launch has kC2CWaves wavefronts: the reloaded planes
+// come from L2.
+// Chunks of 32 planes -> cut: 20x20x280 FP64 29.6 -> 5.3 us, 48x48x250 FP64
+// 36 -> 10.5 us, 61x45x131 FP32 28.7 -> 5.9 us; 128x128x512 FP32 keeps 32
+// planes, 53 us (201 MB at 3.8 TB/s).
+//
+// zero [nzero] is cleared by the same launch (the counters and the key
+// histogram of the fused step that follows), which saves that step two fill
+// launches of about 4 us.
 // ---------------------------------------------------------------------------
 constexpr int kC2CChunk = 32;
+constexpr int64_t kC2CWaves = 4096;
+inline int c2c_chunk(int64_t columns, int64_t planes) {
+  const int64_t waves = (columns + 63) / 64;
+  int chunk = kC2CChunk;
+  while (chunk > 1 && waves * ((planes + chunk - 1) / chunk) < kC2CWaves) chunk /= 2;
+  return chunk;
+}
 
 // the cells (i-1,j-1), (i,j-1), (i-1,j), (i,j) of plane ck (the (dj, di)
 // order of the sum); v[c] false for a cell outside the grid
@@ -358,8 +374,12 @@ __device__ __forceinline__ void c2c_plane(int IM, int JM, int KM, const R *__res
 }
 
 template <typename R>
-__global__ __launch_bounds__(kBlock) void k_center_to_corner(int IM, int JM, int KM, const R *__restrict__ ucat,
-                                                             R *__restrict__ corner) {
+__global__ __launch_bounds__(kBlock) void k_center_to_corner(int IM, int JM, int KM, int chunk,
+                                                             const R *__restrict__ ucat, R *__restrict__ corner,
+                                                             int32_t *__restrict__ zero, int64_t nzero) {
+  for (int64_t q = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x; q < nzero;
+       q += (int64_t)gridDim.x * gridDim.y * blockDim.x)
+    zero[q] = 0;
   const uint32_t col = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t nI = (uint32_t)IM + 1u;
   if (col >= nI * ((uint32_t)JM + 1u)) return;
@@ -367,9 +387,9 @@ __global__ __launch_bounds__(kBlock) void k_center_to_corner(int IM, int JM, int
   const int64_t plane = (int64_t)nI * (JM + 1);
   // chunks blockIdx.y, blockIdx.y + gridDim.y, ... (one per block unless the
   // grid's y limit binds)
-  for (int64_t kc = (int64_t)blockIdx.y * kC2CChunk; kc < (int64_t)KM + 1; kc += (int64_t)gridDim.y * kC2CChunk) {
+  for (int64_t kc = (int64_t)blockIdx.y * chunk; kc < (int64_t)KM + 1; kc += (int64_t)gridDim.y * chunk) {
   const int k0 = (int)kc;
-  const int k1 = k0 + kC2CChunk < KM + 1 ? k0 + kC2CChunk : KM + 1;
+  const int k1 = k0 + chunk < KM + 1 ? k0 + chunk : KM + 1;
   R lo[4][3], hi[4][3];
   bool vlo[4], vhi[4];
   c2c_plane(IM, JM, KM, ucat, i, j, k0 - 1, lo, vlo);

@@ -706,18 +706,21 @@ static int do_remove(picgpu_ctx *c, int check_lost, int check_box, int64_t *remo
   return PICGPU_OK;
 }
 
-static int do_center_to_corner(picgpu_ctx *c) {
+// Node velocities from the cell ones; zero [nzero] is cleared by the same launch.
+static int do_center_to_corner(picgpu_ctx *c, int32_t *zero = nullptr, int64_t nzero = 0) {
   if (!c->have_ucat) {
     set_error("ucat not uploaded");
     return PICGPU_E_STATE;
   }
   return dispatch_real(c, [&](auto *tag) -> int {
     using R = std::remove_pointer_t<decltype(tag)>;
-    // node columns (i, j) x chunks of kC2CChunk planes
-    const int64_t nch = (c->KM + 1 + kC2CChunk - 1) / kC2CChunk;
-    const dim3 grid((unsigned)nblocks((int64_t)(c->IM + 1) * (c->JM + 1)), (unsigned)std::min<int64_t>(nch, 65535));
-    PG_LAUNCH(c, "center_to_corner", grid, kBlock, k_center_to_corner<R>, c->IM, c->JM, c->KM, c->ucat.as<R>(),
-              c->corner.as<R>());
+    // node columns (i, j) x chunks of planes
+    const int64_t columns = (int64_t)(c->IM + 1) * (c->JM + 1);
+    const int chunk = c2c_chunk(columns, (int64_t)c->KM + 1);
+    const int64_t nch = ((int64_t)c->KM + chunk) / chunk;
+    const dim3 grid((unsigned)nblocks(columns), (unsigned)std::min<int64_t>(nch, 65535));
+    PG_LAUNCH(c, "center_to_corner", grid, kBlock, k_center_to_corner<R>, c->IM, c->JM, c->KM, chunk, c->ucat.as<R>(),
+              c->corner.as<R>(), zero, nzero);
     return PICGPU_OK;
   });
 }
@@ -974,16 +977,19 @@ static int face_out(picgpu_ctx *c, void *fo_out) {
   });
 }
 
-static int launch_face_seams(picgpu_ctx *c, const void *fo_in) {
+static SeamCounts seam_counts(const picgpu_ctx *c) {
   const TileMap tm = tile_map(c);
-  const int64_t ni = (int64_t)(tm.NTI - 1) * c->JM * c->KM, nj = (int64_t)(tm.NTJ - 1) * c->IM * c->KM,
-                nk = (int64_t)(tm.NTK - 1) * c->IM * c->JM;
-  if (ni + nj + nk == 0) return PICGPU_OK;
+  return SeamCounts{(int32_t)((int64_t)(tm.NTI - 1) * c->JM * c->KM), (int32_t)((int64_t)(tm.NTJ - 1) * c->IM * c->KM),
+                    (int32_t)((int64_t)(tm.NTK - 1) * c->IM * c->JM)};
+}
+
+static int launch_face_seams(picgpu_ctx *c, const void *fo_in) {
+  const SeamCounts sc = seam_counts(c);
+  if (sc.total() == 0) return PICGPU_OK;
   return dispatch_real(c, [&](auto *tag) -> int {
     using R = std::remove_pointer_t<decltype(tag)>;
     const FaceOut<R> &fo = *static_cast<const FaceOut<R> *>(fo_in);
-    PG_LAUNCH(c, "face_seams", nblocks(ni + nj + nk), kBlock, k_face_seams<R>, c->IM, c->JM, c->KM, (int32_t)ni,
-              (int32_t)nj, (int32_t)nk, fo);
+    PG_LAUNCH(c, "face_seams", nblocks(sc.total()), kBlock, k_face_seams<R>, c->IM, c->JM, c->KM, sc, fo);
     return PICGPU_OK;
   });
 }
@@ -1066,10 +1072,10 @@ static int do_step_fused(picgpu_ctx *c, double dt, unsigned flags, int step, boo
   const int cur = c->kcur, nxt = cur ^ 1;
   PG_CHECK(c->kstart[nxt].ensure(sizeof(int32_t) * (size_t)(nkeys + 2)));
   PG_CHECK(c->kidx[nxt].ensure(sizeof(int32_t) * (size_t)(n > 0 ? n : 1)));
-  PG_HIP(hipMemsetAsync(c->kcount.ptr, 0, sizeof(int32_t) * (size_t)(nkeys + 1), c->stream));
-  // defer list [n] and its length
-  PG_CHECK(c->defer.ensure(sizeof(int32_t) * (size_t)((n > 0 ? n : 1) + 1)));
-  PG_HIP(hipMemsetAsync(c->defer.as<int32_t>() + (n > 0 ? n : 1), 0, sizeof(int32_t), c->stream));
+  // kcount, its last word the length of the defer list, was cleared with the
+  // node velocities (step_batch); building the index here used it since
+  if (fresh) PG_HIP(hipMemsetAsync(c->kcount.ptr, 0, sizeof(int32_t) * (size_t)(nkeys + 2), c->stream));
+  PG_CHECK(c->defer.ensure(sizeof(int32_t) * (size_t)(n > 0 ? n : 1)));
   unsigned long long *hist = hist_reset(c);
   const int32_t *idx = c->kidx[cur].as<int32_t>();
   const int32_t *kstart = c->kstart[cur].as<int32_t>();
@@ -1091,7 +1097,7 @@ static int do_step_fused(picgpu_ctx *c, double dt, unsigned flags, int step, boo
       a.deposit = dep ? 1 : 0;
       if (dep) a.fo = *reinterpret_cast<const FaceOut<R> *>(fo_buf);
       a.defer_list = c->defer.as<int32_t>();
-      a.defer_count = c->defer.as<int32_t>() + (n > 0 ? n : 1);
+      a.defer_count = c->kcount.as<int32_t>() + nkeys + 1;
       constexpr bool EX = sizeof(R) == sizeof(double);
       const char *name = EX ? "step_fused_fp64" : "step_fused_fp32";
       const char *name_list = EX ? "step_list_fp64" : "step_list_fp32";
@@ -1104,7 +1110,10 @@ static int do_step_fused(picgpu_ctx *c, double dt, unsigned flags, int step, boo
         PG_LAUNCH(c, name, nt, kBlock, (k_step_tiled<R, EX, RK, WU>), a, idx, kstart, kbase);
         if (fresh && u1 > u0)
           PG_LAUNCH(c, name_list, nblocks(u1 - u0), kBlock, (k_step_list<R, EX, RK>), a, idx, u0, u1);
-        if (n > 0) PG_LAUNCH(c, "step_deferred", dblocks, kBlock, (k_step_deferred<R, EX, RK>), a);
+        const SeamCounts sc = dep ? seam_counts(c) : SeamCounts{0, 0, 0};
+        if (dblocks + sc.total() > 0)
+          PG_LAUNCH(c, sc.total() ? "face_seams" : "step_deferred", dblocks + nblocks(sc.total()), kBlock,
+                    (k_step_deferred<R, EX, RK>), a, (int)dblocks, sc);
         return PICGPU_OK;
       };
       using T = std::true_type;
@@ -1114,18 +1123,18 @@ static int do_step_fused(picgpu_ctx *c, double dt, unsigned flags, int step, boo
     });
     PG_CHECK(r);
   }
-  if (dep) {
-    PG_CHECK(launch_face_seams(c, fo_buf));
-    c->have_faces = true;
-  }
+  if (dep) c->have_faces = true;
   PG_CHECK(scan_exclusive_i32(c, c->kcount.as<int32_t>(), c->kstart[nxt].as<int32_t>(), nkeys + 1));
   if (n > 0)
     PG_LAUNCH(c, "key_reindex", nblocks(n, kBlock * kReindexPer), kBlock, k_key_reindex, n, m_dev, idx,
               c->sw.cell.as<int32_t>(),
               c->kslot.as<int32_t>(), kbase, CellIdx{c->IM, c->JM, grid_view(c).rI, grid_view(c).rIJ}, tm,
               c->kstart[nxt].as<int32_t>(), c->kidx[nxt].as<int32_t>());
-  if (n > 0 && (flags & (PICGPU_STEP_DEPOSIT_CELLS | PICGPU_STEP_DEPOSIT_FACES))) {
-    if (!c->pid32_valid) {
+  const int32_t *nidx = c->kidx[nxt].as<int32_t>();
+  const int32_t *nstart = c->kstart[nxt].as<int32_t>();
+  const bool cells = (flags & PICGPU_STEP_DEPOSIT_CELLS) != 0;
+  if (cells || faces) {
+    if (n > 0 && !c->pid32_valid) {
       // the 32-bit PID copy, made once after the swarm changed; compaction moves it
       PG_CHECK(c->pid_wide.ensure(sizeof(int32_t)));
       PG_HIP(hipMemsetAsync(c->pid_wide.ptr, 0, sizeof(int32_t), c->stream));
@@ -1133,24 +1142,26 @@ static int do_step_fused(picgpu_ctx *c, double dt, unsigned flags, int step, boo
                 c->pid_wide.as<int32_t>());
       c->pid32_valid = true;
     }
-    PG_LAUNCH(c, "bucket_pid_order", nblocks(nkeys), kBlock, k_bucket_pid_order, nkeys, c->kstart[nxt].as<int32_t>(),
-              c->kidx[nxt].as<int32_t>(), c->sw.pid.as<int64_t>(), c->sw.pid32.as<int32_t>(),
-              c->pid_wide.as<int32_t>());
+    PG_CHECK(dispatch_real(c, [&](auto *tag) -> int {
+      using R = std::remove_pointer_t<decltype(tag)>;
+      auto launch = [&](auto cells_tag) -> int {
+        PG_LAUNCH(c, "bucket_pid_order", nblocks(nkeys), kBlock, (k_bucket_pid_order<R, decltype(cells_tag)::value>),
+                  nkeys, nstart, c->kidx[nxt].as<int32_t>(), c->sw.pid.as<int64_t>(), c->sw.pid32.as<int32_t>(),
+                  c->pid_wide.as<int32_t>(), c->IM, c->JM, c->KM, tm, c->sw.P.as<R>(), c->pavg.as<R>());
+        return PICGPU_OK;
+      };
+      if (!cells) return launch(std::false_type{});
+      PG_CHECK(c->pavg.ensure(sizeof(R) * (size_t)c->ncell));
+      c->have_pavg = true;
+      return launch(std::true_type{});
+    }));
   }
   if (hist) PG_CHECK(hist_read(c));
   // every survivor of a fused step is located: the next index has no unlocated bucket
   c->kcur = nxt;
   c->kbegin_unloc = c->kend_unloc = -1;  // known after the call's counters are read
-  const int32_t *nidx = c->kidx[nxt].as<int32_t>();
-  const int32_t *nstart = c->kstart[nxt].as<int32_t>();
   int r = dispatch_real(c, [&](auto *tag) -> int {
     using R = std::remove_pointer_t<decltype(tag)>;
-    if (flags & PICGPU_STEP_DEPOSIT_CELLS) {
-      PG_CHECK(c->pavg.ensure(sizeof(R) * (size_t)c->ncell));
-      PG_LAUNCH(c, "scatter_P", nblocks(c->ncell), kBlock, k_scatter_P_keyed<R>, c->IM, c->JM, c->KM, tm, nstart,
-                nidx, c->sw.P.as<R>(), c->pavg.as<R>());
-      c->have_pavg = true;
-    }
     if (wu && faces) {
       // weights and velocities were written: the step's deposition is a pass of its own
       for (int dir = 0; dir < 3; ++dir) PG_CHECK(c->face[dir].ensure(sizeof(R) * 4 * (size_t)nface(c, dir)));
@@ -1217,12 +1228,14 @@ static int step_batch(picgpu_ctx *c, double dt, unsigned flags, int s0, int nb, 
   PG_HIP(hipMemsetAsync(c->step_counters.ptr, 0, sizeof(unsigned long long) * kStepCounterWords * (size_t)nb,
                         c->stream));
   unsigned long long *ctr = c->step_counters.as<unsigned long long>();
+  const int64_t nkeys = ntiles(tile_map(c)) * TS;
+  PG_CHECK(c->kcount.ensure(sizeof(int32_t) * (size_t)(nkeys + 2)));
   int64_t m0 = -1;  // entries of the index the batch starts from
   int compacted_at = -1;
   for (int b = 0; b < nb; ++b) {
     const int s = s0 + b;
     if (fields) PG_CHECK(eulerian_fields_async(c));
-    PG_CHECK(do_center_to_corner(c));
+    PG_CHECK(do_center_to_corner(c, c->kcount.as<int32_t>(), nkeys + 2));
     bool compacted = false;
     int64_t entries = 0;
     PG_CHECK(do_step_fused(c, dt, flags, s, s == nsteps - 1, ctr + (size_t)b * kStepCounterWords, &compacted,
