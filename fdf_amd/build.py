@@ -15,8 +15,9 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libpicgpu.so")
-SOURCES = ["picgpu.hip", "scan.hip", "mlp.hip", "eulerian.hip", "io.hip", "seed.hip", "noalloc.hip"]
-HEADERS = ["picgpu_internal.hpp", "kernels.hpp", "walk.hpp"]
+SOURCES = ["picgpu.hip", "scan.hip", "mlp.hip", "eulerian.hip", "io.hip", "seed.hip", "noalloc.hip",
+           "transfer.hip"]
+HEADERS = ["picgpu_internal.hpp", "kernels.hpp", "walk.hpp", "transfer.hpp"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

@@ -761,23 +761,19 @@ __device__ __forceinline__ double cell_volume(const GridView &g, int i, int j, i
 // Face volume fraction = count * V_p / V_dual with V_dual = half the summed
 // volumes of the adjacent cells (lower cell first).
 template <typename R>
-__global__ __launch_bounds__(kBlock) void k_face_volfrac(int dir, GridView g, const R *__restrict__ face,
-                                                         double vp, double *__restrict__ out) {
-  const int IM = g.IM, JM = g.JM, KM = g.KM;
-  const int fI = IM + (dir == 0), fJ = JM + (dir == 1), fK = KM + (dir == 2);
-  const int64_t nf = (int64_t)fI * fJ * fK;
-  int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= nf) return;
-  int i = (int)(f % fI);
-  int64_t r = f / fI;
-  int j = (int)(r % fJ);
-  int k = (int)(r / fJ);
+__device__ __forceinline__ double face_volfrac(int dir, const GridView &g, const R *__restrict__ face, double vp,
+                                               int64_t f) {
+  const int fI = g.IM + (dir == 0), fJ = g.JM + (dir == 1);
+  const int i = (int)(f % fI);
+  const int64_t r = f / fI;
+  const int j = (int)(r % fJ);
+  const int k = (int)(r / fJ);
   double s = 0.0;
-  int li = i - (dir == 0), lj = j - (dir == 1), lk = k - (dir == 2);
+  const int li = i - (dir == 0), lj = j - (dir == 1), lk = k - (dir == 2);
   if (li >= 0 && lj >= 0 && lk >= 0) s += cell_volume(g, li, lj, lk);
-  if (i < IM && j < JM && k < KM) s += cell_volume(g, i, j, k);
-  double vd = 0.5 * s;
-  out[f] = ((double)face[4 * f] * vp) / vd;
+  if (i < g.IM && j < g.JM && k < g.KM) s += cell_volume(g, i, j, k);
+  const double vd = 0.5 * s;
+  return ((double)face[4 * f] * vp) / vd;
 }
 
 // ---------------------------------------------------------------------------

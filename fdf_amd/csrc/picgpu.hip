@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "fused.hpp"
+#include "transfer.hpp"
 
 using namespace picgpu;
 
@@ -279,6 +280,7 @@ int picgpu_destroy(picgpu_ctx *c) {
                     &c->defer, &c->walk_hist};
   for (DevBuf *b : bufs) b->release();
   c->step_counters.release();
+  c->ring.release();
   c->seams.release();
   eulerian_release(c);
   SwarmBufs *sws[] = {&c->sw, &c->alt};
@@ -442,30 +444,28 @@ int picgpu_upload_particles(picgpu_ctx *c, int64_t n, const double *pos, const d
   c->swarm_invalid = false;
   c->pid32_valid = false;
   if (n == 0) return PICGPU_OK;
-  PG_HIP(hipMemcpy(c->sw.pos.ptr, pos, sizeof(double) * 3 * (size_t)n, hipMemcpyHostToDevice));
-  PG_HIP(hipMemcpy(c->sw.pid.ptr, pid, sizeof(int64_t) * (size_t)n, hipMemcpyHostToDevice));
-  {
-    std::vector<int32_t> hc((size_t)n), hs((size_t)n);
-    for (int64_t p = 0; p < n; ++p) {
-      int64_t i = cell[3 * p], j = cell[3 * p + 1], k = cell[3 * p + 2];
-      bool ok = i >= 0 && j >= 0 && k >= 0 && i < c->IM && j < c->JM && k < c->KM;
-      hc[p] = ok ? (int32_t)(i + (int64_t)c->IM * (j + (int64_t)c->JM * k)) : -1;
-      hs[p] = (int32_t)status[p];
-    }
-    PG_HIP(hipMemcpy(c->sw.cell.ptr, hc.data(), sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice));
-    PG_HIP(hipMemcpy(c->sw.status.ptr, hs.data(), sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice));
-  }
-  return dispatch_real(c, [&](auto *tag) -> int {
-    using R = std::remove_pointer_t<decltype(tag)>;
-    std::vector<R> h((size_t)n * 3);
-    for (int64_t q = 0; q < 3 * n; ++q) h[q] = vel ? (R)vel[q] : (R)0;
-    PG_HIP(hipMemcpy(c->sw.vel.ptr, h.data(), sizeof(R) * 3 * (size_t)n, hipMemcpyHostToDevice));
-    for (int64_t q = 0; q < 3 * n; ++q) h[q] = weight ? (R)weight[q] : (R)0;
-    PG_HIP(hipMemcpy(c->sw.w.ptr, h.data(), sizeof(R) * 3 * (size_t)n, hipMemcpyHostToDevice));
-    for (int64_t q = 0; q < n; ++q) h[q] = P ? (R)P[q] : (R)101325.0;
-    PG_HIP(hipMemcpy(c->sw.P.ptr, h.data(), sizeof(R) * (size_t)n, hipMemcpyHostToDevice));
-    return PICGPU_OK;
-  });
+  HostSeg seg[7];
+  int m = 0;
+  auto add = [&](HostKind kind, DevBuf &dev, const void *host, int64_t count, size_t stride) {
+    seg[m++] = HostSeg{kind, dev.ptr, const_cast<void *>(host), count, stride};
+  };
+  add(HostKind::Copy8, c->sw.pos, pos, 3 * n, 8);
+  add(HostKind::Copy8, c->sw.pid, pid, n, 8);
+  add(HostKind::Cell, c->sw.cell, cell, n, 24);
+  add(HostKind::Int32, c->sw.status, status, n, 8);
+  if (vel)
+    add(HostKind::Real, c->sw.vel, vel, 3 * n, 8);
+  else
+    PG_CHECK(fill_real(c, c->sw.vel.ptr, 3 * n, 0.0));
+  if (weight)
+    add(HostKind::Real, c->sw.w, weight, 3 * n, 8);
+  else
+    PG_CHECK(fill_real(c, c->sw.w.ptr, 3 * n, 0.0));
+  if (P)
+    add(HostKind::Real, c->sw.P, P, n, 8);
+  else
+    PG_CHECK(fill_real(c, c->sw.P.ptr, n, 101325.0));
+  return host_upload(c, seg, m);
 }
 
 int picgpu_num_particles(picgpu_ctx *c, int64_t *n) {
@@ -480,41 +480,23 @@ int picgpu_download_particles(picgpu_ctx *c, double *pos, double *vel, int64_t *
   PG_HIP(hipSetDevice(c->device));
   PG_CHECK(settle_swarm(c));
   const int64_t n = c->n;
-  PG_HIP(hipStreamSynchronize(c->stream));
-  if (n == 0) return PICGPU_OK;
-  if (pos) PG_HIP(hipMemcpy(pos, c->sw.pos.ptr, sizeof(double) * 3 * (size_t)n, hipMemcpyDeviceToHost));
-  if (pid) PG_HIP(hipMemcpy(pid, c->sw.pid.ptr, sizeof(int64_t) * (size_t)n, hipMemcpyDeviceToHost));
-  if (cell || status) {
-    std::vector<int32_t> hc((size_t)n), hs((size_t)n);
-    PG_HIP(hipMemcpy(hc.data(), c->sw.cell.ptr, sizeof(int32_t) * (size_t)n, hipMemcpyDeviceToHost));
-    PG_HIP(hipMemcpy(hs.data(), c->sw.status.ptr, sizeof(int32_t) * (size_t)n, hipMemcpyDeviceToHost));
-    for (int64_t p = 0; p < n; ++p) {
-      if (cell) {
-        int32_t v = hc[p];
-        if (v < 0) {
-          cell[3 * p] = cell[3 * p + 1] = cell[3 * p + 2] = -1;
-        } else {
-          cell[3 * p] = v % c->IM;
-          cell[3 * p + 1] = (v / c->IM) % c->JM;
-          cell[3 * p + 2] = v / ((int64_t)c->IM * c->JM);
-        }
-      }
-      if (status) status[p] = hs[p];
-    }
-  }
-  return dispatch_real(c, [&](auto *tag) -> int {
-    using R = std::remove_pointer_t<decltype(tag)>;
-    std::vector<R> h((size_t)n * 3);
-    if (vel) {
-      PG_HIP(hipMemcpy(h.data(), c->sw.vel.ptr, sizeof(R) * 3 * (size_t)n, hipMemcpyDeviceToHost));
-      for (int64_t q = 0; q < 3 * n; ++q) vel[q] = (double)h[q];
-    }
-    if (weight) {
-      PG_HIP(hipMemcpy(h.data(), c->sw.w.ptr, sizeof(R) * 3 * (size_t)n, hipMemcpyDeviceToHost));
-      for (int64_t q = 0; q < 3 * n; ++q) weight[q] = (double)h[q];
-    }
+  if (n == 0) {
+    PG_HIP(hipStreamSynchronize(c->stream));
     return PICGPU_OK;
-  });
+  }
+  HostSeg seg[6];
+  int m = 0;
+  auto add = [&](HostKind kind, DevBuf &dev, void *host, int64_t count, size_t stride) {
+    if (host) seg[m++] = HostSeg{kind, dev.ptr, host, count, stride};
+  };
+  add(HostKind::Copy8, c->sw.pos, pos, 3 * n, 8);
+  add(HostKind::Copy8, c->sw.pid, pid, n, 8);
+  add(HostKind::Cell, c->sw.cell, cell, n, 24);
+  add(HostKind::Int32, c->sw.status, status, n, 8);
+  add(HostKind::Real, c->sw.vel, vel, 3 * n, 8);
+  add(HostKind::Real, c->sw.w, weight, 3 * n, 8);
+  if (m == 0) PG_HIP(hipStreamSynchronize(c->stream));
+  return host_download(c, seg, m);
 }
 
 int picgpu_download_walk_steps(picgpu_ctx *c, int32_t *steps) {
@@ -1495,88 +1477,47 @@ int picgpu_download_grid_field(picgpu_ctx *c, int which, double *out) {
   if (!c || !out) return PICGPU_E_ARG;
   PG_HIP(hipSetDevice(c->device));
   PG_CHECK(need_grid(c));
-  PG_HIP(hipStreamSynchronize(c->stream));
-  const int64_t nx = c->IM + 1, ny = c->JM + 1;
+  auto get = [&](HostKind kind, const void *dev, int64_t count, int dir = 0) {
+    const HostSeg seg{kind, const_cast<void *>(dev), out, count, 8, dir};
+    return host_download(c, &seg, 1);
+  };
   if (which >= PICGPU_FIELD_UCAT && which <= PICGPU_FIELD_AJ) {
     const double *p = nullptr;
     int64_t count = 0;
     PG_CHECK(eulerian_field(c, which, &p, &count));
-    PG_HIP(hipMemcpy(out, p, sizeof(double) * (size_t)count, hipMemcpyDeviceToHost));
-    return PICGPU_OK;
+    return get(HostKind::Copy8, p, count);
   }
-  if (which == PICGPU_FIELD_PARTICLE_COUNT) {
-    PG_CHECK(ensure_cell_counts(c));
-    PG_HIP(hipStreamSynchronize(c->stream));
-    std::vector<int32_t> h((size_t)c->ncell);
-    PG_HIP(hipMemcpy(h.data(), c->cell_count.ptr, sizeof(int32_t) * (size_t)c->ncell, hipMemcpyDeviceToHost));
-    memset(out, 0, sizeof(double) * (size_t)c->nnode);
-    for (int64_t k = 0; k < c->KM; ++k)
-      for (int64_t j = 0; j < c->JM; ++j)
-        for (int64_t i = 0; i < c->IM; ++i) out[(k * ny + j) * nx + i] = (double)h[(k * c->JM + j) * c->IM + i];
-    return PICGPU_OK;
-  }
-  return dispatch_real(c, [&](auto *tag) -> int {
-    using R = std::remove_pointer_t<decltype(tag)>;
-    if (which == PICGPU_FIELD_P_AVERAGE) {
+  switch (which) {
+    case PICGPU_FIELD_PARTICLE_COUNT:
+      PG_CHECK(ensure_cell_counts(c));
+      return get(HostKind::NodeCount, c->cell_count.ptr, c->nnode);
+    case PICGPU_FIELD_P_AVERAGE:
       if (!c->have_pavg) {
         set_error("P average not computed");
         return PICGPU_E_STATE;
       }
-      std::vector<R> h((size_t)c->ncell);
-      PG_HIP(hipMemcpy(h.data(), c->pavg.ptr, sizeof(R) * (size_t)c->ncell, hipMemcpyDeviceToHost));
-      memset(out, 0, sizeof(double) * (size_t)c->nnode);
-      for (int64_t k = 0; k < c->KM; ++k)
-        for (int64_t j = 0; j < c->JM; ++j)
-          for (int64_t i = 0; i < c->IM; ++i) out[(k * ny + j) * nx + i] = (double)h[(k * c->JM + j) * c->IM + i];
-      return PICGPU_OK;
-    }
-    if (which == PICGPU_FIELD_CORNER_VELOCITY) {
+      return get(HostKind::NodeReal, c->pavg.ptr, c->nnode);
+    case PICGPU_FIELD_CORNER_VELOCITY:
       if (!c->have_ucat) return PICGPU_E_STATE;
-      std::vector<R> h((size_t)c->nnode * 3);
-      PG_HIP(hipMemcpy(h.data(), c->corner.ptr, sizeof(R) * h.size(), hipMemcpyDeviceToHost));
-      for (size_t q = 0; q < h.size(); ++q) out[q] = (double)h[q];
-      return PICGPU_OK;
-    }
-    if (which >= PICGPU_FIELD_IFACE && which <= PICGPU_FIELD_KFACE) {
+      return get(HostKind::Real, c->corner.ptr, 3 * c->nnode);
+    case PICGPU_FIELD_IFACE:
+    case PICGPU_FIELD_JFACE:
+    case PICGPU_FIELD_KFACE:
+    case PICGPU_FIELD_IFACE_VOLFRAC:
+    case PICGPU_FIELD_JFACE_VOLFRAC:
+    case PICGPU_FIELD_KFACE_VOLFRAC: {
       if (!c->have_faces) {
         set_error("faces not deposited");
         return PICGPU_E_STATE;
       }
-      int dir = which - PICGPU_FIELD_IFACE;
-      std::vector<R> h((size_t)nface(c, dir) * 4);
-      PG_HIP(hipMemcpy(h.data(), c->face[dir].ptr, sizeof(R) * h.size(), hipMemcpyDeviceToHost));
-      for (size_t q = 0; q < h.size(); ++q) out[q] = (double)h[q];
-      return PICGPU_OK;
+      const bool sums = which <= PICGPU_FIELD_KFACE;
+      const int dir = which - (sums ? PICGPU_FIELD_IFACE : PICGPU_FIELD_IFACE_VOLFRAC);
+      if (sums) return get(HostKind::Real, c->face[dir].ptr, 4 * nface(c, dir));
+      return get(HostKind::Volfrac, c->face[dir].ptr, nface(c, dir), dir);
     }
-    if (which >= PICGPU_FIELD_IFACE_VOLFRAC && which <= PICGPU_FIELD_KFACE_VOLFRAC) {
-      if (!c->have_faces) {
-        set_error("faces not deposited");
-        return PICGPU_E_STATE;
-      }
-      int dir = which - PICGPU_FIELD_IFACE_VOLFRAC;
-      int64_t nf = nface(c, dir);
-      DevBuf tmp;
-      PG_CHECK(tmp.ensure(sizeof(double) * (size_t)nf));
-      {
-        TimerRec _rec;
-        timer_begin(c, "face_volfrac", _rec);
-        hipLaunchKernelGGL(k_face_volfrac<R>, dim3(nblocks(nf)), dim3(kBlock), 0, c->stream, dir, grid_view(c),
-                           c->face[dir].as<R>(), c->particle_volume, tmp.as<double>());
-        timer_end(c, _rec);
-      }
-      hipError_t e1 = hipGetLastError();
-      hipError_t e2 = hipMemcpyAsync(out, tmp.ptr, sizeof(double) * (size_t)nf, hipMemcpyDeviceToHost, c->stream);
-      hipError_t e3 = hipStreamSynchronize(c->stream);
-      tmp.release();
-      if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess) {
-        set_error("face volume fraction failed");
-        return PICGPU_E_HIP;
-      }
-      return PICGPU_OK;
-    }
-    set_error("unknown field %d", which);
-    return PICGPU_E_ARG;
-  });
+  }
+  set_error("unknown field %d", which);
+  return PICGPU_E_ARG;
 }
 
 // ---------------------------------------------------------------------------

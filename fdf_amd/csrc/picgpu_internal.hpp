@@ -58,6 +58,15 @@ struct DevBuf {
   }
 };
 
+// Pinned slots through which host arrays go to and from the device, and the
+// event of the last kernel on each (transfer.hip); made by the first transfer.
+struct HostRing {
+  static constexpr int kSlots = 8;
+  void *p = nullptr;
+  hipEvent_t ev[kSlots] = {};
+  void release();
+};
+
 // Particle arrays (structure of arrays).  vel, w and P hold `real` elements:
 // double in PICGPU_FP64 mode, float in PICGPU_FP32 mode.
 struct SwarmBufs {
@@ -188,6 +197,8 @@ struct picgpu_ctx {
 
   // scratch for scans
   picgpu::DevBuf scan_tmp;
+
+  picgpu::HostRing ring;
 
   // counters
   picgpu::DevBuf counters;  // uint64 [kCounterStripes][C_NUM]
