@@ -259,6 +259,7 @@ int picgpu_create(picgpu_ctx **out, const picgpu_options *opt) {
     delete c;
     return rs;
   }
+  rings_open();
   *out = c;
   return PICGPU_OK;
 }
@@ -280,7 +281,8 @@ int picgpu_destroy(picgpu_ctx *c) {
                     &c->defer, &c->walk_hist};
   for (DevBuf *b : bufs) b->release();
   c->step_counters.release();
-  c->ring.release();
+  c->transfer.release();
+  rings_close();
   c->seams.release();
   eulerian_release(c);
   SwarmBufs *sws[] = {&c->sw, &c->alt};

@@ -58,11 +58,9 @@ struct DevBuf {
   }
 };
 
-// Pinned slots through which host arrays go to and from the device, and the
-// event of the last kernel on each (transfer.hip); made by the first transfer.
-struct HostRing {
+// The event of the last kernel on each pinned slot of a transfer (transfer.hip).
+struct TransferEvents {
   static constexpr int kSlots = 8;
-  void *p = nullptr;
   hipEvent_t ev[kSlots] = {};
   void release();
 };
@@ -198,7 +196,7 @@ struct picgpu_ctx {
   // scratch for scans
   picgpu::DevBuf scan_tmp;
 
-  picgpu::HostRing ring;
+  picgpu::TransferEvents transfer;
 
   // counters
   picgpu::DevBuf counters;  // uint64 [kCounterStripes][C_NUM]

@@ -18,6 +18,7 @@
 
 #include <atomic>
 #include <memory>
+#include <mutex>
 #include <new>
 #include <thread>
 #include <vector>
@@ -28,6 +29,7 @@ namespace picgpu {
 // slot's time (kernels writing 1 MiB: 52 GB/s, 256 KiB 43, 128 KiB 35).  A
 // small transfer fills its slots less, so that the host's copies overlap too,
 // but not below 512 KiB: an event and its wait take about 10 us.
+constexpr int kSlots = TransferEvents::kSlots;
 constexpr size_t kSlotBytes = 1 << 20, kMinFill = 512 << 10;
 // one thread more for every 2 MiB, up to 7: memory copies reach 30 GB/s on one
 // thread, 81 on four, 124 on eight; starting 7 threads takes 0.1 ms
@@ -191,27 +193,59 @@ static hipError_t launch_unpack(picgpu_ctx *c, const HostSeg &s, int64_t e0, int
 }
 
 // ---------------------------------------------------------------- the ring
-void HostRing::release() {
+// The slots.  The host's first touch of pinned memory costs 0.38 ms a MiB (a
+// fault a page), so the rings of transfers that have ended are kept for the
+// next ones, at most kRingsKept of them, until the last context is destroyed.
+// A transfer holds its ring alone; any device may use it.
+constexpr int kRingsKept = 2;
+static std::mutex g_rings_mu;
+static void *g_rings[kRingsKept];
+static int g_ring_users;
+
+void rings_open() {
+  std::lock_guard<std::mutex> lock(g_rings_mu);
+  ++g_ring_users;
+}
+void rings_close() {
+  std::lock_guard<std::mutex> lock(g_rings_mu);
+  if (--g_ring_users > 0) return;
+  for (void *&r : g_rings) {
+    if (r) (void)hipHostFree(r);
+    r = nullptr;
+  }
+}
+static int take_ring(void **out) {
+  {
+    std::lock_guard<std::mutex> lock(g_rings_mu);
+    for (void *&r : g_rings)
+      if (r) {
+        *out = r;
+        r = nullptr;
+        return PICGPU_OK;
+      }
+  }
+  if (hipHostMalloc(out, kSlotBytes * kSlots, hipHostMallocPortable) == hipSuccess) return PICGPU_OK;
+  (void)hipGetLastError();
+  set_error("hipHostMalloc(%zu) failed", kSlotBytes * kSlots);
+  return PICGPU_E_NOMEM;
+}
+static void give_ring(void *ring) {
+  {
+    std::lock_guard<std::mutex> lock(g_rings_mu);
+    for (void *&r : g_rings)
+      if (!r) {
+        r = ring;
+        return;
+      }
+  }
+  (void)hipHostFree(ring);
+}
+
+void TransferEvents::release() {
   for (hipEvent_t &e : ev) {
     if (e) (void)hipEventDestroy(e);
     e = nullptr;
   }
-  if (p) (void)hipHostFree(p);
-  p = nullptr;
-}
-
-static int ensure_ring(picgpu_ctx *c) {
-  HostRing &r = c->ring;
-  if (r.p) return PICGPU_OK;
-  for (hipEvent_t &e : r.ev)
-    if (!e) PG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  if (hipHostMalloc(&r.p, kSlotBytes * HostRing::kSlots, 0) != hipSuccess) {
-    (void)hipGetLastError();
-    r.p = nullptr;
-    set_error("hipHostMalloc(%zu) failed", kSlotBytes * HostRing::kSlots);
-    return PICGPU_E_NOMEM;
-  }
-  return PICGPU_OK;
 }
 
 namespace {
@@ -237,6 +271,7 @@ struct Group {
 // claimed or can issue, and ends on an error.
 struct Transfer {
   picgpu_ctx *c;
+  char *ring;
   const HostSeg *segs;
   const std::vector<Chunk> &chunks;
   const std::vector<Group> &groups;
@@ -246,8 +281,8 @@ struct Transfer {
   std::atomic_flag issuing = ATOMIC_FLAG_INIT;
   std::atomic<int> err{0};
 
-  char *slot(int64_t k) const { return static_cast<char *>(c->ring.p) + (size_t)(k % HostRing::kSlots) * kSlotBytes; }
-  hipEvent_t event(int64_t k) const { return c->ring.ev[k % HostRing::kSlots]; }
+  char *slot(int64_t k) const { return ring + (size_t)(k % kSlots) * kSlotBytes; }
+  hipEvent_t event(int64_t k) const { return c->transfer.ev[k % kSlots]; }
   void copy(int64_t k) const {
     for (size_t q = groups[(size_t)k].first; q < groups[(size_t)k].end; ++q) {
       const Chunk &ch = chunks[q];
@@ -280,7 +315,7 @@ struct Transfer {
     if (issuing.test_and_set(std::memory_order_acquire)) return;
     const int64_t N = (int64_t)groups.size();
     for (int64_t k = issued.load(); k < N && !err.load(); ++k) {
-      if (k >= HostRing::kSlots && !done[k - HostRing::kSlots].load(std::memory_order_acquire)) break;
+      if (k >= kSlots && !done[k - kSlots].load(std::memory_order_acquire)) break;
       if (!launch(k)) break;
       issued.store(k + 1, std::memory_order_release);
     }
@@ -306,8 +341,8 @@ struct Transfer {
     while (!err.load()) {
       const int64_t k = claimed.fetch_add(1);
       if (k >= N) return;
-      if (k >= HostRing::kSlots) {
-        while (!done[k - HostRing::kSlots].load(std::memory_order_acquire)) {
+      if (k >= kSlots) {
+        while (!done[k - kSlots].load(std::memory_order_acquire)) {
           if (err.load()) return;
           std::this_thread::yield();
         }
@@ -327,12 +362,8 @@ struct Transfer {
 };
 }  // namespace
 
-static int host_transfer(picgpu_ctx *c, const HostSeg *segs, int nsegs, bool down) {
-  size_t total = 0;
-  for (int s = 0; s < nsegs; ++s) total += (size_t)segs[s].n * segs[s].stride;
-  if (total == 0) return PICGPU_OK;
-  PG_CHECK(ensure_ring(c));
-  size_t fill = total / HostRing::kSlots;
+static int move_host(picgpu_ctx *c, void *ring, const HostSeg *segs, int nsegs, size_t total, bool down) {
+  size_t fill = total / kSlots;
   fill = fill < kMinFill ? kMinFill : fill > kSlotBytes ? kSlotBytes : fill;
   std::vector<std::thread> helpers;
   try {
@@ -355,7 +386,7 @@ static int host_transfer(picgpu_ctx *c, const HostSeg *segs, int nsegs, bool dow
     }
     std::unique_ptr<std::atomic<unsigned char>[]> done(new std::atomic<unsigned char>[groups.size()]);
     for (size_t k = 0; k < groups.size(); ++k) done[k].store(0);
-    Transfer t{c, segs, chunks, groups, done.get(), down};
+    Transfer t{c, static_cast<char *>(ring), segs, chunks, groups, done.get(), down};
     if (down) t.issue();
     const size_t want = total / kBytesPerThread;
     const int nth = want < (size_t)kMaxThreads ? (int)want : kMaxThreads;
@@ -382,6 +413,19 @@ static int host_transfer(picgpu_ctx *c, const HostSeg *segs, int nsegs, bool dow
     return PICGPU_E_NOMEM;
   }
   return PICGPU_OK;
+}
+
+static int host_transfer(picgpu_ctx *c, const HostSeg *segs, int nsegs, bool down) {
+  size_t total = 0;
+  for (int s = 0; s < nsegs; ++s) total += (size_t)segs[s].n * segs[s].stride;
+  if (total == 0) return PICGPU_OK;
+  for (hipEvent_t &e : c->transfer.ev)
+    if (!e) PG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  void *ring = nullptr;
+  PG_CHECK(take_ring(&ring));
+  const int r = move_host(c, ring, segs, nsegs, total, down);
+  give_ring(ring);
+  return r;
 }
 
 int host_download(picgpu_ctx *c, const HostSeg *segs, int nsegs) { return host_transfer(c, segs, nsegs, true); }

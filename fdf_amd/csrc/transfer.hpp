@@ -22,6 +22,11 @@ struct HostSeg {
   int dir = 0;
 };
 
+// every context between its creation and its destruction: the pinned slots
+// are kept while there is one
+void rings_open();
+void rings_close();
+
 // Both wait until the arrays have been moved.
 int host_download(picgpu_ctx *c, const HostSeg *segs, int nsegs);
 int host_upload(picgpu_ctx *c, const HostSeg *segs, int nsegs);
