@@ -35,8 +35,8 @@ constexpr int H = PICGPU_MLP_HIDDEN;  // 64
 constexpr int NP = H * 3 + H + H * H + H + 3 * H + 3;
 constexpr int OFF_W1 = 0, OFF_B1 = 3 * H, OFF_W2 = OFF_B1 + H, OFF_B2 = OFF_W2 + H * H, OFF_W3 = OFF_B2 + H,
               OFF_B3 = OFF_W3 + 3 * H;
-constexpr int TILE = 32;          // samples per wavefront
-constexpr int MLP_THREADS = 64;   // one wavefront per block
+constexpr int TILE = 32;          // samples per workgroup of the training kernel
+constexpr int MLP_THREADS = 256;  // four wavefronts per 32-sample tile
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -63,102 +63,19 @@ __device__ __forceinline__ float act_d(float z) {
   return (u > 0.0f && u < 1.0f) ? __builtin_fmaf(kActC, z, u) : act_gate(z);
 }
 
-// C[32x32] += A[32xK] * B[Kx32]; A(m,k) = A[m*sAm + k*sAk], B(k,n) = B[k*sBk + n*sBn]
-// (bf16 in LDS or global).  Operand layout of v_mfma_f32_32x32x8_bf16: lane l
-// holds A(l%32, 4*(l/32)+v) and B(4*(l/32)+v, l%32), v = 0..3; the result
-// register r of lane l is C(8*(r/4) + 4*(l/32) + r%4, l%32).
-__device__ __forceinline__ void mm32(const uint16_t *A, int sAm, int sAk, const uint16_t *B, int sBk, int sBn, int K,
-                                     f32x16 &acc) {
-  const int l = threadIdx.x & 63;
-  const int r = l & 31, h = l >> 5;
-  for (int k0 = 0; k0 < K; k0 += 8) {
-    bf16x4 a, b;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int k = k0 + 4 * h + v;
-      a[v] = (short)A[r * sAm + k * sAk];
-      b[v] = (short)B[k * sBk + r * sBn];
-    }
-    acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, b, acc, 0, 0, 0);
-  }
-}
+// Operand layout of v_mfma_f32_32x32x8_bf16: lane l holds A(l%32, 4*(l/32)+v)
+// and B(4*(l/32)+v, l%32), v = 0..3; the result register r of lane l is
+// C(8*(r/4) + 4*(l/32) + r%4, l%32).
 __device__ __forceinline__ int res_row(int reg) { return 8 * (reg / 4) + 4 * ((threadIdx.x & 63) >> 5) + (reg % 4); }
 __device__ __forceinline__ int res_col() { return threadIdx.x & 31; }
+__device__ __forceinline__ f32x16 mfma8(bf16x4 a, bf16x4 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, b, c, 0, 0, 0);
+}
 
 struct MlpWeights {
   const float *p;      // FP32 master parameters (biases are read from here)
   const uint16_t *wb;  // BF16 W1 [64][3], W2 [64][64], W3 [3][64] (same offsets as the master)
 };
-
-struct TileLds {
-  float x[TILE][3];
-  float z1[TILE][H];
-  float z2[TILE][H];
-  uint16_t a1[TILE][H];
-  uint16_t a2[TILE][H];
-  uint16_t g2[TILE][H];
-  float y[TILE][3];
-  float g3[TILE][3];
-  float g1[TILE][H];
-};
-
-// Forward of one 32-sample tile held in L.x; fills z1, a1, z2, a2, y.
-__device__ void tile_forward(const MlpWeights &Wt, TileLds &L) {
-  const int l = threadIdx.x & 63;
-  // layer 1 (VALU): lane l owns hidden unit q = l for all 32 samples
-  {
-    const int q = l;
-    const float w0 = bf2f(Wt.wb[OFF_W1 + 3 * q]), w1 = bf2f(Wt.wb[OFF_W1 + 3 * q + 1]),
-                w2 = bf2f(Wt.wb[OFF_W1 + 3 * q + 2]), b = Wt.p[OFF_B1 + q];
-    for (int m = 0; m < TILE; ++m) {
-      float z = __builtin_fmaf(w0, L.x[m][0], __builtin_fmaf(w1, L.x[m][1], __builtin_fmaf(w2, L.x[m][2], b)));
-      L.z1[m][q] = z;
-      L.a1[m][q] = f2bf(act(z));
-    }
-  }
-  __syncthreads();
-  // layer 2 (MFMA): Z2 = A1 (32x64) * W2^T, two 32-column tiles
-  for (int t = 0; t < 2; ++t) {
-    const int n = 32 * t + res_col();
-    const float b = Wt.p[OFF_B2 + n];
-    f32x16 acc;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = b;  // the bias is the first term of each sum
-    mm32(&L.a1[0][0], H, 1, Wt.wb + OFF_W2 + 32 * t * H, 1, H, H, acc);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int m = res_row(r);
-      const float z = acc[r];
-      L.z2[m][n] = z;
-      L.a2[m][n] = f2bf(act(z));
-    }
-  }
-  __syncthreads();
-  // layer 3 (MFMA): Y = A2 (32x64) * W3^T, columns 0..2 of one tile
-  {
-    const int l3 = res_col();
-    const int h = l >> 5;
-    const float b3 = l3 < 3 ? Wt.p[OFF_B3 + l3] : 0.0f;
-    f32x16 acc;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = b3;
-    for (int k0 = 0; k0 < H; k0 += 8) {
-      bf16x4 a, b;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int k = k0 + 4 * h + v;
-        a[v] = (short)L.a2[l3][k];
-        b[v] = l3 < 3 ? (short)Wt.wb[OFF_W3 + l3 * H + k] : (short)0;
-      }
-      acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, b, acc, 0, 0, 0);
-    }
-    if (l3 < 3) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) L.y[res_row(r)][l3] = acc[r];
-    }
-  }
-  __syncthreads();
-}
 
 // ---------------------------------------------------------------- inference
 // normalised input of a physical position
@@ -348,146 +265,275 @@ __device__ __forceinline__ uint64_t mix64(uint64_t z) {
   return z ^ (z >> 31);
 }
 
-// Forward + backward of one 32-sample tile per block.  Rows are samples
-// base..base+31 of x/t, or (when npairs > 0) random pairs drawn with the
-// SplitMix64 hash of (seed, iteration, row).  Writes the tile's gradient
-// (parameter layout) and its summed squared error to part[block].
+// z mod n for n < 2^31, given inv = floor((2^64 - 1) / n): the quotient
+// umulhi(z, inv) is at most two short.
+__device__ __forceinline__ uint64_t fast_mod(uint64_t z, uint64_t n, uint64_t inv) {
+  uint64_t r = z - __umul64hi(z, inv) * n;
+  r = r >= n ? r - n : r;
+  return r >= n ? r - n : r;
+}
+
+constexpr int RS = H + 4;  // BF16 row stride in LDS: 8-byte reads of 32 rows meet 64 different banks
+struct TileLds {
+  float x[TILE][3], t[TILE][3], y[TILE][3], g3[TILE][3];
+  float z1[TILE][H], z2[TILE][H];  // z2 then holds the FP32 dZ2
+  float g1[TILE][H];
+  uint16_t w2[H][RS];
+  uint16_t a1[TILE][RS], a2[TILE][RS], g2[TILE][RS];
+};
+// four consecutive BF16 of a row, or one column's of four rows
+__device__ __forceinline__ bf16x4 row4(const uint16_t *p) { return *reinterpret_cast<const bf16x4 *>(p); }
+__device__ __forceinline__ bf16x4 col4(const uint16_t (*m)[RS], int row, int col) {
+  bf16x4 v;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) v[k] = (short)m[row + k][col];
+  return v;
+}
+
+// Forward + backward of one 32-sample tile per workgroup of four wavefronts.
+// Rows are samples base..base+31 of x/t, or (when npairs > 0) random pairs
+// drawn with the SplitMix64 hash of (seed, iteration, row).  Writes the
+// tile's gradient (parameter layout) and its summed squared error to
+// part[block].
+//
+// A batch is a few hundred tiles, less than one wavefront a SIMD, so the time
+// is one tile's chain of products and sums, not their number.  The tile's
+// elementwise work is split over the wavefronts by samples, its products by
+// 32x32 blocks and its long sums (over samples, in sample order) one to a
+// wavefront; W2 is staged in LDS while the samples are fetched, and every
+// operand row is padded so that 8-byte reads are free of bank conflicts.
+// Batch of 4096 (128 tiles): 15.0 us with one wavefront a tile, 7.8 with four;
+// with the reduction and Adam in one launch (6.4 + 2.8 -> 3.1 us) an iteration
+// takes 11 instead of 25 us.
 __global__ __launch_bounds__(MLP_THREADS) void k_mlp_fwd_bwd(int64_t n, const float *__restrict__ x,
                                                              const float *__restrict__ t, int64_t npairs,
-                                                             uint64_t seed, int iter, float scale, MlpWeights Wt,
-                                                             float *__restrict__ part) {
-  __shared__ TileLds L;
-  __shared__ float tl[TILE][3];
-  __shared__ int valid[TILE];
-  const int l = threadIdx.x;
+                                                             uint64_t inv, uint64_t seed, int iter, float scale,
+                                                             MlpWeights Wt, float *__restrict__ part) {
+  __shared__ __align__(16) TileLds L;
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int r32 = l & 31, h4 = 4 * (l >> 5);
   const int64_t base = (int64_t)blockIdx.x * TILE;
-  if (l < TILE) {
+  bool valid = false;  // wavefront 0, lanes below 32: sample l counts
+  if (w < 2 && l < TILE) {
     int64_t s = base + l;
-    int ok = s < n;
-    if (npairs > 0) s = (int64_t)(mix64(seed ^ mix64(((uint64_t)iter << 32) + (uint64_t)(base + l))) % (uint64_t)npairs);
-    valid[l] = ok;
-    for (int c = 0; c < 3; ++c) {
-      L.x[l][c] = ok ? x[3 * s + c] : 0.f;
-      tl[l][c] = ok ? t[3 * s + c] : 0.f;
-    }
-  }
-  __syncthreads();
-  tile_forward(Wt, L);
-  float *g = part + (int64_t)blockIdx.x * (NP + 1);
-  // output error
-  float sq = 0.f;
-  if (l < TILE) {
-    for (int c = 0; c < 3; ++c) {
-      const float e = valid[l] ? L.y[l][c] - tl[l][c] : 0.f;
-      sq = __builtin_fmaf(e, e, sq);
-      L.g3[l][c] = e * scale;
-    }
-  }
-  for (int off = 32; off > 0; off >>= 1) sq += __shfl_xor(sq, off);
-  if (l == 0) g[NP] = sq;
-  __syncthreads();
-  // layer 3 gradients and dA2 -> g2 (lane n owns hidden unit n)
-  {
-    const int nn = l;
-    float gw0 = 0.f, gw1 = 0.f, gw2 = 0.f, gb2 = 0.f;
-    const float w30 = bf2f(Wt.wb[OFF_W3 + nn]), w31 = bf2f(Wt.wb[OFF_W3 + H + nn]),
-                w32 = bf2f(Wt.wb[OFF_W3 + 2 * H + nn]);
-    for (int m = 0; m < TILE; ++m) {
-      const float a2 = bf2f(L.a2[m][nn]);
-      gw0 = __builtin_fmaf(L.g3[m][0], a2, gw0);
-      gw1 = __builtin_fmaf(L.g3[m][1], a2, gw1);
-      gw2 = __builtin_fmaf(L.g3[m][2], a2, gw2);
-      const float da2 = __builtin_fmaf(L.g3[m][0], w30, __builtin_fmaf(L.g3[m][1], w31, L.g3[m][2] * w32));
-      const float g2 = da2 * act_d(L.z2[m][nn]);
-      gb2 += g2;
-      L.g2[m][nn] = f2bf(g2);
-    }
-    g[OFF_W3 + nn] = gw0;
-    g[OFF_W3 + H + nn] = gw1;
-    g[OFF_W3 + 2 * H + nn] = gw2;
-    g[OFF_B2 + nn] = gb2;
-    if (l < 3) {
-      float s = 0.f;
-      for (int m = 0; m < TILE; ++m) s += L.g3[m][l];
-      g[OFF_B3 + l] = s;
-    }
-  }
-  __syncthreads();
-  // dW2[n][q] = sum_m g2[m][n] a1[m][q]  (M = n, N = q, K = m)
-  for (int tn = 0; tn < 2; ++tn)
-    for (int tq = 0; tq < 2; ++tq) {
-      f32x16 acc = {};
-      mm32(&L.g2[0][32 * tn], 1, H, &L.a1[0][32 * tq], H, 1, TILE, acc);
+    valid = s < n;
+    if (npairs > 0)
+      s = (int64_t)fast_mod(mix64(seed ^ mix64(((uint64_t)iter << 32) + (uint64_t)(base + l))), (uint64_t)npairs, inv);
+    const float *src = w == 0 ? x : t;
+    float(*dst)[3] = w == 0 ? L.x : L.t;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) g[OFF_W2 + (32 * tn + res_row(r)) * H + 32 * tq + res_col()] = acc[r];
+    for (int c = 0; c < 3; ++c) dst[l][c] = valid ? src[3 * s + c] : 0.f;
+  }
+  {
+    const int row = threadIdx.x >> 2, col = 16 * (threadIdx.x & 3);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      *reinterpret_cast<bf16x4 *>(&L.w2[row][col + 4 * k]) = row4(Wt.wb + OFF_W2 + row * H + col + 4 * k);
+  }
+  const float w10 = bf2f(Wt.wb[OFF_W1 + 3 * l]), w11 = bf2f(Wt.wb[OFF_W1 + 3 * l + 1]),
+              w12 = bf2f(Wt.wb[OFF_W1 + 3 * l + 2]), b1 = Wt.p[OFF_B1 + l];
+  const float w30 = bf2f(Wt.wb[OFF_W3 + l]), w31 = bf2f(Wt.wb[OFF_W3 + H + l]),
+              w32 = bf2f(Wt.wb[OFF_W3 + 2 * H + l]);
+  bf16x4 w3b[H / 8];  // layer 3's B operand (columns 0..2)
+  float b3 = 0.f, b2 = 0.f;
+  if (w == 0) {
+#pragma unroll
+    for (int k = 0; k < H / 8; ++k) {
+      const bf16x4 zero = {};
+      w3b[k] = r32 < 3 ? row4(Wt.wb + OFF_W3 + r32 * H + 8 * k + h4) : zero;
     }
-  // dA1[m][q] = sum_n g2[m][n] W2[n][q]  (M = m, N = q, K = n) -> g1
-  for (int tq = 0; tq < 2; ++tq) {
-    f32x16 acc = {};
-    mm32(&L.g2[0][0], H, 1, Wt.wb + OFF_W2 + 32 * tq, H, 1, H, acc);
+    b3 = r32 < 3 ? Wt.p[OFF_B3 + r32] : 0.f;
+  }
+  if (w < 2) b2 = Wt.p[OFF_B2 + 32 * w + r32];
+  __syncthreads();
+  // layer 1 (VALU): lane l is hidden unit l
+#pragma unroll
+  for (int q = 0; q < TILE / 4; ++q) {
+    const int m = TILE / 4 * w + q;
+    const float z = __builtin_fmaf(w10, L.x[m][0], __builtin_fmaf(w11, L.x[m][1], __builtin_fmaf(w12, L.x[m][2], b1)));
+    L.z1[m][l] = z;
+    L.a1[m][l] = f2bf(act(z));
+  }
+  __syncthreads();
+  // layer 2 (MFMA): Z2 = A1 (32x64) W2^T, a 32-column block for wavefronts 0 and 1
+  if (w < 2) {
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = b2;  // the bias is the first term of each sum
+#pragma unroll
+    for (int k0 = 0; k0 < H; k0 += 8) acc = mfma8(row4(&L.a1[r32][k0 + h4]), row4(&L.w2[32 * w + r32][k0 + h4]), acc);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int m = res_row(r), q = 32 * tq + res_col();
-      L.g1[m][q] = acc[r] * act_d(L.z1[m][q]);
+      L.z2[res_row(r)][32 * w + r32] = acc[r];
+      L.a2[res_row(r)][32 * w + r32] = f2bf(act(acc[r]));
     }
   }
   __syncthreads();
-  // layer 1 gradients (lane q owns hidden unit q)
-  {
-    const int q = l;
-    float gx = 0.f, gy = 0.f, gz = 0.f, gb = 0.f;
-    for (int m = 0; m < TILE; ++m) {
-      const float g1 = L.g1[m][q];
-      gx = __builtin_fmaf(g1, L.x[m][0], gx);
-      gy = __builtin_fmaf(g1, L.x[m][1], gy);
-      gz = __builtin_fmaf(g1, L.x[m][2], gz);
-      gb += g1;
+  // layer 3 (MFMA): Y = A2 (32x64) W3^T, columns 0..2 of one block
+  if (w == 0) {
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = b3;
+#pragma unroll
+    for (int k = 0; k < H / 8; ++k) acc = mfma8(row4(&L.a2[r32][8 * k + h4]), w3b[k], acc);
+    if (r32 < 3) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) L.y[res_row(r)][r32] = acc[r];
     }
-    g[OFF_W1 + 3 * q] = gx;
-    g[OFF_W1 + 3 * q + 1] = gy;
-    g[OFF_W1 + 3 * q + 2] = gz;
-    g[OFF_B1 + q] = gb;
+  }
+  __syncthreads();
+  float *g = part + (int64_t)blockIdx.x * (NP + 1);
+  // output error
+  if (w == 0) {
+    float sq = 0.f;
+    if (l < TILE) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const float e = valid ? L.y[l][c] - L.t[l][c] : 0.f;
+        sq = __builtin_fmaf(e, e, sq);
+        L.g3[l][c] = e * scale;
+      }
+    }
+    for (int off = 32; off > 0; off >>= 1) sq += __shfl_xor(sq, off);
+    if (l == 0) g[NP] = sq;
+  }
+  __syncthreads();
+  // dZ2 = dA2 act'(z2): lane l is hidden unit l
+#pragma unroll
+  for (int q = 0; q < TILE / 4; ++q) {
+    const int m = TILE / 4 * w + q;
+    const float da2 = __builtin_fmaf(L.g3[m][0], w30, __builtin_fmaf(L.g3[m][1], w31, L.g3[m][2] * w32));
+    const float g2 = da2 * act_d(L.z2[m][l]);
+    L.z2[m][l] = g2;
+    L.g2[m][l] = f2bf(g2);
+  }
+  __syncthreads();
+  // dW2[n][q] = sum_m g2[m][n] a1[m][q], block (tn, tq)
+  auto dw2 = [&](int tn, int tq) {
+    f32x16 acc = {};
+#pragma unroll
+    for (int k0 = 0; k0 < TILE; k0 += 8)
+      acc = mfma8(col4(L.g2, k0 + h4, 32 * tn + r32), col4(L.a1, k0 + h4, 32 * tq + r32), acc);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) g[OFF_W2 + (32 * tn + res_row(r)) * H + 32 * tq + r32] = acc[r];
+  };
+  // row c of dW3
+  auto dw3 = [&](int c) {
+    float s = 0.f;
+#pragma unroll
+    for (int m = 0; m < TILE; ++m) s = __builtin_fmaf(L.g3[m][c], bf2f(L.a2[m][l]), s);
+    g[OFF_W3 + c * H + l] = s;
+  };
+  if (w < 2) {
+    // dA1[m][q] = sum_n g2[m][n] W2[n][q] -> dZ1, the chain the rest waits for
+    f32x16 acc = {};
+#pragma unroll
+    for (int k0 = 0; k0 < H; k0 += 8)
+      acc = mfma8(row4(&L.g2[r32][k0 + h4]), col4(L.w2, k0 + h4, 32 * w + r32), acc);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int m = res_row(r), q = 32 * w + r32;
+      L.g1[m][q] = acc[r] * act_d(L.z1[m][q]);
+    }
+  } else {
+    dw2(1, w - 2);
+    if (w == 2) {
+      dw3(2);
+    } else {
+      float s = 0.f, s3 = 0.f;
+#pragma unroll
+      for (int m = 0; m < TILE; ++m) s += L.z2[m][l];
+      g[OFF_B2 + l] = s;
+      if (l < 3) {
+#pragma unroll
+        for (int m = 0; m < TILE; ++m) s3 += L.g3[m][l];
+        g[OFF_B3 + l] = s3;
+      }
+    }
+  }
+  __syncthreads();
+  if (w < 2) {
+    dw2(0, w);
+    dw3(w);
+  } else {
+    // layer 1 gradients: lane l is hidden unit l
+    float s0 = 0.f, s1 = 0.f;
+    if (w == 2) {
+#pragma unroll
+      for (int m = 0; m < TILE; ++m) {
+        s0 = __builtin_fmaf(L.g1[m][l], L.x[m][0], s0);
+        s1 = __builtin_fmaf(L.g1[m][l], L.x[m][1], s1);
+      }
+      g[OFF_W1 + 3 * l] = s0;
+      g[OFF_W1 + 3 * l + 1] = s1;
+    } else {
+#pragma unroll
+      for (int m = 0; m < TILE; ++m) {
+        s0 = __builtin_fmaf(L.g1[m][l], L.x[m][2], s0);
+        s1 += L.g1[m][l];
+      }
+      g[OFF_W1 + 3 * l + 2] = s0;
+      g[OFF_B1 + l] = s1;
+    }
   }
 }
+
+struct AdamArgs {
+  float *p, *m, *v;
+  uint16_t *wb;
+  float lr, b1, b2, eps, bc1, bc2;
+};
 
 // grad[j] = sum over tiles of part[tile][j], j < NP + 1, in a fixed order:
 // wavefront g of a block sums the tiles b = g (mod RED_GROUPS) in ascending
 // order, then the RED_GROUPS partial sums are added in ascending g.  Each
 // block covers 64 consecutive j, one per lane, so every load is a coalesced
-// 256-byte row segment and RED_GROUPS loads are in flight per j.
-constexpr int RED_GROUPS = 8;
+// 256-byte row segment; RED_AHEAD of a wavefront's loads are issued before
+// their sums.  With ADAM the wavefront that holds the sum takes its parameter's
+// step and refreshes the BF16 weight copy, in place of a launch for that.
+constexpr int RED_GROUPS = 8, RED_AHEAD = 16;
+template <bool ADAM>
 __global__ __launch_bounds__(64 * RED_GROUPS) void k_mlp_reduce(int ntiles, const float *__restrict__ part,
-                                                                float *__restrict__ grad) {
+                                                                float *__restrict__ grad, AdamArgs ad) {
   __shared__ float ps[RED_GROUPS][64];
   const int lane = threadIdx.x & 63, grp = threadIdx.x >> 6;
   const int j = blockIdx.x * 64 + lane;
+  float p0 = 0.f, m0 = 0.f, v0 = 0.f;
+  if (ADAM && grp == 0 && j < NP) {
+    p0 = ad.p[j];
+    m0 = ad.m[j];
+    v0 = ad.v[j];
+  }
   float s = 0.f;
   if (j <= NP)
-    for (int b = grp; b < ntiles; b += RED_GROUPS) s += part[(int64_t)b * (NP + 1) + j];
+    for (int b0 = grp; b0 < ntiles; b0 += RED_AHEAD * RED_GROUPS) {
+      float q[RED_AHEAD];
+#pragma unroll
+      for (int u = 0; u < RED_AHEAD; ++u) {
+        const int b = b0 + u * RED_GROUPS;
+        q[u] = b < ntiles ? part[(int64_t)b * (NP + 1) + j] : 0.f;
+      }
+#pragma unroll
+      for (int u = 0; u < RED_AHEAD; ++u)
+        if (b0 + u * RED_GROUPS < ntiles) s += q[u];
+    }
   ps[grp][lane] = s;
   __syncthreads();
   if (grp == 0 && j <= NP) {
-    float t = ps[0][lane];
+    float gj = ps[0][lane];
 #pragma unroll
-    for (int q = 1; q < RED_GROUPS; ++q) t += ps[q][lane];
-    grad[j] = t;
+    for (int q = 1; q < RED_GROUPS; ++q) gj += ps[q][lane];
+    grad[j] = gj;
+    if (ADAM && j < NP) {
+      const float mj = ad.b1 * m0 + (1.f - ad.b1) * gj;
+      const float vj = ad.b2 * v0 + (1.f - ad.b2) * gj * gj;
+      ad.m[j] = mj;
+      ad.v[j] = vj;
+      const float pj = p0 - ad.lr * (mj / ad.bc1) / (sqrtf(vj / ad.bc2) + ad.eps);
+      ad.p[j] = pj;
+      ad.wb[j] = f2bf(pj);
+    }
   }
-}
-
-// Adam on the FP32 master, then refresh the BF16 weight copy.
-__global__ __launch_bounds__(256) void k_mlp_adam(float *__restrict__ p, float *__restrict__ m, float *__restrict__ v,
-                                                  const float *__restrict__ g, uint16_t *__restrict__ wb, float lr,
-                                                  float b1, float b2, float eps, float bc1, float bc2) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= NP) return;
-  const float gj = g[j];
-  const float mj = b1 * m[j] + (1.f - b1) * gj;
-  const float vj = b2 * v[j] + (1.f - b2) * gj * gj;
-  m[j] = mj;
-  v[j] = vj;
-  const float pj = p[j] - lr * (mj / bc1) / (sqrtf(vj / bc2) + eps);
-  p[j] = pj;
-  wb[j] = f2bf(pj);
 }
 
 __global__ __launch_bounds__(256) void k_mlp_to_bf16(const float *__restrict__ p, uint16_t *__restrict__ wb) {
@@ -581,16 +627,22 @@ static int upload_params(picgpu_ctx *c, const float *h) {
   return PICGPU_OK;
 }
 
-// device forward+backward over host-visible device arrays x, t (n samples)
+// device forward+backward over device arrays x, t (n samples); with adam, its
+// step on the gradient
 static int loss_grad_device(picgpu_ctx *c, int64_t n, const float *dx, const float *dt, int64_t npairs, uint64_t seed,
-                            int iter, float *loss_host) {
+                            int iter, float *loss_host, const AdamArgs *adam = nullptr) {
   const int64_t tiles = (n + TILE - 1) / TILE;
   PG_CHECK(c->mlp_partial.ensure(sizeof(float) * (size_t)tiles * (NP + 1)));
   const float scale = 2.0f / (3.0f * (float)n);
-  PG_LAUNCH(c, "mlp_fwd_bwd", tiles, MLP_THREADS, k_mlp_fwd_bwd, n, dx, dt, npairs, seed, iter, scale, weights(c),
-            c->mlp_partial.as<float>());
-  PG_LAUNCH(c, "mlp_reduce", (NP + 1 + 63) / 64, 64 * RED_GROUPS, k_mlp_reduce, (int)tiles, c->mlp_partial.as<float>(),
-            c->mlp_grad.as<float>());
+  PG_LAUNCH(c, "mlp_fwd_bwd", tiles, MLP_THREADS, k_mlp_fwd_bwd, n, dx, dt, npairs,
+            npairs > 0 ? UINT64_MAX / (uint64_t)npairs : 0, seed, iter, scale, weights(c), c->mlp_partial.as<float>());
+  const int64_t blocks = (NP + 1 + 63) / 64;
+  if (adam)
+    PG_LAUNCH(c, "mlp_reduce", blocks, 64 * RED_GROUPS, k_mlp_reduce<true>, (int)tiles, c->mlp_partial.as<float>(),
+              c->mlp_grad.as<float>(), *adam);
+  else
+    PG_LAUNCH(c, "mlp_reduce", blocks, 64 * RED_GROUPS, k_mlp_reduce<false>, (int)tiles, c->mlp_partial.as<float>(),
+              c->mlp_grad.as<float>(), AdamArgs{});
   if (loss_host) {
     float sq = 0.f;
     PG_HIP(hipMemcpyAsync(&sq, c->mlp_grad.as<float>() + NP, sizeof(float), hipMemcpyDeviceToHost, c->stream));
@@ -745,14 +797,13 @@ int picgpu_mlp_train(picgpu_ctx *c, int64_t max_pairs, int batch, int iters, flo
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   float bc1 = 1.f, bc2 = 1.f;
   for (int it = 0; it < iters; ++it) {
-    PG_CHECK(loss_grad_device(c, batch, c->mlp_x.as<float>(), c->mlp_t.as<float>(), npairs, seed, it, nullptr));
     bc1 *= b1;
     bc2 *= b2;
     // cosine decay to lr/20
     const float lr_t = (float)(lr * (0.05 + 0.95 * 0.5 * (1.0 + cos(3.141592653589793 * it / (double)iters))));
-    PG_LAUNCH(c, "mlp_adam", (NP + 255) / 256, 256, k_mlp_adam, c->mlp_master.as<float>(), c->mlp_adam_m.as<float>(),
-              c->mlp_adam_v.as<float>(), c->mlp_grad.as<float>(), c->mlp_bf16.as<uint16_t>(), lr_t, b1, b2, eps,
-              1.f - bc1, 1.f - bc2);
+    const AdamArgs adam{c->mlp_master.as<float>(), c->mlp_adam_m.as<float>(), c->mlp_adam_v.as<float>(),
+                        c->mlp_bf16.as<uint16_t>(), lr_t, b1, b2, eps, 1.f - bc1, 1.f - bc2};
+    PG_CHECK(loss_grad_device(c, batch, c->mlp_x.as<float>(), c->mlp_t.as<float>(), npairs, seed, it, nullptr, &adam));
   }
   // loss over the first pairs (up to 64 K) with the trained weights
   const int64_t ne = npairs < 65536 ? ((int64_t)npairs / TILE) * TILE : 65536;
