@@ -1569,7 +1569,9 @@ __global__ __launch_bounds__(kBlock) void k_bucket_pid_order(int64_t nkeys, cons
 // likewise along j and k; faces sum count and momentum.  The lower face of
 // cell c in direction d is the sum over the lower neighbour's particles
 // (weight a_d) plus the sum over c's own (weight 1-a_d), each summed from
-// zero in PID order (buckets ordered by k_bucket_pid_order).
+// zero in PID order.  KEYED: through the key index, its buckets ordered by
+// k_bucket_pid_order; otherwise kstart is the cells' starts and the swarm
+// itself is in that order (the stage-wise sort), idx unused.
 //
 // One workgroup per 8x8x4 tile of the extended range [0..IM]x[0..JM]x[0..KM].
 // Pass 1: each thread runs its cell's particles once and leaves, per
@@ -1583,7 +1585,7 @@ __global__ __launch_bounds__(kBlock) void k_bucket_pid_order(int64_t nkeys, cons
 // a few contiguous lines.  In FP32 the kernel is held to at least 6
 // wavefronts per SIMD (at most 80 VGPRs; it takes 69, so 7 fit, with no
 // spills); FP64 needs more registers (4 per SIMD).
-template <typename R>
+template <typename R, bool KEYED>
 __global__ __launch_bounds__(kBlock, sizeof(R) == 4 ? 6 : 1) void k_deposit_tiles(
     int IM, int JM, int KM, TileMap tm, TileMap xm, const int32_t *__restrict__ kstart,
     const int32_t *__restrict__ idx, const R *__restrict__ w, const R *__restrict__ vel, R *__restrict__ fi,
@@ -1617,21 +1619,19 @@ __global__ __launch_bounds__(kBlock, sizeof(R) == 4 ? 6 : 1) void k_deposit_tile
   }
   const bool halo = l < NH && hi >= 0 && hj >= 0 && hk >= 0 && hi < IM && hj < JM && hk < KM;
   int32_t s_own = 0, n_own = 0, sh = 0, nh = 0;
-  if (own) {
-    const int32_t key = cell_key(tm, i, j, k);
-    s_own = kstart[key];
-    n_own = kstart[key + 1] - s_own;
-  }
-  if (halo) {
-    const int32_t key = cell_key(tm, hi, hj, hk);
-    sh = kstart[key];
-    nh = kstart[key + 1] - sh;
-  }
+  auto bucket = [&](int bi3, int bj3, int bk3, int32_t &s, int32_t &n) {
+    const int32_t key = KEYED ? cell_key(tm, bi3, bj3, bk3) : pack_cell(bi3, bj3, bk3, IM, JM);
+    s = kstart[key];
+    n = kstart[key + 1] - s;
+  };
+  auto entry = [&](int32_t q) -> int32_t { return KEYED ? idx[q] : q; };
+  if (own) bucket(i, j, k, s_own, n_own);
+  if (halo) bucket(hi, hj, hk, sh, nh);
   int32_t qo[K], qh[K];
 #pragma unroll
   for (int u = 0; u < K; ++u) {
-    qo[u] = u < n_own ? idx[s_own + u] : 0;
-    qh[u] = u < nh ? idx[sh + u] : 0;
+    qo[u] = u < n_own ? entry(s_own + u) : 0;
+    qh[u] = u < nh ? entry(sh + u) : 0;
   }
   R cw[K][3], cv[K][3], hw[K], hv[K][3];
 #pragma unroll
@@ -1653,7 +1653,7 @@ __global__ __launch_bounds__(kBlock, sizeof(R) == 4 ? 6 : 1) void k_deposit_tile
   auto load_batch = [&](int32_t s, int32_t n, int32_t t0, R bw[K][3], R bu[K][3]) {
     int32_t qq[K];
 #pragma unroll
-    for (int u = 0; u < K; ++u) qq[u] = t0 + u < n ? idx[s + t0 + u] : 0;
+    for (int u = 0; u < K; ++u) qq[u] = t0 + u < n ? entry(s + t0 + u) : 0;
 #pragma unroll
     for (int u = 0; u < K; ++u)
       if (t0 + u < n) {

@@ -156,6 +156,11 @@ static GridView grid_view(picgpu_ctx *c) {
                   c->IM > 0 && c->JM > 0 ? 1.0 / ((double)c->IM * (double)c->JM) : 0.0};
 }
 
+static TileMap tile_map(const picgpu_ctx *c) {
+  return TileMap{(c->IM + TX - 1) / TX, (c->JM + TY - 1) / TY, (c->KM + TZ - 1) / TZ};
+}
+static int64_t ntiles(const TileMap &t) { return (int64_t)t.NTI * t.NTJ * t.NTK; }
+
 // Padded bounding box of all nodes (grid.c:762-883 on one rank) and state reset
 // after a grid upload.
 static int finish_grid(picgpu_ctx *c) {
@@ -737,13 +742,21 @@ static int do_sort(picgpu_ctx *c) {
   }
   PG_CHECK(scan_exclusive_i32(c, c->cell_count.as<int32_t>(), c->cell_start.as<int32_t>(), c->ncell));
   if (n > 0) {
+    // the order under construction: kidx and pos0 hold nothing else here
+    DevBuf &sidx = c->kidx[c->kcur], &spid = c->pos0;
+    c->keyed = false;
+    PG_CHECK(sidx.ensure(sizeof(int32_t) * (size_t)n));
+    PG_CHECK(spid.ensure(sizeof(int64_t) * (size_t)n));
+    const int32_t *start = c->cell_start.as<int32_t>();
+    PG_LAUNCH(c, "slot_scatter", nblocks(n), kBlock, k_slot_scatter, n, c->rank.as<int32_t>(), start,
+              c->sw.cell.as<int32_t>(), c->sw.pid.as<int64_t>(), sidx.as<int32_t>(), spid.as<int64_t>());
     int r = dispatch_real(c, [&](auto *tag) -> int {
       using R = std::remove_pointer_t<decltype(tag)>;
-      PG_LAUNCH(c, "sort_scatter", nblocks(n), kBlock, k_sort_scatter<R>, n, c->rank.as<int32_t>(),
-                c->cell_start.as<int32_t>(), c->sw.pos.as<double>(), c->sw.vel.as<R>(), c->sw.w.as<R>(),
-                c->sw.cell.as<int32_t>(), c->sw.status.as<int32_t>(), c->sw.pid.as<int64_t>(), c->sw.P.as<R>(),
-                c->alt.pos.as<double>(), c->alt.vel.as<R>(), c->alt.w.as<R>(), c->alt.cell.as<int32_t>(),
-                c->alt.status.as<int32_t>(), c->alt.pid.as<int64_t>(), c->alt.P.as<R>());
+      PG_LAUNCH(c, "sort_gather", nblocks(n), kBlock, k_sort_gather<R>, start + c->ncell, start, sidx.as<int32_t>(),
+                spid.as<int64_t>(), c->sw.pos.as<double>(), c->sw.vel.as<R>(), c->sw.w.as<R>(),
+                c->sw.cell.as<int32_t>(), c->sw.status.as<int32_t>(), c->sw.P.as<R>(), c->alt.pos.as<double>(),
+                c->alt.vel.as<R>(), c->alt.w.as<R>(), c->alt.cell.as<int32_t>(), c->alt.status.as<int32_t>(),
+                c->alt.pid.as<int64_t>(), c->alt.P.as<R>());
       return PICGPU_OK;
     });
     PG_CHECK(r);
@@ -782,7 +795,7 @@ static int do_scatter_P(picgpu_ctx *c) {
   int r = dispatch_real(c, [&](auto *tag) -> int {
     using R = std::remove_pointer_t<decltype(tag)>;
     PG_LAUNCH(c, "scatter_P", nblocks(c->ncell), kBlock, k_scatter_P<R>, c->ncell, c->cell_start.as<int32_t>(),
-              c->sw.pid.as<int64_t>(), c->sw.P.as<R>(), c->pavg.as<R>());
+              c->sw.P.as<R>(), c->pavg.as<R>());
     return PICGPU_OK;
   });
   PG_CHECK(r);
@@ -794,21 +807,28 @@ static int64_t nface(picgpu_ctx *c, int dir) {
   return (int64_t)(c->IM + (dir == 0)) * (c->JM + (dir == 1)) * (c->KM + (dir == 2));
 }
 
-static int do_deposit_faces(picgpu_ctx *c) {
+// Face sums over the particles of each cell (all three directions): through
+// the key index kstart / idx, or over the swarm sorted by cell (idx null,
+// kstart the cells' starts).
+static int launch_deposit_tiles(picgpu_ctx *c, const int32_t *kstart, const int32_t *idx) {
   for (int dir = 0; dir < 3; ++dir) PG_CHECK(c->face[dir].ensure(c->rsize * 4 * (size_t)nface(c, dir)));
-  int r = dispatch_real(c, [&](auto *tag) -> int {
+  const TileMap tm = tile_map(c);
+  const TileMap xm{c->IM / TX + 1, c->JM / TY + 1, c->KM / TZ + 1};  // tiles over [0..IM]x[0..JM]x[0..KM]
+  PG_CHECK(dispatch_real(c, [&](auto *tag) -> int {
     using R = std::remove_pointer_t<decltype(tag)>;
-    for (int dir = 0; dir < 3; ++dir) {
-      PG_LAUNCH(c, "deposit_faces", nblocks(nface(c, dir)), kBlock, k_deposit_faces<R>, dir, c->IM, c->JM, c->KM,
-                c->cell_start.as<int32_t>(), c->sw.pid.as<int64_t>(), c->sw.w.as<R>(), c->sw.vel.as<R>(),
-                c->face[dir].as<R>());
-    }
-    return PICGPU_OK;
-  });
-  PG_CHECK(r);
+    auto launch = [&](auto keyed) -> int {
+      PG_LAUNCH(c, "deposit_faces", ntiles(xm), kBlock, (k_deposit_tiles<R, decltype(keyed)::value>), c->IM, c->JM,
+                c->KM, tm, xm, kstart, idx, c->sw.w.as<R>(), c->sw.vel.as<R>(), c->face[0].as<R>(),
+                c->face[1].as<R>(), c->face[2].as<R>());
+      return PICGPU_OK;
+    };
+    return idx ? launch(std::true_type{}) : launch(std::false_type{});
+  }));
   c->have_faces = true;
   return PICGPU_OK;
 }
+
+static int do_deposit_faces(picgpu_ctx *c) { return launch_deposit_tiles(c, c->cell_start.as<int32_t>(), nullptr); }
 
 static int do_rk2(picgpu_ctx *c, double dt) {
   const int64_t n = c->n;
@@ -851,11 +871,6 @@ static int do_rk2(picgpu_ctx *c, double dt) {
 // kCompactEvery steps and at the end of picgpu_step.
 // ---------------------------------------------------------------------------
 static constexpr int kCompactEvery = 16;
-
-static TileMap tile_map(const picgpu_ctx *c) {
-  return TileMap{(c->IM + TX - 1) / TX, (c->JM + TY - 1) / TY, (c->KM + TZ - 1) / TZ};
-}
-static int64_t ntiles(const TileMap &t) { return (int64_t)t.NTI * t.NTJ * t.NTK; }
 
 // Index of the current swarm in kidx[kcur] / kstart[kcur]: live particles by
 // key, the live ones without a cell in the last bucket, removed ones left out.
@@ -1144,19 +1159,8 @@ static int do_step_fused(picgpu_ctx *c, double dt, unsigned flags, int step, boo
   // every survivor of a fused step is located: the next index has no unlocated bucket
   c->kcur = nxt;
   c->kbegin_unloc = c->kend_unloc = -1;  // known after the call's counters are read
-  int r = dispatch_real(c, [&](auto *tag) -> int {
-    using R = std::remove_pointer_t<decltype(tag)>;
-    if (wu && faces) {
-      // weights and velocities were written: the step's deposition is a pass of its own
-      for (int dir = 0; dir < 3; ++dir) PG_CHECK(c->face[dir].ensure(sizeof(R) * 4 * (size_t)nface(c, dir)));
-      const TileMap xm{c->IM / TX + 1, c->JM / TY + 1, c->KM / TZ + 1};  // tiles over [0..IM]x[0..JM]x[0..KM]
-      PG_LAUNCH(c, "deposit_faces", ntiles(xm), kBlock, k_deposit_tiles<R>, c->IM, c->JM, c->KM, tm, xm, nstart, nidx,
-                c->sw.w.as<R>(), c->sw.vel.as<R>(), c->face[0].as<R>(), c->face[1].as<R>(), c->face[2].as<R>());
-      c->have_faces = true;
-    }
-    return PICGPU_OK;
-  });
-  PG_CHECK(r);
+  // weights and velocities were written: the step's deposition is a pass of its own
+  if (wu && faces) PG_CHECK(launch_deposit_tiles(c, nstart, nidx));
   c->steps_since_compact++;
   c->compact_pending = true;
   if (c->steps_since_compact >= kCompactEvery) {

@@ -75,3 +75,55 @@ def test_bucket_order_and_averages(oracle, precision, wide, per_cell):
         assert np.abs(avg - ref).max() <= 1e-5 * 101375.0
         for a, b in zip(faces, refs):
             assert np.abs(a - b).max() <= 1e-5 * max(1.0, np.abs(b).max())
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("n,crowd", [(1, 0), (300, 0), (257, 257), (6000, 3000)])
+def test_stage_sort(oracle, precision, wide, n, crowd):
+    """The stage-wise sort: cells in order, PIDs in order within a cell (also
+    with `crowd` particles in one cell), the particles without a cell after
+    them; the averages and face sums of that swarm."""
+    from fdf_amd.swarm import PicGpu
+
+    print("[gpu-case] stage sort", precision, wide, n, crowd, flush=True)
+    IM, JM, KM = 9, 5, 7
+    rng = np.random.default_rng(n)
+    pos = rng.random((n, 3))
+    pos[:crowd] = (np.array([4, 2, 3]) + rng.random((crowd, 3))) / [IM, JM, KM]
+    pos[crowd + 3::11] += 2.0  # outside: no cell
+    pid = rng.permutation(n).astype(np.int64) * 3 + ((1 << 33) if wide else 0)
+    P = 101325.0 + 50.0 * rng.random(n)
+    with PicGpu(precision=precision) as g:
+        g.upload_grid(IM, JM, KM, W.uniform_grid(IM, JM, KM))
+        g.upload_ucat(rng.standard_normal(3 * (IM + 1) * (JM + 1) * (KM + 1)))
+        g.upload_particles(pos, pid=pid, P=P)
+        g.LocateAllParticlesInGrid()
+        g.InterpolateAllFieldsToSwarm()
+        before = g.download_particles()
+        g.ScatterAllParticleFieldsToEulerFields()
+        g.DepositParticlesToFaces(1e-9)
+        d = g.download_particles()
+        avg = g.field(L.FIELD_P_AVERAGE)
+        faces = [g.field(f) for f in (L.FIELD_IFACE, L.FIELD_JFACE, L.FIELD_KFACE)]
+    flat = lambda c: np.where(c[:, 0] < 0, 1 << 40, c[:, 0] + IM * (c[:, 1] + JM * c[:, 2]))  # noqa: E731
+    fb = flat(before["cell"])
+    order = np.lexsort((np.where(fb < 1 << 40, before["pid"], np.arange(n)), fb))
+    for k in d:
+        np.testing.assert_array_equal(d[k], before[k][order])
+    at = d["cell"][:, 0] >= 0
+    c, w, v, ids = d["cell"][at], d["weight"][at], d["vel"][at], d["pid"][at]
+    Pd = np.empty(3 * n)
+    Pd[pid - pid.min()] = P
+    Pd = Pd[ids - pid.min()]
+    if precision == "fp32":
+        Pd = Pd.astype(np.float32).astype(np.float64)
+    ref = oracle.scatter_P(IM, JM, KM, c, Pd, ids, oracle.count_cells(IM, JM, KM, c))
+    refs = oracle.deposit_faces(IM, JM, KM, c, w, v, ids)
+    if precision == "fp64":
+        assert np.array_equal(avg, ref)
+        assert all(np.array_equal(a, b) for a, b in zip(faces, refs))
+    else:
+        assert np.abs(avg - ref).max() <= 1e-5 * 101375.0
+        for a, b in zip(faces, refs):  # n terms of at most |v|, one rounding each
+            assert np.abs(a - b).max() <= max(1e-5, n * 2.0 ** -24) * max(1.0, np.abs(b).max())
