@@ -96,8 +96,13 @@ __global__ __launch_bounds__(kBlock) void k_reset_advect(int64_t n, double *__re
 // at different iterations, and a wavefront would otherwise pay for the FP64
 // path in nearly every one (groups of 8, 24 and 48 measure alike).
 // 8,388,608 particles moved by up to 1.5 cells an axis in 128x128x256 cells, in
-// random order, FP64: 2.60 -> 1.33 ms (about 9.1 -> 6.3 GB of record lines);
-// 10,000 particles from cell (0,0,0) of 20x20x280: 2.12 -> 0.33 ms.
+// random order, FP64: 2.60 -> 1.33 ms (about 9.1 -> 6.3 GB of record lines).
+//
+// Long walks are bound by instructions (four wavefronts a SIMD, about 300 an
+// iteration), so the iterations run in a loop of their own, branch-free but for
+// the walk's ends (about 120): the wavefront turns to ended walks, new particles
+// and full evaluations when kStopped lanes have stopped.  10,000 particles from
+// cell (0,0,0) of 128x128x192, FP64: 395 -> 242 us; of 24x24x24: 60 -> 44.
 // ---------------------------------------------------------------------------
 template <typename R>
 struct LocateArgs {
@@ -126,175 +131,77 @@ struct LocateArgs {
 // there are enough, so that a wavefront's last, long walks weigh little.
 // 3,000 particles, FP32, call and wait: 63 us at 256 a wavefront, 42 us at 16.
 constexpr int64_t kLocateWaves = 4096;
-inline int64_t locate_chunk(int64_t n) {
-  const int64_t c = (n + kLocateWaves - 1) / kLocateWaves;
-  return c < 16 ? 16 : c > 256 ? 256 : c;
+inline int64_t locate_chunk(int64_t n, int lanes) {
+  const int64_t c = (n + kLocateWaves - 1) / kLocateWaves, least = lanes > 1 ? 64 / lanes : 16;
+  return c < least ? least : c > 256 ? 256 : c;
 }
 inline int64_t locate_blocks(int64_t n, int64_t chunk) {
   const int64_t waves = (n + chunk - 1) / chunk;
   return (waves * 64 + kBlock - 1) / kBlock;
 }
 constexpr int kExactGroup = 24;
+constexpr int kHeld = 2;      // full evaluations that took a walk on before it is taken on by them alone
+constexpr int kStopped = 16;  // lanes without a walk at which a wavefront turns to them
 
-template <typename R, bool EXACT>
-__global__ __launch_bounds__(kBlock, 4) void k_locate(LocateArgs<R> a) {
-  __shared__ int32_t shist[64];
-  if (threadIdx.x < 64) shist[threadIdx.x] = 0;
-  __syncthreads();
-  const int lane = threadIdx.x & 63;
-  const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const int64_t base = wave * a.chunk;
-  const int64_t end = base + a.chunk < a.n ? base + a.chunk : a.n;
-  int64_t cursor = base;
-  int32_t p = 0;  // n < 2^31
-  int ph = 0;  // 0: no particle, 1: walking, 2: waiting for the FP64 evaluation of its cell
-  int ci = 0, cj = 0, ck = 0, steps = 0;
-  int32_t lc = 0;  // ci + IM (cj + JM ck); used only inside the grid
-  const int32_t sj = a.g.IM, sk = a.g.IM * a.g.JM;
-  CycleGuard cyc;
-  double x[3] = {0.0, 0.0, 0.0};
-  unsigned long long my_iters = 0;
-  unsigned long long my_fb = 0;
-  unsigned my_max = 0, my_loc = 0, my_lost = 0;
-  int my_err = 0;
-  const unsigned long long lane_mask_lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  // the step of walkingsearch.c:919-946 on certified or FP64 distances
-  auto step = [&](const auto d[6]) {
-    if (d[F_FRONT] < 0) {
-      ck += 1;
-      lc += sk;
-    } else if (d[F_BACK] < 0) {
-      ck -= 1;
-      lc -= sk;
-    }
-    if (d[F_LEFT] < 0) {
-      ci -= 1;
-      lc -= 1;
-    } else if (d[F_RIGHT] < 0) {
-      ci += 1;
-      lc += 1;
-    }
-    if (d[F_BOTTOM] < 0) {
-      cj -= 1;
-      lc -= sj;
-    } else if (d[F_TOP] < 0) {
-      cj += 1;
-      lc += sj;
-    }
-  };
-  while (true) {
-    const unsigned long long idle = __ballot(ph == 0);
-    if (idle != 0ull && cursor < end) {
-      if (ph == 0) {
-        const int64_t q = cursor + __popcll(idle & lane_mask_lt);
-        if (q < end) {
-          const int32_t pq = a.order ? a.order[q] : (int32_t)q;
-          const int32_t st = a.status[pq];
-          int32_t c = a.cell[pq];
+// Walks that all start in cell (0,0,0) are long.  In a grid of at least
+// kLocateLong cells along some axis, lanes a particle (k_locate_ahead): 16 up to
+// 16,384 particles, 4 up to 131,072, while the evaluations that no walk reaches
+// still find idle lanes.  The locate in FP64, us, one lane / 16 / 4:
+//   n          20x20x280          63x47x129        24x24x24
+//   10,000     221 /  74 / 106    166 / 108 / 125   44 / 53 / 52
+//   60,000     452 /   - / 247    245 /   - / 202   70 /  - / 76
+//   100,000    499 /   - / 344    271 /   - / 271   76 /  - / 101
+// and before both, 342, 265 and 60 at 10,000.
+constexpr int kLocateLong = 48;
+inline int locate_ahead(int64_t n) { return n <= kLocateWaves * 4 ? 16 : n <= kLocateWaves * 32 ? 4 : 1; }
+// From this many on, the records' lines through LDS (wave_records): 2,000,000 in
+// 128x128x192, 3.48 -> 3.12 ms in FP64, 4.20 -> 3.45 in FP32; 300,000 there 738
+// -> 728 us; 300,000 short walks in a 48x48x250 tube 205 -> 276.
+constexpr int64_t kLocateLines = 1 << 19;
+
+// The FP32 record of cell l for each lane of a wavefront (l < 0: none), all
+// lanes taking part; stage: 64 records of LDS, the wavefront's own.
+// A lane that reads the 128 bytes of its own record makes 8 loads that each
+// touch a line of its own in every lane.  Here 8 lanes read one record's line
+// together and LDS turns it round; the chunks of record r are stored XORed
+// with r mod 8, so that neither the writes (8 chunks of a record) nor the
+// reads (a chunk of 8 records) meet in a bank.
+__device__ __forceinline__ CellPlanes32 wave_records(const CellPlanes32 *__restrict__ recs, int32_t l, float4 *stage,
+                                                     int lane) {
+  const int row = lane >> 3, col = lane & 7;
+  const float4 *src = reinterpret_cast<const float4 *>(recs);
+  float4 v[8];
 #pragma unroll
-          for (int t = 0; t < 3; ++t) x[t] = a.pos[3 * (int64_t)pq + t];
-          if (!(st == ST_LOCATED || (a.skip_lost && st == ST_LOST))) {
-            p = pq;
-            ph = 1;
-            if (c < 0 && a.guess) c = a.guess[pq];
-            ci = cj = ck = 0;  // (info.xs, info.ys, info.zs) on one rank, walkingsearch.c:611-616
-            if (c >= 0) unpack_cell(c, cell_idx(a.g), ci, cj, ck);
-            lc = c >= 0 ? c : 0;
-            steps = 0;
-            cyc = CycleGuard();
-          } else if (a.steps_out) {
-            a.steps_out[pq] = 0;
-          }
-        }
-      }
-      cursor += __popcll(idle);
-    }
-    const unsigned long long walking = __ballot(ph == 1);
-    unsigned long long waiting = 0ull;
-    if constexpr (EXACT) waiting = __ballot(ph == 2);
-    if ((walking | waiting) == 0ull) {
-      if (cursor >= end) break;
-      continue;
-    }
-    bool done = false, located = false;
-    const bool exact_turn = EXACT && (walking == 0ull || __popcll(waiting) >= kExactGroup);
-    if (exact_turn) {
-      if constexpr (EXACT) {
-        if (ph == 2) {
-          ph = 1;
-          R d[6];
-          if (!eval_planes_exact(static_cast<const CellPlanes64 *>(a.planes)[lc], x, d)) {
-            my_err = 1;
-            done = true;
-          } else if (point_accepted<R>(d)) {
-            R wv[3];
-            weights_from_distances<R>(d, a.clamp, wv);
-#pragma unroll
-            for (int t = 0; t < 3; ++t) a.w[3 * (int64_t)p + t] = wv[t];
-            located = true;
-            done = true;
-          } else {
-            step(d);
-            if (steps >= a.max_traversal) done = true;  // MAX_TRAVERSAL (:1206-1212)
-          }
-        }
-      }
-    } else if (ph == 1) {
-      // ---- one iteration of the walk (walkingsearch.c:1123-1203) ----
-      steps++;
-      if (ci < 0 || ci >= a.g.IM || cj < 0 || cj >= a.g.JM || ck < 0 || ck >= a.g.KM) {
-        done = true;  // walked outside the global domain: LOST (:1127-1132)
-      } else if (cyc.revisit(lc)) {
-        done = true;  // periodic walk: LOST at MAX_TRAVERSAL (:1206-1212)
-        steps = a.max_traversal;
-      } else if constexpr (EXACT) {
-        float d[6];
-        // certified: no distance is zero, so the point is inside or beyond a face
-        if (a.filter && planes_fp32_distances(a.filter[lc], x, d) == 0u && !point_accepted<float>(d)) {
-          step(d);
-          if (steps >= a.max_traversal) done = true;
-        } else {
-          ph = 2;
-        }
-      } else {
-        R d[6];
-        const FilterResult fr = eval_planes_fp32(static_cast<const CellPlanes32 *>(a.planes)[lc], a.g, ci, cj, ck, x,
-                                                 a.thresh_scale, d);
-        my_fb += fr.fallbacks;
-        if (fr.degenerate) {
-          my_err = 1;
-          done = true;
-        } else if (point_accepted<R>(d)) {
-          R wv[3];
-          weights_from_distances<R>(d, a.clamp, wv);
-#pragma unroll
-          for (int t = 0; t < 3; ++t) a.w[3 * (int64_t)p + t] = wv[t];
-          located = true;
-          done = true;
-        } else {
-          step(d);
-          if (steps >= a.max_traversal) done = true;
-        }
-      }
-    }
-    if (done) {
-      if (located) {
-        a.cell[p] = lc;
-        a.status[p] = ST_LOCATED;
-        my_loc++;
-      } else if (!my_err) {
-        a.cell[p] = -1;
-        a.status[p] = ST_LOST;
-        my_lost++;
-      }
-      if (a.steps_out) a.steps_out[p] = steps;
-      if (a.walk_hist) atomicAdd(&shist[steps < 63 ? steps : 63], 1);
-      my_iters += steps;
-      my_max = my_max > (unsigned)steps ? my_max : (unsigned)steps;
-      ph = 0;
-    }
+  for (int b = 0; b < 8; ++b) {
+    const int32_t lr = __shfl(l, 8 * b + row);
+    v[b] = src[(int64_t)(lr < 0 ? 0 : lr) * 8 + col];
   }
-  // wave-level reduction of the statistics, one atomic per wave
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int b = 0; b < 8; ++b) stage[(8 * b + row) * 8 + (col ^ row)] = v[b];
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  CellPlanes32 r;
+#pragma unroll
+  for (int c = 0; c < 6; ++c) r.plane[c] = stage[lane * 8 + (c ^ col)];
+  const float4 t0 = stage[lane * 8 + (6 ^ col)], t1 = stage[lane * 8 + (7 ^ col)];
+  r.v0[0] = __hiloint2double(__float_as_int(t0.y), __float_as_int(t0.x));
+  r.v0[1] = __hiloint2double(__float_as_int(t0.w), __float_as_int(t0.z));
+  r.v0[2] = __hiloint2double(__float_as_int(t1.y), __float_as_int(t1.x));
+  r.thr = t1.z;
+  r.amax = t1.w;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  return r;
+}
+
+// Statistics of a locate launch: one atomic a wavefront and word, and the
+// workgroup's histogram of walk iterations.
+template <typename R>
+__device__ __forceinline__ void locate_tally(const LocateArgs<R> &a, int64_t base, int lane,
+                                             unsigned long long my_iters, unsigned long long my_fb, unsigned my_max,
+                                             unsigned my_loc, unsigned my_lost, int my_err,
+                                             const int32_t *shist) {
   if (base < a.n) {
     for (int off = 32; off > 0; off >>= 1) {
       my_iters += __shfl_xor(my_iters, off);
@@ -321,6 +228,398 @@ __global__ __launch_bounds__(kBlock, 4) void k_locate(LocateArgs<R> a) {
       atomicAdd(&a.walk_hist[(blockIdx.x & (kCounterStripes - 1)) * 64 + threadIdx.x],
                 (unsigned long long)shist[threadIdx.x]);
   }
+}
+
+template <typename R, bool EXACT, bool LINES>
+__global__ __launch_bounds__(kBlock, 4) void k_locate(LocateArgs<R> a) {
+  __shared__ int32_t shist[64];
+  __shared__ float4 stage[LINES ? kBlock * 8 : 1];
+  float4 *const my_stage = stage + (LINES ? (threadIdx.x & ~63) * 8 : 0);
+  if (threadIdx.x < 64) shist[threadIdx.x] = 0;
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+  const int64_t base = wave * a.chunk;
+  const int64_t end = base + a.chunk < a.n ? base + a.chunk : a.n;
+  int64_t cursor = base;
+  // a lane's state: no particle; walking; at a cell whose evaluation waits
+  // (kHold: FP64's owner, and what the filter does not certify); ended
+  enum : int { kIdle = 0, kWalk = 1, kHold = 2, kOwner = 3, kLost = 4 };
+  int ph = kIdle;
+  int32_t p = 0;  // n < 2^31
+  int ci = 0, cj = 0, ck = 0, steps = 0;
+  int32_t lc = 0;  // ci + IM (cj + JM ck); used only inside the grid
+  const int32_t sj = a.g.IM, sk = a.g.IM * a.g.JM;
+  const CellPlanes32 *const recs = EXACT ? a.filter : static_cast<const CellPlanes32 *>(a.planes);
+  int32_t saved = -1;  // cell of the walk's last power-of-two iteration (CycleGuard's test)
+  int held = 0;        // full evaluations of the walk that took it on
+  double x[3] = {0.0, 0.0, 0.0};
+  float d[6];
+  unsigned long long my_iters = 0;
+  unsigned long long my_fb = 0;
+  unsigned my_max = 0, my_loc = 0, my_lost = 0;
+  int my_err = 0;
+  const unsigned long long lane_mask_lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  auto step = [&](const auto dist[6]) {
+    int di, dj, dk;
+    step_of(dist, di, dj, dk);
+    ci += di;
+    cj += dj;
+    ck += dk;
+    lc += di + dj * sj + dk * sk;
+    ph = steps >= a.max_traversal ? kLost : kWalk;  // MAX_TRAVERSAL (:1206-1212)
+  };
+  // an iteration's tests before its evaluation (walkingsearch.c:1123-1132)
+  auto arrive = [&]() {
+    steps++;
+    if ((unsigned)ci >= (unsigned)a.g.IM || (unsigned)cj >= (unsigned)a.g.JM || (unsigned)ck >= (unsigned)a.g.KM) {
+      ph = kLost;  // walked outside the global domain: LOST
+    } else if (lc == saved) {
+      ph = kLost;  // periodic walk: LOST at MAX_TRAVERSAL (:1206-1212)
+      steps = a.max_traversal;
+    } else {
+      if ((steps & (steps - 1)) == 0) saved = lc;
+      ph = kHold;
+    }
+  };
+  while (true) {
+    const unsigned long long idle = __ballot(ph == kIdle);
+    if (idle != 0ull && cursor < end) {
+      if (ph == kIdle) {
+        const int64_t q = cursor + __popcll(idle & lane_mask_lt);
+        if (q < end) {
+          const int32_t pq = a.order ? a.order[q] : (int32_t)q;
+          const int32_t st = a.status[pq];
+          int32_t c = a.cell[pq];
+#pragma unroll
+          for (int t = 0; t < 3; ++t) x[t] = a.pos[3 * (int64_t)pq + t];
+          if (!(st == ST_LOCATED || (a.skip_lost && st == ST_LOST))) {
+            p = pq;
+            ph = kWalk;
+            if (c < 0 && a.guess) c = a.guess[pq];
+            ci = cj = ck = 0;  // (info.xs, info.ys, info.zs) on one rank, walkingsearch.c:611-616
+            if (c >= 0) unpack_cell(c, cell_idx(a.g), ci, cj, ck);
+            lc = c >= 0 ? c : 0;
+            steps = 0;
+            saved = -1;
+            held = 0;
+          } else if (a.steps_out) {
+            a.steps_out[pq] = 0;
+          }
+        }
+      }
+      cursor += __popcll(idle);
+    }
+    unsigned long long walking = __ballot(ph == kWalk);
+    if (walking != 0ull) {
+      // iterations of the walk (walkingsearch.c:1123-1203) until kStopped lanes have stopped
+      const int least = cursor < end ? 64 - kStopped : 0;
+      do {
+        bool eval = false;
+        if (ph == kWalk) {
+          arrive();
+          eval = ph == kHold;
+        }
+        auto decide = [&](const CellPlanes32 &rec) {
+          if (planes_fp32_certified(rec, x, d)) {
+            if (certified_outside(d))
+              step(d);
+            else if (!EXACT)
+              ph = kOwner;
+          }
+        };
+        if constexpr (LINES) {
+          const CellPlanes32 rec = wave_records(recs, eval ? lc : -1, my_stage, lane);
+          if (eval) decide(rec);
+        } else {
+          if (eval && (!EXACT || recs)) decide(recs[lc]);
+        }
+        walking = __ballot(ph == kWalk);
+      } while (__popcll(walking) > least);
+    }
+    const unsigned long long waiting = __ballot(ph == kHold);
+    if ((walking | waiting) == 0ull && __ballot(ph != kIdle) == 0ull && cursor >= end) break;
+    if (waiting != 0ull && (walking == 0ull || __popcll(waiting) >= kExactGroup)) {
+      // the last walks of a wavefront that are certified nowhere (a point within
+      // the filter's bound of a plane along the grid) stay here to their end
+      const bool last = walking == 0ull && cursor >= end;
+      while (ph == kHold) {
+        R df[6];
+        unsigned long long fb = 0;
+        if (!eval_cell_planes<R, EXACT>(a.planes, a.g, ci, cj, ck, x, a.thresh_scale, df, fb)) {
+          my_err = 1;
+          ph = kLost;
+        } else if (point_accepted<R>(df)) {
+          if constexpr (EXACT) {
+            R wv[3];
+            weights_from_distances<R>(df, a.clamp, wv);
+#pragma unroll
+            for (int t = 0; t < 3; ++t) a.w[3 * (int64_t)p + t] = wv[t];
+          } else {
+#pragma unroll
+            for (int t = 0; t < 6; ++t) d[t] = df[t];
+          }
+          ph = kOwner;
+        } else {
+          step(df);
+          if (++held > kHeld && last && ph == kWalk) arrive();
+        }
+        my_fb += fb;
+      }
+    }
+    if (ph >= kOwner) {
+      if (ph == kOwner) {
+        if constexpr (!EXACT) {
+          float wv[3];
+          weights_from_distances<float>(d, a.clamp, wv);
+#pragma unroll
+          for (int t = 0; t < 3; ++t) a.w[3 * (int64_t)p + t] = wv[t];
+        }
+        a.cell[p] = lc;
+        a.status[p] = ST_LOCATED;
+        my_loc++;
+      } else if (!my_err) {
+        a.cell[p] = -1;
+        a.status[p] = ST_LOST;
+        my_lost++;
+      }
+      if (a.steps_out) a.steps_out[p] = steps;
+      if (a.walk_hist) atomicAdd(&shist[steps < 63 ? steps : 63], 1);
+      my_iters += steps;
+      my_max = my_max > (unsigned)steps ? my_max : (unsigned)steps;
+      ph = kIdle;
+    }
+  }
+  locate_tally(a, base, lane, my_iters, my_fb, my_max, my_loc, my_lost, my_err, shist);
+}
+
+// The walk of few particles: G lanes a particle, which evaluate the next G
+// cells of its walk at once.  A launch of few particles is bound by the
+// latency of a walk's record loads, one after another, while most lanes of the
+// chip have no particle.  A walk mostly goes on in the direction of its last
+// step: lane m evaluates the cell m such steps ahead, and the walk takes the
+// lanes' steps as long as each is the predicted one, up to and with the first
+// that is not.  These are the cells, steps and iterations of the walk taken
+// one by one; an evaluation that the walk does not reach is dropped.
+// The group looks twice as far ahead as the row it has just taken, so that a
+// walk with many turns costs few loads.
+template <typename R, bool EXACT, int G>
+__global__ __launch_bounds__(kBlock, 4) void k_locate_ahead(LocateArgs<R> a) {
+  static_assert(G >= 2 && G <= 16 && (G & (G - 1)) == 0, "G lanes a particle");
+  constexpr unsigned kGroupMask = (1u << G) - 1u;
+  __shared__ int32_t shist[64];
+  if (threadIdx.x < 64) shist[threadIdx.x] = 0;
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int m = lane & (G - 1), first = lane & ~(G - 1);  // place in the group, the group's first lane
+  const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+  const int64_t base = wave * a.chunk;
+  const int64_t end = base + a.chunk < a.n ? base + a.chunk : a.n;
+  int64_t cursor = base;
+  // the same in every lane of a group, but for d in the lane of the owner
+  enum : int { kIdle = 0, kWalk = 1, kHold = 2, kOwner = 3, kLost = 4 };
+  int ph = kIdle;
+  int32_t p = 0;  // n < 2^31
+  int ci = 0, cj = 0, ck = 0, steps = 0;
+  int di = 0, dj = 0, dk = 0;  // the last step
+  int32_t lc = 0, dl = 0;      // cell and step in the linear index
+  int reach = 1;               // lanes that look ahead
+  int owner = 0;               // the lane (of the group) that holds the owner's distances
+  const int32_t sj = a.g.IM, sk = a.g.IM * a.g.JM;
+  const CellPlanes32 *const recs = EXACT ? a.filter : static_cast<const CellPlanes32 *>(a.planes);
+  int32_t saved = -1;  // cell of an earlier round (CycleGuard's test)
+  int round = 0;
+  int held = 0;        // full evaluations of the walk that took it on
+  double x[3] = {0.0, 0.0, 0.0};
+  float d[6];
+  unsigned long long my_iters = 0;
+  unsigned long long my_fb = 0;
+  unsigned my_max = 0, my_loc = 0, my_lost = 0;
+  int my_err = 0;
+  const unsigned long long groups_lt = first == 0 ? 0ull : (~0ull >> (64 - first));
+  auto move = [&](int count) {
+    ci += count * di;
+    cj += count * dj;
+    ck += count * dk;
+    lc += count * dl;
+  };
+  auto turn = [&]() {
+    dl = di + dj * sj + dk * sk;
+    move(1);
+    ph = steps >= a.max_traversal ? kLost : kWalk;  // MAX_TRAVERSAL (:1206-1212)
+  };
+  while (true) {
+    const unsigned long long idle = __ballot(ph == kIdle);
+    if (idle != 0ull && cursor < end) {
+      if (ph == kIdle) {
+        const int64_t q = cursor + __popcll(idle & groups_lt) / G;
+        if (q < end) {
+          const int32_t st = a.status[q];
+          int32_t c = a.cell[q];
+#pragma unroll
+          for (int t = 0; t < 3; ++t) x[t] = a.pos[3 * q + t];
+          if (!(st == ST_LOCATED || (a.skip_lost && st == ST_LOST))) {
+            p = (int32_t)q;
+            ph = kWalk;
+            if (c < 0 && a.guess) c = a.guess[q];
+            ci = cj = ck = 0;  // (info.xs, info.ys, info.zs) on one rank, walkingsearch.c:611-616
+            if (c >= 0) unpack_cell(c, cell_idx(a.g), ci, cj, ck);
+            lc = c >= 0 ? c : 0;
+            di = dj = dk = 0;
+            dl = 0;
+            reach = 1;
+            steps = 0;
+            saved = -1;
+            round = 0;
+            held = 0;
+          } else if (a.steps_out && m == 0) {
+            a.steps_out[q] = 0;
+          }
+        }
+      }
+      cursor += __popcll(idle) / G;
+    }
+    unsigned long long walking = __ballot(ph == kWalk);
+    if (walking != 0ull) {
+      const int least = cursor < end ? 64 - kStopped : 0;
+      do {
+        // up to G iterations of each group's walk (walkingsearch.c:1123-1203)
+        enum : int { STEP = 0, OUT = 1, HOLD = 2, OWNER = 3 };
+        int kind = HOLD, si = 0, sj_ = 0, sk_ = 0;
+        bool periodic = false;
+        if (ph == kWalk) {
+          const int i = ci + m * di, j = cj + m * dj, k = ck + m * dk;
+          if ((unsigned)i >= (unsigned)a.g.IM || (unsigned)j >= (unsigned)a.g.JM ||
+              (unsigned)k >= (unsigned)a.g.KM) {
+            kind = OUT;  // walked outside the global domain: LOST (:1127-1132)
+          } else if (m < reach && planes_fp32_certified(recs[lc + m * dl], x, d)) {
+            if (certified_outside(d)) {
+              kind = STEP;
+              step_of<float>(d, si, sj_, sk_);
+            } else if (!EXACT) {
+              kind = OWNER;
+            }
+          }
+        }
+        // (the lanes beyond reach break the row of predicted steps)
+        const bool predicted = m + 1 < reach && kind == STEP && si == di && sj_ == dj && sk_ == dk;
+        const unsigned go = (unsigned)(__ballot(predicted) >> first) & kGroupMask;
+        const int len = __ffs(~go) - 1;  // < reach
+        // the evaluation after the predicted ones, one number for its kind and step
+        const int at = __shfl(kind | (si + 1) << 2 | (sj_ + 1) << 4 | (sk_ + 1) << 6, first + len);
+        if (ph == kWalk) {
+          // out of the domain, lc is no cell (the kind tells)
+          periodic = lc == saved && !(len == 0 && (at & 3) == OUT);
+          if ((round & (round + 1)) == 0) saved = (len == 0 && (at & 3) == OUT) ? -1 : lc;
+          ++round;
+          if (periodic || len >= a.max_traversal - steps) {
+            steps = a.max_traversal;  // LOST there, and a periodic walk at once (:1206-1212)
+            ph = kLost;
+          } else {
+            steps += len + 1;
+            move(len);
+            reach = 2 * len + 2 < G ? 2 * len + 2 : G;
+            if ((at & 3) == STEP) {
+              di = ((at >> 2) & 3) - 1;
+              dj = ((at >> 4) & 3) - 1;
+              dk = ((at >> 6) & 3) - 1;
+              turn();
+            } else {
+              ph = (at & 3) == OUT ? kLost : (at & 3) == HOLD ? kHold : kOwner;
+              owner = len;
+            }
+          }
+        }
+        walking = __ballot(ph == kWalk);
+      } while (__popcll(walking) > least);
+    }
+    const unsigned long long waiting = __ballot(ph == kHold);
+    if ((walking | waiting) == 0ull && __ballot(ph != kIdle) == 0ull && cursor >= end) break;
+    if (waiting != 0ull && (walking == 0ull || __popcll(waiting) >= kExactGroup)) {
+      // what the filter does not certify (and in FP64 the owner) in full, one
+      // cell, or G ahead once that has taken the walk on
+      R df[6];
+      unsigned long long fb = 0;
+      enum : int { STEP = 0, OUT = 1, ERROR = 2, OWNER = 3 };
+      int kind = ERROR, si = 0, sj_ = 0, sk_ = 0;
+      const int i = ci + m * di, j = cj + m * dj, k = ck + m * dk;
+      const bool reached = m == 0 || held > 0;
+      if (ph == kHold) {
+        if ((unsigned)i >= (unsigned)a.g.IM || (unsigned)j >= (unsigned)a.g.JM || (unsigned)k >= (unsigned)a.g.KM) {
+          kind = OUT;
+        } else if (reached &&
+                   eval_cell_planes<R, EXACT>(a.planes, a.g, i, j, k, x, a.thresh_scale, df, fb)) {
+          kind = OWNER;
+          if (!point_accepted<R>(df)) {
+            kind = STEP;
+            step_of<R>(df, si, sj_, sk_);
+          }
+        }
+      }
+      const bool predicted = m + 1 < G && held > 0 && kind == STEP && si == di && sj_ == dj && sk_ == dk;
+      const unsigned go = (unsigned)(__ballot(predicted) >> first) & kGroupMask;
+      const int len = __ffs(~go) - 1;
+      const int at = __shfl(kind | (si + 1) << 2 | (sj_ + 1) << 4 | (sk_ + 1) << 6, first + len);
+      if (ph == kHold) {
+        if (m <= len) my_fb += fb;
+        if (len > a.max_traversal - steps) {  // (the first of these iterations is counted in steps)
+          steps = a.max_traversal;
+          ph = kLost;
+        } else {
+          steps += len;
+          move(len);
+          const int kd = at & 3;
+          if (kd == STEP) {
+            di = ((at >> 2) & 3) - 1;
+            dj = ((at >> 4) & 3) - 1;
+            dk = ((at >> 6) & 3) - 1;
+            reach = 1;
+            ++held;
+            turn();
+          } else if (kd == OWNER) {
+            if (m == len) {
+              R wv[3];
+              weights_from_distances<R>(df, a.clamp, wv);
+#pragma unroll
+              for (int t = 0; t < 3; ++t) a.w[3 * (int64_t)p + t] = wv[t];
+            }
+            owner = -1;
+            ph = kOwner;
+          } else {
+            if (kd == ERROR) my_err = 1;
+            ph = kLost;
+          }
+        }
+      }
+    }
+    if (ph >= kOwner) {
+      if constexpr (!EXACT) {
+        if (ph == kOwner && m == owner) {
+          float wv[3];
+          weights_from_distances<float>(d, a.clamp, wv);
+#pragma unroll
+          for (int t = 0; t < 3; ++t) a.w[3 * (int64_t)p + t] = wv[t];
+        }
+      }
+      if (m == 0) {
+        if (ph == kOwner) {
+          a.cell[p] = lc;
+          a.status[p] = ST_LOCATED;
+          my_loc++;
+        } else if (!my_err) {
+          a.cell[p] = -1;
+          a.status[p] = ST_LOST;
+          my_lost++;
+        }
+        if (a.steps_out) a.steps_out[p] = steps;
+        if (a.walk_hist) atomicAdd(&shist[steps < 63 ? steps : 63], 1);
+        my_iters += steps;
+        my_max = my_max > (unsigned)steps ? my_max : (unsigned)steps;
+      }
+      ph = kIdle;
+    }
+  }
+  locate_tally(a, base, lane, my_iters, my_fb, my_max, my_loc, my_lost, my_err, shist);
 }
 
 // ---------------------------------------------------------------------------

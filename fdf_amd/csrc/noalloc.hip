@@ -90,7 +90,7 @@ extern "C" int picgpu_locate_device_noalloc(picgpu_ctx *c, int64_t n, const doub
                      ptr, (int64_t)kScratchWords);
   PG_HIP(hipGetLastError());
   if (n > 0) {
-    const int64_t chunk = locate_chunk(n), blocks = locate_blocks(n, chunk);
+    const int64_t chunk = locate_chunk(n, 1), blocks = locate_blocks(n, chunk);
     auto launch = [&](auto *tag) -> int {
       using R = std::remove_pointer_t<decltype(tag)>;
       LocateArgs<R> a;
@@ -113,7 +113,7 @@ extern "C" int picgpu_locate_device_noalloc(picgpu_ctx *c, int64_t n, const doub
       a.clamp = (R)c->opt.weight_clamp;
       a.skip_lost = 0;
       constexpr bool EX = sizeof(R) == sizeof(double);
-      hipLaunchKernelGGL((k_locate<R, EX>), dim3((unsigned)blocks), dim3(kBlock), 0, c->stream, a);
+      hipLaunchKernelGGL((k_locate<R, EX, false>), dim3((unsigned)blocks), dim3(kBlock), 0, c->stream, a);
       PG_HIP(hipGetLastError());
       return PICGPU_OK;
     };

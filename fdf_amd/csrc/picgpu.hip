@@ -392,6 +392,7 @@ int picgpu_init_particles_device(picgpu_ctx *c, int64_t n, const double *d_pos, 
   c->sorted = c->keyed = c->key_ordered = c->compact_pending = false;
   c->swarm_invalid = false;
   c->pid32_valid = false;
+  c->cells_unset = true;
   if (n == 0) return PICGPU_OK;
   int r = dispatch_real(c, [&](auto *tag) -> int {
     using R = std::remove_pointer_t<decltype(tag)>;
@@ -450,6 +451,9 @@ int picgpu_upload_particles(picgpu_ctx *c, int64_t n, const double *pos, const d
   c->sorted = c->keyed = c->key_ordered = c->compact_pending = false;
   c->swarm_invalid = false;
   c->pid32_valid = false;
+  // a few of them tell how far the walks go: the launch depends on it, the results do not
+  c->cells_unset = true;
+  for (int q = 0; q < 16 && c->cells_unset && n > 0; ++q) c->cells_unset = cell[3 * ((n - 1) * q / 15)] < 0;
   if (n == 0) return PICGPU_OK;
   HostSeg seg[7];
   int m = 0;
@@ -612,8 +616,11 @@ static int do_locate(picgpu_ctx *c, int skip_lost) {
       PG_CHECK(build_key_index(c, guess));
       if (c->n_live == n) order = c->kidx[c->kcur].as<int32_t>();
     }
+    const bool records = c->opt.precision == PICGPU_FP32 || c->have_filter;
+    const bool from_origin = records && c->cells_unset && !guess;
+    const int ahead = from_origin && std::max(c->IM, std::max(c->JM, c->KM)) >= kLocateLong ? locate_ahead(n) : 1;
+    const bool lines = from_origin && n >= kLocateLines;
     unsigned long long *hist = hist_reset(c);
-    const int64_t chunk = locate_chunk(n), blocks = locate_blocks(n, chunk);
     int r = dispatch_real(c, [&](auto *tag) -> int {
       using R = std::remove_pointer_t<decltype(tag)>;
       LocateArgs<R> a;
@@ -621,7 +628,7 @@ static int do_locate(picgpu_ctx *c, int skip_lost) {
       a.planes = c->planes.ptr;
       a.filter = c->have_filter ? c->filter.as<CellPlanes32>() : nullptr;
       a.n = n;
-      a.chunk = chunk;
+      a.chunk = locate_chunk(n, ahead);
       a.pos = c->sw.pos.as<double>();
       a.cell = c->sw.cell.as<int32_t>();
       a.w = c->sw.w.as<R>();
@@ -636,7 +643,16 @@ static int do_locate(picgpu_ctx *c, int skip_lost) {
       a.clamp = (R)c->opt.weight_clamp;
       a.skip_lost = skip_lost;
       constexpr bool EX = sizeof(R) == sizeof(double);
-      PG_LAUNCH(c, EX ? "locate_fp64" : "locate_fp32", blocks, kBlock, (k_locate<R, EX>), a);
+      const char *name = EX ? "locate_fp64" : "locate_fp32";
+      const int64_t blocks = locate_blocks(n, a.chunk);
+      if (ahead == 16)
+        PG_LAUNCH(c, name, blocks, kBlock, (k_locate_ahead<R, EX, 16>), a);
+      else if (ahead == 4)
+        PG_LAUNCH(c, name, blocks, kBlock, (k_locate_ahead<R, EX, 4>), a);
+      else if (lines)
+        PG_LAUNCH(c, name, blocks, kBlock, (k_locate<R, EX, true>), a);
+      else
+        PG_LAUNCH(c, name, blocks, kBlock, (k_locate<R, EX, false>), a);
       return PICGPU_OK;
     });
     PG_CHECK(r);
@@ -654,6 +670,7 @@ static int do_locate(picgpu_ctx *c, int skip_lost) {
   c->stats.lost = (int64_t)h[C_LOST];
   if (n > 0) PG_CHECK(hist_read(c));
   c->sorted = c->keyed = c->key_ordered = c->compact_pending = false;
+  c->cells_unset = false;
   return PICGPU_OK;
 }
 

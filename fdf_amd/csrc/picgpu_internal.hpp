@@ -152,6 +152,7 @@ struct picgpu_ctx {
   picgpu::DevBuf guess;     // int32 [n] MLP start cell
   picgpu::DevBuf pos0, vel0;// RK2 saved state
   bool sorted = false;      // particles sorted by cell, cell_start valid
+  bool cells_unset = false; // the particles have no cells yet: the next locate's walks start in cell (0,0,0)
   int64_t n_live = 0;       // particles not removed (equals n outside picgpu_step)
   int steps_since_compact = 0;
 

@@ -186,6 +186,12 @@ __device__ __forceinline__ bool point_accepted(const R d[6]) {
 
 // walkingsearch.c:919-946
 template <typename R>
+__device__ __forceinline__ void step_of(const R d[6], int &di, int &dj, int &dk) {
+  dk = d[F_FRONT] < (R)0 ? 1 : d[F_BACK] < (R)0 ? -1 : 0;
+  di = d[F_LEFT] < (R)0 ? -1 : d[F_RIGHT] < (R)0 ? 1 : 0;
+  dj = d[F_BOTTOM] < (R)0 ? -1 : d[F_TOP] < (R)0 ? 1 : 0;
+}
+template <typename R>
 __device__ __forceinline__ void step_indices(const R d[6], int &i, int &j, int &k) {
   if (d[F_FRONT] < (R)0)
     k += 1;
@@ -483,6 +489,29 @@ __device__ __forceinline__ unsigned planes_fp32_distances(const CellPlanes32 &r,
   need |= plane_fp32<4>(r, q, band, d) ? 0u : 16u;
   need |= plane_fp32<5>(r, q, band, d) ? 0u : 32u;
   return need;
+}
+
+// The same distances where only one question is asked of the bound: does it
+// certify every face?  A NaN position gives six NaN distances, an infinite or
+// overflowing one an infinite band, so the minimum hides no NaN.
+__device__ __forceinline__ bool planes_fp32_certified(const CellPlanes32 &r, const double p[3], float d[6]) {
+  const float q[3] = {(float)(p[0] - r.v0[0]), (float)(p[1] - r.v0[1]), (float)(p[2] - r.v0[2])};
+  const float Q = fmaxf(fabsf(q[0]), fmaxf(fabsf(q[1]), fabsf(q[2])));
+  const float u = 5.9604645e-08f;  // 2^-24
+  const float band = r.thr + u * (4.f * r.amax + 16.f * Q);
+  plane_fp32<0>(r, q, band, d);
+  plane_fp32<1>(r, q, band, d);
+  plane_fp32<2>(r, q, band, d);
+  plane_fp32<3>(r, q, band, d);
+  plane_fp32<4>(r, q, band, d);
+  plane_fp32<5>(r, q, band, d);
+  const float least = fminf(fminf(fminf(fabsf(d[0]), fabsf(d[1])), fminf(fabsf(d[2]), fabsf(d[3]))),
+                            fminf(fabsf(d[4]), fabsf(d[5])));
+  return least > band;
+}
+// Certified distances: is some face's negative, so that the walk goes on?
+__device__ __forceinline__ bool certified_outside(const float d[6]) {
+  return fminf(fminf(fminf(d[0], d[1]), fminf(d[2], d[3])), fminf(d[4], d[5])) < 0.f;
 }
 
 __device__ __forceinline__ FilterResult eval_planes_fp32(const CellPlanes32 &r, const GridView &g, int i, int j, int k,
