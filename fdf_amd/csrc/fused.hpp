@@ -207,6 +207,7 @@ enum EvalOutcome : int { EV_OK = 0, EV_DEGENERATE = 1, EV_DEFER = 2 };
 
 template <typename R, bool TILE, bool DEFER = false>
 struct PlaneSrc {
+  static constexpr bool kCertified = DEFER;  // eval's distances are certified where it gives EV_OK
   GridView g;
   const R *corner;
   const typename PlanesOf<R>::type *planes;
@@ -217,7 +218,7 @@ struct PlaneSrc {
                                       unsigned long long &fb) const {
     if constexpr (DEFER && !EXACT) {
       const int64_t c = (int64_t)i + (int64_t)g.IM * ((int64_t)j + (int64_t)g.JM * k);
-      return planes_fp32_distances(planes[c], x, d) ? EV_DEFER : EV_OK;
+      return planes_fp32_certified(planes[c], x, d) ? EV_OK : EV_DEFER;
     } else {
       return eval_cell_planes<R, EXACT>(planes, g, i, j, k, x, ts, d, fb) ? EV_OK : EV_DEGENERATE;
     }
@@ -227,7 +228,7 @@ struct PlaneSrc {
   __device__ __forceinline__ int eval_lin(int i, int j, int k, int32_t lc, const double x[3], double ts, R d[6],
                                           unsigned long long &fb) const {
     if constexpr (DEFER && !EXACT) {
-      return planes_fp32_distances(planes[lc], x, d) ? EV_DEFER : EV_OK;
+      return planes_fp32_certified(planes[lc], x, d) ? EV_OK : EV_DEFER;
     } else if constexpr (EXACT) {
       return eval_planes_exact(planes[lc], x, d) ? EV_OK : EV_DEGENERATE;
     } else {
@@ -301,6 +302,15 @@ __global__ __launch_bounds__(kBlock) void k_cell_planes32(GridView g, double thr
 // revisited cell: the reference would cycle until MAX_TRAVERSAL).
 enum WalkOutcome : int { W_LOCATED = 0, W_LOST = 1, W_DEGENERATE = 2, W_CONTINUE = 3, W_DEFER = 4 };
 
+// point_accepted; certified FP32 distances are never zero
+template <typename R, bool CERTIFIED>
+__device__ __forceinline__ bool accepted(const R d[6]) {
+  if constexpr (CERTIFIED && sizeof(R) == sizeof(float))
+    return !certified_outside(d);
+  else
+    return point_accepted<R>(d);
+}
+
 template <typename R, bool EXACT, class Src>
 __device__ __forceinline__ int walk_iter(const Src &src, const double x[3], int &ci, int &cj, int &ck, int &steps,
                                          CycleGuard &cyc, int max_traversal, double thresh_scale, R clamp, R wv[3],
@@ -317,7 +327,7 @@ __device__ __forceinline__ int walk_iter(const Src &src, const double x[3], int 
   const int ev = src.template eval<EXACT>(ci, cj, ck, x, thresh_scale, d, fallbacks);
   if (ev == EV_DEGENERATE) return W_DEGENERATE;
   if (ev == EV_DEFER) return W_DEFER;
-  if (point_accepted<R>(d)) {
+  if (accepted<R, Src::kCertified>(d)) {
     weights_from_distances<R>(d, clamp, wv);
     return W_LOCATED;
   }
@@ -347,7 +357,7 @@ __device__ __forceinline__ int walk_iter_lin(const Src &src, const double x[3], 
   const int ev = src.template eval_lin<EXACT>(ci, cj, ck, lc, x, thresh_scale, d, fallbacks);
   if (ev == EV_DEGENERATE) return W_DEGENERATE;
   if (ev == EV_DEFER) return W_DEFER;
-  if (point_accepted<R>(d)) {
+  if (accepted<R, Src::kCertified>(d)) {
     weights_from_distances<R>(d, clamp, wv);
     return W_LOCATED;
   }
@@ -404,7 +414,8 @@ __device__ __forceinline__ void interp_at(const Src &src, int ci, int cj, int ck
 }
 
 struct StepTally {
-  unsigned long long located = 0, lost = 0, oob = 0, iters = 0, fb = 0;
+  unsigned located = 0, lost = 0, oob = 0;
+  unsigned long long iters = 0, fb = 0;
   int err = 0;
 };
 
@@ -517,7 +528,7 @@ __device__ __forceinline__ void step_particle(const StepArgs<R> &a, const Src &s
 // lane's particle counts fit 32 bits, so the wave sums them in 32 bits (one
 // shuffle per step instead of two); walk iterations keep 64.
 __device__ __forceinline__ void flush_tally(StepTally &t, unsigned long long *counters) {
-  unsigned v_loc = (unsigned)t.located, v_lost = (unsigned)t.lost, v_oob = (unsigned)t.oob, v_fb = (unsigned)t.fb;
+  unsigned v_loc = t.located, v_lost = t.lost, v_oob = t.oob, v_fb = (unsigned)t.fb;
   unsigned long long v_it = t.iters;
   const bool any_err = __any(t.err != 0);
   for (int off = 32; off > 0; off >>= 1) {
@@ -648,7 +659,7 @@ __device__ __forceinline__ void start_state(const StepArgs<R> &a, const Src &src
   if constexpr (EXACT)
     eval_planes_exact(src.planes[lc], x0, d);
   else
-    certain = planes_fp32_distances(src.planes[lc], x0, d) == 0u;
+    certain = planes_fp32_certified(src.planes[lc], x0, d);
   if (certain) {
     weights_from_distances<R>(d, a.clamp, w0);
     interp_at<R>(src, ci, cj, ck, w0, u0);
@@ -914,7 +925,7 @@ __global__ __launch_bounds__(kBlock, sizeof(R) == 4 ? 4 : 1) void k_step_tiled(
         if constexpr (EXACT)
           return eval_planes_exact(src.planes[lc], x, d);
         else
-          return planes_fp32_distances(rec32, x, d) == 0u;
+          return planes_fp32_certified(rec32, x, d);
       };
       if (recompute) {
         R d0[6], w0[3];
@@ -935,7 +946,7 @@ __global__ __launch_bounds__(kBlock, sizeof(R) == 4 ? 4 : 1) void k_step_tiled(
       for (int c = 0; c < 3; ++c) x1[c] = ps.x0[c] + (double)ps.u0[c] * a.dt;
       R d[6];
       bool cert = dist(x1, d);
-      fast = cert && point_accepted<R>(d);
+      fast = cert && accepted<R, !EXACT>(d);
       bool corr = !RK2;  // the walk in progress is the corrector (Euler: the only walk)
       // One step of the walk, taken here: the walk in progress evaluated its
       // cell (certified, not accepted); it steps to the neighbour by
@@ -955,7 +966,7 @@ __global__ __launch_bounds__(kBlock, sizeof(R) == 4 ? 4 : 1) void k_step_tiled(
           lc += di + dj * a.g.IM + dk * (a.g.IM * a.g.JM);
           if constexpr (!EXACT) rec32 = src.planes[lc];
           cert = dist(x1, d);
-          fast = cert && point_accepted<R>(d);
+          fast = cert && accepted<R, !EXACT>(d);
           mv = corr ? 2 : 1;
         }
       };
@@ -968,7 +979,7 @@ __global__ __launch_bounds__(kBlock, sizeof(R) == 4 ? 4 : 1) void k_step_tiled(
         for (int c = 0; c < 3; ++c) x1[c] = ps.x0[c] + ((double)ps.u0[c] + (double)us[c]) * h;
         corr = true;
         cert = dist(x1, d);  // the corrector walk starts in the predictor's cell
-        fast = cert && point_accepted<R>(d);
+        fast = cert && accepted<R, !EXACT>(d);
         if (cert && !fast && mv == 0) step_once();
       }
       if (!fast) {
