@@ -1226,12 +1226,16 @@ __global__ __launch_bounds__(kBlock, sizeof(R) == 4 ? 4 : 1) void k_step_tiled(
 // the steps do not make): every particle's weights and velocity at its
 // position and cell, written to w and vel, and, with a.deposit, the face
 // deposition of that state.  One workgroup per tile, as k_step_tiled.
-template <typename R, bool EXACT>
+//
+// STORED: the step wrote the weights and velocities (k_step_list); the pass
+// only deposits them.
+template <typename R, bool EXACT, bool STORED>
 __global__ __launch_bounds__(kBlock) void k_step_finish(StepArgs<R> a, const int32_t *__restrict__ idx,
                                                         const int32_t *__restrict__ kstart) {
-  constexpr int CAPD = DepCap<R>::value;
-  __shared__ R sk[BN * 3];
-  __shared__ R sdx[StageLen<R, false>::value];
+  // STORED: tiles of few particles, and no more LDS than the exchange takes
+  constexpr int CAPD = STORED ? 2 * TS : DepCap<R>::value;
+  __shared__ R sk[STORED ? 1 : BN * 3];
+  __shared__ R sdx[STORED ? 12 * TS : StageLen<R, false>::value];
   R(*const sd)[6] = reinterpret_cast<R(*)[6]>(sdx);
   R(*const xch)[TS] = reinterpret_cast<R(*)[TS]>(sdx);
   const int t = step_tile(blockIdx.x, a.tm);
@@ -1241,7 +1245,17 @@ __global__ __launch_bounds__(kBlock) void k_step_finish(StepArgs<R> a, const int
   PlaneSrc<R, true, !EXACT> src{a.g, a.corner, (const typename PlanesOf<R>::type *)a.planes, (lds_ptr<R>)sk,
                                 ti * TX - 1, tj * TY - 1, tk * TZ - 1};
   const int32_t B = (int32_t)blockDim.x;
-  if (s < e) {
+  if constexpr (STORED) {
+    // the first CAPD of them to LDS, as tile_face_sums reads them
+    for (int32_t q = s + (int32_t)threadIdx.x; q < e && q - s < CAPD; q += B) {
+      const int64_t p = idx[q];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        sd[q - s][c] = a.w[3 * p + c];
+        sd[q - s][3 + c] = a.vel[3 * p + c];
+      }
+    }
+  } else if (s < e) {
     int32_t q = s + (int32_t)threadIdx.x;
     int32_t p = q < e ? idx[q] : -1;
     int32_t pn = q + B < e ? idx[q + B] : -1;
@@ -1372,13 +1386,15 @@ __global__ __launch_bounds__(kBlock) void k_step_deferred(StepArgs<R> a, int dbl
   flush_tally(tally, a.counters);
 }
 
-// Particles idx[q0 .. q1) from global memory (particles without a cell).
+// Particles idx[q0 .. q1) from global memory: those without a cell, or, where
+// a tile holds few particles (sparse_steps in picgpu.hip), all of them, q1 then
+// their number on the device (m_dev).
 template <typename R, bool EXACT, bool RK2>
 __global__ __launch_bounds__(kBlock) void k_step_list(StepArgs<R> a, const int32_t *__restrict__ idx, int64_t q0,
-                                                      int64_t q1) {
+                                                      int64_t q1, const int32_t *__restrict__ m_dev) {
   const int64_t q = q0 + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   StepTally tally;
-  if (q < q1) {
+  if (q < (m_dev ? (int64_t)*m_dev : q1)) {
     const int64_t p = idx[q];
     PState<R> ps;
     load_state(a, p, ps);

@@ -1065,10 +1065,10 @@ static constexpr size_t kStepCounterWords = (size_t)kCounterStripes * C_NUM;
 // last: the call's last step, which compacts with weights and statuses if the
 // schedule falls on it.  counters: this step's counter block.  *compacted:
 // set when this step compacted the swarm.
-static int do_step_fused(picgpu_ctx *c, double dt, unsigned flags, int step, bool last,
+static int do_step_fused(picgpu_ctx *c, double dt, unsigned flags, int step, bool last, bool sparse,
                          unsigned long long *counters, bool *compacted, int64_t *entries) {
   const bool rk2 = (flags & PICGPU_STEP_RK2) != 0;
-  const bool wu = (flags & PICGPU_STEP_FIELDS) != 0;
+  const bool fields = (flags & PICGPU_STEP_FIELDS) != 0, wu = fields || sparse;
   const bool faces = (flags & PICGPU_STEP_DEPOSIT_FACES) != 0;
   *compacted = false;
   PG_CHECK(ensure_planes(c));
@@ -1123,9 +1123,14 @@ static int do_step_fused(picgpu_ctx *c, double dt, unsigned flags, int step, boo
       const int64_t dblocks = std::min<int64_t>(1024, nblocks(n));
       auto launch = [&](auto rk2_tag, auto wu_tag) -> int {
         constexpr bool RK = decltype(rk2_tag)::value, WU = decltype(wu_tag)::value;
+        if (sparse) {
+          PG_LAUNCH(c, name, nblocks(n), kBlock, (k_step_list<R, EX, RK>), a, idx, (int64_t)0, (int64_t)0, m_dev);
+          return PICGPU_OK;
+        }
         PG_LAUNCH(c, name, nt, kBlock, (k_step_tiled<R, EX, RK, WU>), a, idx, kstart, kbase);
         if (fresh && u1 > u0)
-          PG_LAUNCH(c, name_list, nblocks(u1 - u0), kBlock, (k_step_list<R, EX, RK>), a, idx, u0, u1);
+          PG_LAUNCH(c, name_list, nblocks(u1 - u0), kBlock, (k_step_list<R, EX, RK>), a, idx, u0, u1,
+                    (const int32_t *)nullptr);
         const SeamCounts sc = dep ? seam_counts(c) : SeamCounts{0, 0, 0};
         if (dblocks + sc.total() > 0)
           PG_LAUNCH(c, sc.total() ? "face_seams" : "step_deferred", dblocks + nblocks(sc.total()), kBlock,
@@ -1177,7 +1182,7 @@ static int do_step_fused(picgpu_ctx *c, double dt, unsigned flags, int step, boo
   c->kcur = nxt;
   c->kbegin_unloc = c->kend_unloc = -1;  // known after the call's counters are read
   // weights and velocities were written: the step's deposition is a pass of its own
-  if (wu && faces) PG_CHECK(launch_deposit_tiles(c, nstart, nidx));
+  if (fields && faces) PG_CHECK(launch_deposit_tiles(c, nstart, nidx));
   c->steps_since_compact++;
   c->compact_pending = true;
   if (c->steps_since_compact >= kCompactEvery) {
@@ -1199,8 +1204,11 @@ static int do_step_fused(picgpu_ctx *c, double dt, unsigned flags, int step, boo
 // After the last step of a call (weights and velocities not kept between
 // steps): every particle's weights and velocity at its final position, and
 // the last step's face deposition.
-static int finish_step_call(picgpu_ctx *c, unsigned flags, unsigned long long *counters) {
+// stored: they were kept (sparse steps); only the deposition is left, of the
+// last step or, before a later one, of the step before it.
+static int finish_step_call(picgpu_ctx *c, unsigned flags, bool stored, bool last, unsigned long long *counters) {
   const bool faces = (flags & PICGPU_STEP_DEPOSIT_FACES) && !(flags & PICGPU_STEP_FACES_OF_START);
+  if (stored && !faces) return PICGPU_OK;
   const TileMap tm = tile_map(c);
   const int64_t nt = ntiles(tm);
   alignas(16) unsigned char fo_buf[sizeof(FaceOut<double>)];
@@ -1212,9 +1220,13 @@ static int finish_step_call(picgpu_ctx *c, unsigned flags, unsigned long long *c
     a.deposit = faces ? 1 : 0;
     if (faces) a.fo = *reinterpret_cast<const FaceOut<R> *>(fo_buf);
     constexpr bool EX = sizeof(R) == sizeof(double);
-    PG_LAUNCH(c, EX ? "step_finish_fp64" : "step_finish_fp32", nt, kBlock, (k_step_finish<R, EX>), a,
-              c->kidx[c->kcur].as<int32_t>(), c->kstart[c->kcur].as<int32_t>());
-    return PICGPU_OK;
+    const char *name = !last ? "step_deposit" : EX ? "step_finish_fp64" : "step_finish_fp32";
+    auto launch = [&](auto st) -> int {
+      PG_LAUNCH(c, name, nt, kBlock, (k_step_finish<R, EX, decltype(st)::value>), a,
+                c->kidx[c->kcur].as<int32_t>(), c->kstart[c->kcur].as<int32_t>());
+      return PICGPU_OK;
+    };
+    return stored ? launch(std::true_type{}) : launch(std::false_type{});
   });
   PG_CHECK(r);
   if (faces) {
@@ -1224,10 +1236,34 @@ static int finish_step_call(picgpu_ctx *c, unsigned flags, unsigned long long *c
   return PICGPU_OK;
 }
 
+// A tile's workgroup pays the same chain of loads for 5 particles as for 500,
+// and four of them fit on a CU.  Where a tile holds few particles a lane a
+// particle over the index (k_step_list) is faster: it writes weights and
+// velocities, and the previous step's faces are a pass of their own.  The line,
+// from 16-step calls (us a step, tiles -> list):
+//   particles a cell              0.08         0.36-0.38     0.51         0.73-0.75    0.95
+//   128x128x192 FP32 RK2          191 -> 106   257 -> 203    274 -> 233   309 -> 307   344 -> 387
+//                    with faces   246 -> 177   301 -> 275    316 -> 307   350 -> 384   383 -> 476
+//   128x128x192 FP64 RK2          307 -> 180   412 -> 367    453 -> 425   535 -> 551   617 -> 690
+//                    with faces   436 -> 327   537 -> 515    580 -> 577   667 -> 707   746 -> 851
+//   61x45x131 FP32 with faces      60 ->  51                 74 ->  61    78 ->  68
+//   61x45x131 FP64 with faces      79 ->  64                 91 ->  86    99 ->  99
+// In a grid of up to kFewTiles tiles (a few rounds on the chip) the line with
+// faces lies where it does without.  Up to kFewParticles the list is faster at
+// any density (24x24x24: 30,000 58 -> 49 in FP32 with faces, 100,000 111 -> 95).
+static constexpr int64_t kFewTiles = 4096, kFewParticles = 65536;
+static bool sparse_steps(const picgpu_ctx *c, unsigned flags) {
+  if (flags & PICGPU_STEP_FACES_OF_START) return false;  // the faces that the tiles' last launch leaves
+  const bool faces = (flags & PICGPU_STEP_DEPOSIT_FACES) != 0;
+  const int64_t n = live_particles(c);
+  if (n <= kFewParticles) return true;
+  return faces && ntiles(tile_map(c)) > kFewTiles ? 2 * n < c->ncell : 4 * n < 3 * c->ncell;
+}
+
 // Fused steps s0 .. s0 + nb - 1 of a call of nsteps: queued, then one read of
 // their counters, which settles the live count, the array length after a
 // compaction and the statistics.
-static int step_batch(picgpu_ctx *c, double dt, unsigned flags, int s0, int nb, int nsteps) {
+static int step_batch(picgpu_ctx *c, double dt, unsigned flags, int s0, int nb, int nsteps, bool sparse) {
   const bool fields = (flags & PICGPU_STEP_FIELDS) != 0;
   PG_CHECK(c->step_counters.ensure(sizeof(unsigned long long) * kStepCounterWords * kStepBatch));
   PG_HIP(hipMemsetAsync(c->step_counters.ptr, 0, sizeof(unsigned long long) * kStepCounterWords * (size_t)nb,
@@ -1241,14 +1277,16 @@ static int step_batch(picgpu_ctx *c, double dt, unsigned flags, int s0, int nb, 
     const int s = s0 + b;
     if (fields) PG_CHECK(eulerian_fields_async(c));
     PG_CHECK(do_center_to_corner(c, c->kcount.as<int32_t>(), nkeys + 2));
+    unsigned long long *const sc = ctr + (size_t)b * kStepCounterWords;
+    if (sparse && !fields && s > 0) PG_CHECK(finish_step_call(c, flags, true, false, sc));
     bool compacted = false;
     int64_t entries = 0;
-    PG_CHECK(do_step_fused(c, dt, flags, s, s == nsteps - 1, ctr + (size_t)b * kStepCounterWords, &compacted,
-                           &entries));
+    PG_CHECK(do_step_fused(c, dt, flags, s, s == nsteps - 1, sparse, sc, &compacted, &entries));
     if (b == 0) m0 = entries;
     if (compacted) compacted_at = b;
   }
-  if (!fields && s0 + nb == nsteps) PG_CHECK(finish_step_call(c, flags, ctr + (size_t)(nb - 1) * kStepCounterWords));
+  if (!fields && s0 + nb == nsteps)
+    PG_CHECK(finish_step_call(c, flags, sparse, true, ctr + (size_t)(nb - 1) * kStepCounterWords));
   std::vector<unsigned long long> h(kStepCounterWords * (size_t)nb);
   PG_HIP(hipMemcpyAsync(h.data(), ctr, sizeof(unsigned long long) * h.size(), hipMemcpyDeviceToHost, c->stream));
   PG_HIP(hipStreamSynchronize(c->stream));
@@ -1383,8 +1421,9 @@ int picgpu_step(picgpu_ctx *c, double dt, int nsteps, unsigned flags) {
   const bool fields = (flags & PICGPU_STEP_FIELDS) != 0;
   if (fields) PG_CHECK(eulerian_fields_begin(c));
   if (!(flags & PICGPU_STEP_STAGED)) {
+    const bool sparse = sparse_steps(c, flags);
     for (int s0 = 0; s0 < nsteps; s0 += kStepBatch)
-      PG_CHECK(step_batch(c, dt, flags, s0, std::min(kStepBatch, nsteps - s0), nsteps));
+      PG_CHECK(step_batch(c, dt, flags, s0, std::min(kStepBatch, nsteps - s0), nsteps, sparse));
   }
   for (int s = 0; s < nsteps && (flags & PICGPU_STEP_STAGED); ++s) {
     if (fields) PG_CHECK(eulerian_fields_async(c));
