@@ -249,21 +249,66 @@ __device__ __forceinline__ void mirror_store(R *mirror, int IM, int JM, int KM, 
 }
 
 struct FaceBC {
-  int face, handler;
+  int handler;
   double vel[3];
   double vmax;
 };
+struct FaceBCs {
+  FaceBC f[6];
+  unsigned writes;  // bit f: face f's handler writes its ghost nodes
+};
 
-// One boundary handler on one face: one thread per node of the face plane
-// p (0 or m-1 along the face axis); q is the plane inside next to it and u
-// the plane of the face's contravariant flux (0 or m-2).  Within a face no
-// thread reads what another writes.
-template <typename R>
-__global__ __launch_bounds__(kEBlock) void k_bc_face(NodeDims d, FaceBC bc, const double *__restrict__ csi,
-                                                     const double *__restrict__ eta, const double *__restrict__ zet,
-                                                     double *__restrict__ ucat, double *__restrict__ ucont,
-                                                     R *__restrict__ mirror, int IM, int JM, int KM) {
-  const int axis = bc.face >> 1, pos = bc.face & 1;
+// The value that a writing handler of face (axis, pos) gives node (i, j, k)
+// of its plane; in: the value of the node inside next to it.
+__device__ __forceinline__ V3 bc_value(const NodeDims &d, const FaceBC &bc, const double *__restrict__ zet, int i,
+                                       int j, int k, V3 in) {
+  switch (bc.handler) {
+    case PICGPU_BC_WALL_NOSLIP:  // BC_Handlers.c:58-165
+      return {-in.x, -in.y, -in.z};
+    case PICGPU_BC_INLET_CONSTANT_VELOCITY:  // BC_Handlers.c:345-372
+      return {bc.vel[0], bc.vel[1], bc.vel[2]};
+    case PICGPU_BC_INLET_PARABOLIC: {  // BC_Handlers.c:720-780, k faces only
+      const double iw = (double)(d.mx - 2), jw = (double)(d.my - 2);
+      const double ic = 1.0 + iw / 2.0, jc = 1.0 + jw / 2.0;
+      const double in_ = ((double)i - ic) / (iw / 2.0), jn = ((double)j - jc) / (jw / 2.0);
+      const double pi_ = 1.0 - in_ * in_, pj = 1.0 - jn * jn;
+      double mag = bc.vmax * pi_ * pj;
+      if (mag < 0.0) mag = 0.0;
+      const V3 ar = ld3(zet, d.at(i, j, k));
+      const double area = sqrt(ar.x * ar.x + ar.y * ar.y + ar.z * ar.z);
+      V3 dir = {0.0, 0.0, 0.0};
+      if (area > 1e-9) dir = {ar.x / area, ar.y / area, ar.z / area};
+      return {mag * dir.x, mag * dir.y, mag * dir.z};
+    }
+    default:  // PICGPU_BC_NOGRAD_COPY_GHOST, BC_Handlers.c:500-590
+      return in;
+  }
+}
+
+// Boundary handlers: one thread per node of a face plane p (0 or m-1 along
+// the face axis); q is the plane inside next to it and u the plane of the
+// face's contravariant flux (0 or m-2).
+//
+// ALL: the six faces in one launch (blockIdx.y the face), as the sweep over
+// faces 0..5 leaves them.  Within a face no thread reads what another writes,
+// and with at least four planes an axis the two faces of an axis do not meet.
+// A node on planes of several axes is written by each in turn, and its
+// neighbour inside may lie on an earlier axis's plane: the thread of its last
+// writing axis takes the handlers of its axes one after another, from the node
+// that lies inside along all of them, which no face writes.  The fluxes of
+// different axes are different components of Ucont.  128x128x192 cells: 29 us
+// in six launches, 9 in one.
+// Otherwise: face `face` alone, after the faces before it.
+template <typename R, bool ALL>
+__global__ __launch_bounds__(kEBlock) void k_bc_faces(NodeDims d, FaceBCs bcs, int face,
+                                                      const double *__restrict__ csi, const double *__restrict__ eta,
+                                                      const double *__restrict__ zet, double *__restrict__ ucat,
+                                                      double *__restrict__ ucont, R *__restrict__ mirror, int IM,
+                                                      int JM, int KM) {
+  if (ALL) face = (int)blockIdx.y;
+  const int axis = face >> 1, pos = face & 1;
+  const FaceBC &bc = bcs.f[face];
+  if (!((bcs.writes >> face) & 1u)) return;
   const int na = axis == 0 ? d.my : d.mx;
   const int nb = axis == 2 ? d.my : d.mz;
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -271,64 +316,54 @@ __global__ __launch_bounds__(kEBlock) void k_bc_face(NodeDims d, FaceBC bc, cons
   const int a = (int)(t % na), b = (int)(t / na);
   const int m = axis == 0 ? d.mx : axis == 1 ? d.my : d.mz;
   const int p = pos ? m - 1 : 0, q = pos ? p - 1 : p + 1, u = pos ? p - 1 : p;
-  int i, j, k;
-  if (axis == 0) {
-    i = p;
-    j = a;
-    k = b;
-  } else if (axis == 1) {
-    i = a;
-    j = p;
-    k = b;
-  } else {
-    i = a;
-    j = b;
-    k = p;
-  }
-  const int64_t np = d.at(i, j, k);
+  int c[3];  // i, j, k
+  c[0] = axis == 0 ? p : a;
+  c[1] = axis == 0 ? a : axis == 1 ? p : b;
+  c[2] = axis == 2 ? p : b;
+  const int64_t np = d.at(c[0], c[1], c[2]);
   const int64_t stride = axis == 0 ? 1 : axis == 1 ? (int64_t)d.mx : (int64_t)d.mx * d.my;
   const int64_t nq = np + (q - p) * stride, nu = np + (u - p) * stride;
   const double *metric = axis == 0 ? csi : axis == 1 ? eta : zet;
-  V3 out;
+  // the face's flux
   switch (bc.handler) {
-    case PICGPU_BC_WALL_NOSLIP: {  // BC_Handlers.c:58-165
+    case PICGPU_BC_WALL_NOSLIP:
       ucont[3 * nu + axis] = 0.0;
-      const V3 in = ld3(ucat, nq);
-      out = {-in.x, -in.y, -in.z};
       break;
-    }
-    case PICGPU_BC_NOGRAD_COPY_GHOST:  // BC_Handlers.c:500-590
-      out = ld3(ucat, nq);
+    case PICGPU_BC_NOGRAD_COPY_GHOST:
       if (!pos || m >= 3) ucont[3 * np + axis] = ucont[3 * nq + axis];
       break;
-    case PICGPU_BC_INLET_CONSTANT_VELOCITY: {  // BC_Handlers.c:345-372
-      out = {bc.vel[0], bc.vel[1], bc.vel[2]};
+    default: {
+      const V3 v = bc_value(d, bc, zet, c[0], c[1], c[2], V3{0.0, 0.0, 0.0});
       const V3 mm = ld3(metric, nu);
-      ucont[3 * nu + axis] = bc.vel[0] * mm.x + bc.vel[1] * mm.y + bc.vel[2] * mm.z;
-      break;
+      ucont[3 * nu + axis] = v.x * mm.x + v.y * mm.y + v.z * mm.z;
     }
-    case PICGPU_BC_INLET_PARABOLIC: {  // BC_Handlers.c:720-780, k faces only
-      if (axis != 2) return;
-      const double iw = (double)(d.mx - 2), jw = (double)(d.my - 2);
-      const double ic = 1.0 + iw / 2.0, jc = 1.0 + jw / 2.0;
-      const double in = ((double)i - ic) / (iw / 2.0), jn = ((double)j - jc) / (jw / 2.0);
-      const double pi_ = 1.0 - in * in, pj = 1.0 - jn * jn;
-      double mag = bc.vmax * pi_ * pj;
-      if (mag < 0.0) mag = 0.0;
-      const V3 ar = ld3(zet, np);
-      const double area = sqrt(ar.x * ar.x + ar.y * ar.y + ar.z * ar.z);
-      V3 dir = {0.0, 0.0, 0.0};
-      if (area > 1e-9) dir = {ar.x / area, ar.y / area, ar.z / area};
-      out = {mag * dir.x, mag * dir.y, mag * dir.z};
-      const V3 zu = ld3(zet, nu);
-      ucont[3 * nu + 2] = out.x * zu.x + out.y * zu.y + out.z * zu.z;
-      break;
+  }
+  V3 out;
+  if constexpr (ALL) {
+    // the writing faces that the node lies on, by axis (-1: none)
+    const int last[3] = {d.mx - 1, d.my - 1, d.mz - 1};
+    int on[3];
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+      const int f = c[x] == 0 ? 2 * x : c[x] == last[x] ? 2 * x + 1 : -1;
+      on[x] = f >= 0 && ((bcs.writes >> f) & 1u) ? f : -1;
     }
-    default:
-      return;
+    if ((axis < 1 && on[1] >= 0) || (axis < 2 && on[2] >= 0)) return;  // a later face's node
+    int in[3];
+#pragma unroll
+    for (int x = 0; x < 3; ++x) in[x] = on[x] < 0 ? c[x] : (on[x] & 1) ? c[x] - 1 : c[x] + 1;
+    out = ld3(ucat, d.at(in[0], in[1], in[2]));
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+      if (on[x] < 0) continue;
+      in[x] = c[x];
+      out = bc_value(d, bcs.f[on[x]], zet, in[0], in[1], in[2], out);
+    }
+  } else {
+    out = bc_value(d, bc, zet, c[0], c[1], c[2], ld3(ucat, nq));
   }
   st3(ucat, np, out);
-  mirror_store(mirror, IM, JM, KM, i, j, k, out);
+  mirror_store(mirror, IM, JM, KM, c[0], c[1], c[2], out);
 }
 
 // The eight nodes of the box (i-1..i, j-1..j, k-1..k): a[dk][dj][di], index 1
@@ -500,41 +535,47 @@ void node_ijk(const picgpu_ctx *c, unsigned long long n, int *i, int *j, int *k)
   *k = (int)(r / (unsigned long long)d.my);
 }
 
-// Launches k_bc_face for every face, faces 0..5 (Boundaries.c:611-617), or
-// only the inlet handlers (their Initialize, BC_Handlers.c:238-256, 647-664).
+bool handler_built(int handler) {  // BoundaryCondition_Create, Boundaries.c:417-433
+  return handler == PICGPU_BC_NOGRAD_COPY_GHOST || handler == PICGPU_BC_WALL_NOSLIP ||
+         handler == PICGPU_BC_INLET_CONSTANT_VELOCITY || handler == PICGPU_BC_INLET_PARABOLIC;
+}
+
+// The handlers of every face, in the order of faces 0..5 (Boundaries.c:611-617),
+// or only the inlet handlers (their Initialize, BC_Handlers.c:238-256, 647-664).
 int run_boundaries(picgpu_ctx *c, bool inlets_only) {
   const NodeDims d = node_dims(c);
+  FaceBCs bcs;
+  bcs.writes = 0;
   for (int f = 0; f < 6; ++f) {
     const int h = c->eul.bc.handler[f];
     const bool inlet = h == PICGPU_BC_INLET_CONSTANT_VELOCITY || h == PICGPU_BC_INLET_PARABOLIC;
-    if (inlets_only && !inlet) continue;
-    FaceBC fb;
-    fb.face = f;
+    const bool writes = h == PICGPU_BC_INLET_PARABOLIC ? f / 2 == 2 : handler_built(h);
+    if (writes && (inlet || !inlets_only)) bcs.writes |= 1u << f;
+    FaceBC &fb = bcs.f[f];
     fb.handler = h;
     fb.vel[0] = c->eul.bc.velocity[f][0];
     fb.vel[1] = c->eul.bc.velocity[f][1];
     fb.vel[2] = c->eul.bc.velocity[f][2];
     fb.vmax = c->eul.bc.vmax[f];
-    const int axis = f / 2;
-    const int64_t nface = (int64_t)(axis == 0 ? d.my : d.mx) * (axis == 2 ? d.my : d.mz);
-    int r = c->opt.precision == PICGPU_FP32
-                ? [&]() -> int {
-                    PG_LAUNCH(c, "bc_face", eblocks(nface), kEBlock, k_bc_face<float>, d, fb,
-                              c->eul.csi.as<double>(), c->eul.eta.as<double>(), c->eul.zet.as<double>(),
-                              c->eul.ucat.as<double>(), c->eul.ucont.as<double>(), c->ucat.as<float>(), c->IM,
-                              c->JM, c->KM);
-                    return PICGPU_OK;
-                  }()
-                : [&]() -> int {
-                    PG_LAUNCH(c, "bc_face", eblocks(nface), kEBlock, k_bc_face<double>, d, fb,
-                              c->eul.csi.as<double>(), c->eul.eta.as<double>(), c->eul.zet.as<double>(),
-                              c->eul.ucat.as<double>(), c->eul.ucont.as<double>(), c->ucat.as<double>(), c->IM,
-                              c->JM, c->KM);
-                    return PICGPU_OK;
-                  }();
-    PG_CHECK(r);
   }
-  return PICGPU_OK;
+  if (!bcs.writes) return PICGPU_OK;
+  auto launch = [&](auto *tag, auto all, int face, int64_t nface) -> int {
+    using R = std::remove_pointer_t<decltype(tag)>;
+    const dim3 grid((unsigned)eblocks(nface), decltype(all)::value ? 6 : 1);
+    PG_LAUNCH(c, "bc_face", grid, kEBlock, (k_bc_faces<R, decltype(all)::value>), d, bcs, face,
+              c->eul.csi.as<double>(), c->eul.eta.as<double>(), c->eul.zet.as<double>(), c->eul.ucat.as<double>(),
+              c->eul.ucont.as<double>(), c->ucat.as<R>(), c->IM, c->JM, c->KM);
+    return PICGPU_OK;
+  };
+  auto run = [&](auto *tag) -> int {
+    const int64_t plane[3] = {(int64_t)d.my * d.mz, (int64_t)d.mx * d.mz, (int64_t)d.mx * d.my};
+    if (d.mx >= 4 && d.my >= 4 && d.mz >= 4)
+      return launch(tag, std::true_type{}, 0, std::max(plane[0], std::max(plane[1], plane[2])));
+    for (int f = 0; f < 6; ++f)
+      if ((bcs.writes >> f) & 1u) PG_CHECK(launch(tag, std::false_type{}, f, plane[f / 2]));
+    return PICGPU_OK;
+  };
+  return c->opt.precision == PICGPU_FP32 ? run((float *)nullptr) : run((double *)nullptr);
 }
 
 int launch_contra2cart(picgpu_ctx *c) {
@@ -607,11 +648,6 @@ bool handler_valid_for_type(int type, int handler) {
       return handler == PICGPU_BC_INLET_CONSTANT_VELOCITY || handler == PICGPU_BC_INLET_PARABOLIC;
     default: return true;
   }
-}
-
-bool handler_built(int handler) {  // BoundaryCondition_Create, Boundaries.c:417-433
-  return handler == PICGPU_BC_NOGRAD_COPY_GHOST || handler == PICGPU_BC_WALL_NOSLIP ||
-         handler == PICGPU_BC_INLET_CONSTANT_VELOCITY || handler == PICGPU_BC_INLET_PARABOLIC;
 }
 
 int lookup(const char *s, const char *const *names, const int *values, int n, int *out) {
