@@ -156,8 +156,8 @@ constexpr int kLocateLong = 48;
 inline int locate_ahead(int64_t n) { return n <= kLocateWaves * 4 ? 16 : n <= kLocateWaves * 32 ? 4 : 1; }
 // From this many on, the records' lines through LDS (wave_records): 2,000,000 in
 // 128x128x192, 3.48 -> 3.12 ms in FP64, 4.20 -> 3.45 in FP32; 300,000 there 738
-// -> 728 us; 300,000 short walks in a 48x48x250 tube 205 -> 276.
-constexpr int64_t kLocateLines = 1 << 19;
+// -> 728 us and 843 -> 771, in 63x47x129 453 -> 419; 100,000 there 271 -> 328.
+constexpr int64_t kLocateLines = 1 << 18;
 
 // The FP32 record of cell l for each lane of a wavefront (l < 0: none), all
 // lanes taking part; stage: 64 records of LDS, the wavefront's own.

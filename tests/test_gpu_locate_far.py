@@ -16,7 +16,7 @@ IM, JM, KM = 5, 7, 53
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
 @pytest.mark.parametrize("n,cap", [(1, 1000), (3, 1000), (5, 1), (200, 2), (200, 17), (1021, 33), (16_384, 1000),
                                    (16_385, 1000), (16_390, 20), (131_072, 1000), (131_073, 1000),
-                                   ((1 << 19) + 3, 1000)])
+                                   ((1 << 18) + 3, 1000)])
 @pytest.mark.parametrize("grid", ["box", "cube"])
 def test_walks_from_the_first_cell(oracle, precision, n, cap, grid):
     from fdf_amd.swarm import PicGpu
