@@ -1502,10 +1502,14 @@ __global__ __launch_bounds__(kBlock) void k_iota(int64_t n, const int32_t *__res
 
 // Puts every bucket idx[kstart[key] .. kstart[key+1]) in ascending PID order,
 // the summation order of deposition (and of the oracle).  Buckets of up to 8
-// particles are ranked in registers; longer ones, rare at a few particles per
-// cell, are insertion-sorted in place.  The PIDs are read as T: the 32-bit
-// copy pid32 when every PID lies in [0, 2^31) (*wide == 0; the same order,
-// half the bytes), the 64-bit pid otherwise.
+// particles are ranked in a thread's registers.  Longer ones are ranked by
+// several lanes, a particle a lane: sorted by insertion in one thread, their
+// time grew with the square of their particles, one memory access after
+// another (a cell of 20,000 took minutes).  400,000 particles in a graded pipe
+// of 48x48x250 cells, FP64: 15.5 -> 10.4 us; 100,000 in
+// 24x24x24, a whole step in FP32 92 -> 72.  The PIDs are read as
+// T: the 32-bit copy pid32 when every PID lies in [0, 2^31) (*wide == 0; the
+// same order, half the bytes), the 64-bit pid otherwise.
 //
 // With CELLS the thread also averages P over its bucket, in that order, into
 // its cell's pavg (interpolation.c:1838-2036): the bucket's entries are in
@@ -1513,79 +1517,174 @@ __global__ __launch_bounds__(kBlock) void k_iota(int64_t n, const int32_t *__res
 // FP64: 10 + 7.5 us in two launches, 15 in one at 400,000 particles in
 // 48x48x250 cells; 9.0 + 6.1, 13.3 at 500,000 in 64x64x96.
 template <typename T, typename R, bool CELLS>
-__device__ __forceinline__ void bucket_pid_order(int32_t s, int32_t e, int32_t *__restrict__ idx,
+__device__ __forceinline__ void bucket_pid_order(int32_t s, int32_t L, int32_t *__restrict__ idx,
                                                  const T *__restrict__ pid, const R *__restrict__ P, Acc<R> &acc) {
-  const int32_t L = e - s;
-  if (L <= 8) {
-    int32_t q[8], rank[8];
-    T v[8];
-    R val[8];
+  int32_t q[8], rank[8];
+  T v[8];
+  R val[8];
 #pragma unroll
-    for (int t = 0; t < 8; ++t) q[t] = t < L ? idx[s + t] : 0;
+  for (int t = 0; t < 8; ++t) q[t] = t < L ? idx[s + t] : 0;
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+    v[t] = t < L ? pid[q[t]] : (sizeof(T) == 4 ? (T)INT32_MAX : (T)INT64_MAX);
+    if constexpr (CELLS) val[t] = t < L ? P[q[t]] : (R)0;
+  }
+#pragma unroll
+  for (int a = 0; a < 8; ++a) {
+    int r = 0;
+#pragma unroll
+    for (int b = 0; b < 8; ++b) r += (v[b] < v[a] || (v[b] == v[a] && b < a)) ? 1 : 0;
+    rank[a] = r;
+    if (a < L && r != a) idx[s + r] = q[a];  // entries already in place are not rewritten
+  }
+  if constexpr (CELLS) {
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
-      v[t] = t < L ? pid[q[t]] : (sizeof(T) == 4 ? (T)INT32_MAX : (T)INT64_MAX);
-      if constexpr (CELLS) val[t] = t < L ? P[q[t]] : (R)0;
+      if (t >= L) break;
+      R x = val[0];
+#pragma unroll
+      for (int a = 1; a < 8; ++a) x = rank[a] == t ? val[a] : x;
+      acc.add(x);
     }
-#pragma unroll
-    for (int a = 0; a < 8; ++a) {
-      int r = 0;
-#pragma unroll
-      for (int b = 0; b < 8; ++b) r += (v[b] < v[a] || (v[b] == v[a] && b < a)) ? 1 : 0;
-      rank[a] = r;
-      if (a < L && r != a) idx[s + r] = q[a];  // entries already in place are not rewritten
-    }
-    if constexpr (CELLS) {
-#pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        if (t >= L) break;
-        R x = val[0];
-#pragma unroll
-        for (int a = 1; a < 8; ++a) x = rank[a] == t ? val[a] : x;
-        acc.add(x);
+  }
+}
+
+// lane t's value in every lane (t the same in all)
+template <typename V>
+__device__ __forceinline__ V lane_value(V v, int t) {
+  if constexpr (sizeof(V) == 4) {
+    return __builtin_bit_cast(V, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), t));
+  } else {
+    const int2 w = __builtin_bit_cast(int2, v);
+    return __builtin_bit_cast(V, make_int2(__builtin_amdgcn_readlane(w.x, t), __builtin_amdgcn_readlane(w.y, t)));
+  }
+}
+
+// The bucket [s, s + L) by the whole wavefront; tmp [s, s + L) is free.  Each
+// particle's rank is the number of smaller PIDs (of equal ones, those before
+// it); CELLS: acc takes the values of P in that order, the same in every lane.
+template <typename T, typename R, bool CELLS>
+__device__ __forceinline__ void bucket_by_wave(int32_t s, int32_t L, int lane, int32_t *__restrict__ idx,
+                                               int32_t *__restrict__ tmp, const T *__restrict__ pid,
+                                               const R *__restrict__ P, Acc<R> &acc) {
+  for (int32_t t0 = 0; t0 < L; t0 += 64) {
+    const int32_t t = t0 + lane;
+    const int32_t q = t < L ? idx[s + t] : 0;
+    const T v = t < L ? pid[q] : (T)0;
+    int32_t rank = 0;
+    for (int32_t u0 = 0; u0 < L; u0 += 64) {
+      const int32_t u = u0 + lane;
+      const T w = u0 == t0 ? v : u < L ? pid[idx[s + u]] : (T)0;
+      const int32_t m = L - u0 < 64 ? L - u0 : 64;
+      for (int32_t x = 0; x < m; ++x) {
+        const T o = lane_value(w, x);
+        rank += (o < v || (o == v && u0 + x < t)) ? 1 : 0;
       }
     }
-    return;
+    if (t < L) tmp[s + rank] = q;
   }
-  for (int32_t t = s + 1; t < e; ++t) {
-    const int32_t x = idx[t];
-    const T px = pid[x];
-    int32_t u = t - 1;
-    while (u >= s && pid[idx[u]] > px) {
-      idx[u + 1] = idx[u];
-      --u;
+  __threadfence_block();  // the wavefront reads what its other lanes wrote
+  for (int32_t t0 = 0; t0 < L; t0 += 64) {
+    const int32_t t = t0 + lane;
+    const int32_t q = t < L ? tmp[s + t] : 0;
+    if (t < L) idx[s + t] = q;
+    if constexpr (CELLS) {
+      const R x = t < L ? P[q] : (R)0;
+      const int32_t m = L - t0 < 64 ? L - t0 : 64;
+      for (int32_t u = 0; u < m; ++u) acc.add(lane_value(x, u));
     }
-    idx[u + 1] = x;
   }
-  if constexpr (CELLS)
-    for (int32_t t = s; t < e; ++t) acc.add(P[idx[t]]);
 }
+
+// Buckets of 9 to 16 particles, four at a time: 16 lanes take the one of a lane
+// of `lanes`, the same in every lane; acc as above, in that lane.
+template <typename T, typename R, bool CELLS>
+__device__ __forceinline__ void buckets_by_16(unsigned long long lanes, int32_t s, int32_t L, int lane,
+                                              int32_t *__restrict__ idx, const T *__restrict__ pid,
+                                              const R *__restrict__ P, Acc<R> &acc) {
+  const int first = lane & 48, t = lane & 15;
+  while (lanes != 0ull) {
+    unsigned long long m = lanes;
+    for (int g = 0; g < (first >> 4); ++g) m &= m - 1;
+    const int h = m != 0ull ? __ffsll(m) - 1 : 0;
+    const int32_t hs = __shfl(s, h), of = __shfl(L, h), hl = m != 0ull ? of : 0;  // (every lane takes part)
+    const bool on = t < hl;
+    const int32_t q = on ? idx[hs + t] : 0;
+    const T v = on ? pid[q] : (sizeof(T) == 4 ? (T)INT32_MAX : (T)INT64_MAX);
+    int rank = 0;
+#pragma unroll
+    for (int x = 0; x < 16; ++x) {
+      const T o = __shfl(v, first + x);
+      rank += (o < v || (o == v && x < t)) ? 1 : 0;
+    }
+    if (on && rank != t) idx[hs + rank] = q;
+    if constexpr (CELLS) {
+      const R x = on ? P[q] : (R)0;
+      // the lane that holds the value of rank t
+      const int from = __builtin_amdgcn_ds_permute((first + rank) * 4, lane);
+      const R y = __shfl(x, from);
+      Acc<R> sum;
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        const R z = __shfl(y, first + u);
+        if (u < hl) sum.add(z);
+      }
+      const int mine = __popcll(lanes & ((1ull << lane) - 1ull));  // the group of this lane's bucket
+      const R as = __shfl(sum.s, (mine & 3) * 16), ac = __shfl(sum.c, (mine & 3) * 16);
+      if (((lanes >> lane) & 1ull) && mine < 4) {
+        acc.s = as;
+        acc.c = ac;
+      }
+    }
+    for (int g = 0; g < 4; ++g) lanes &= lanes - 1;
+  }
+}
+
+// tmp: as long as idx, free (the index of the step before)
 template <typename R, bool CELLS>
 __global__ __launch_bounds__(kBlock) void k_bucket_pid_order(int64_t nkeys, const int32_t *__restrict__ kstart,
-                                                             int32_t *__restrict__ idx,
+                                                             int32_t *__restrict__ idx, int32_t *__restrict__ tmp,
                                                              const int64_t *__restrict__ pid,
                                                              const int32_t *__restrict__ pid32,
                                                              const int32_t *__restrict__ wide, int IM, int JM, int KM,
                                                              TileMap tm, const R *__restrict__ P,
                                                              R *__restrict__ avg) {
   const int64_t key = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (key >= nkeys) return;
-  const int32_t s = kstart[key], e = kstart[key + 1];
+  const int lane = threadIdx.x & 63;
+  const bool live = key < nkeys;
+  const int32_t s = live ? kstart[key] : 0, L = live ? kstart[key + 1] - s : 0;
   Acc<R> acc;
-  if (e - s == 1) {
+  if (L == 1) {
     if constexpr (CELLS) acc.add(P[idx[s]]);
-  } else if (e - s > 1) {
+  } else if (L > 1 && L <= 8) {
     if (*wide == 0)
-      bucket_pid_order<int32_t, R, CELLS>(s, e, idx, pid32, P, acc);
+      bucket_pid_order<int32_t, R, CELLS>(s, L, idx, pid32, P, acc);
     else
-      bucket_pid_order<int64_t, R, CELLS>(s, e, idx, pid, P, acc);
+      bucket_pid_order<int64_t, R, CELLS>(s, L, idx, pid, P, acc);
+  }
+  const unsigned long long some = __ballot(L > 8 && L <= 16);
+  if (some != 0ull) {
+    if (*wide == 0)
+      buckets_by_16<int32_t, R, CELLS>(some, s, L, lane, idx, pid32, P, acc);
+    else
+      buckets_by_16<int64_t, R, CELLS>(some, s, L, lane, idx, pid, P, acc);
+  }
+  for (unsigned long long rest = __ballot(L > 16); rest != 0ull; rest &= rest - 1) {
+    const int h = __ffsll(rest) - 1;
+    const int32_t hs = __builtin_amdgcn_readlane(s, h), hl = __builtin_amdgcn_readlane(L, h);
+    Acc<R> sum;
+    if (*wide == 0)
+      bucket_by_wave<int32_t, R, CELLS>(hs, hl, lane, idx, tmp, pid32, P, sum);
+    else
+      bucket_by_wave<int64_t, R, CELLS>(hs, hl, lane, idx, tmp, pid, P, sum);
+    if (lane == h) acc = sum;
   }
   if constexpr (CELLS) {
     const int t = (int)(key / TS), l = (int)(key % TS);
     const int i = t % tm.NTI * TX + l % TX, j = t / tm.NTI % tm.NTJ * TY + l / TX % TY,
               k = t / (tm.NTI * tm.NTJ) * TZ + l / (TX * TY);
-    if (i < IM && j < JM && k < KM) {
-      const R cnt = (R)(e - s);
+    if (live && i < IM && j < JM && k < KM) {
+      const R cnt = (R)L;
       avg[(int64_t)i + (int64_t)IM * (j + (int64_t)JM * k)] = cnt > (R)0.5 ? acc.value() / cnt : (R)0;
     }
   }

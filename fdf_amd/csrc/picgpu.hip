@@ -1167,8 +1167,8 @@ static int do_step_fused(picgpu_ctx *c, double dt, unsigned flags, int step, boo
       using R = std::remove_pointer_t<decltype(tag)>;
       auto launch = [&](auto cells_tag) -> int {
         PG_LAUNCH(c, "bucket_pid_order", nblocks(nkeys), kBlock, (k_bucket_pid_order<R, decltype(cells_tag)::value>),
-                  nkeys, nstart, c->kidx[nxt].as<int32_t>(), c->sw.pid.as<int64_t>(), c->sw.pid32.as<int32_t>(),
-                  c->pid_wide.as<int32_t>(), c->IM, c->JM, c->KM, tm, c->sw.P.as<R>(), c->pavg.as<R>());
+                  nkeys, nstart, c->kidx[nxt].as<int32_t>(), c->kidx[cur].as<int32_t>(), c->sw.pid.as<int64_t>(),
+                  c->sw.pid32.as<int32_t>(), c->pid_wide.as<int32_t>(), c->IM, c->JM, c->KM, tm, c->sw.P.as<R>(), c->pavg.as<R>());
         return PICGPU_OK;
       };
       if (!cells) return launch(std::false_type{});
