@@ -1431,21 +1431,29 @@ __global__ __launch_bounds__(kBlock) void k_key_histogram(int64_t n, const int32
   slot[p] = b >= 0 ? atomicAdd(&count[b], 1) : -1;
 }
 
-// idx[kstart[bucket] + slot] = p
+// idx[kstart[bucket] + slot] = p; REC: the particle's number and short fields
+// there instead, for a swarm in arbitrary order that is moved into key order
+// next (SortRec)
+template <typename R, bool REC>
 __global__ __launch_bounds__(kBlock) void k_key_scatter(int64_t n, const int32_t *__restrict__ cell,
                                                         const int32_t *__restrict__ status,
                                                         const int32_t *__restrict__ guess,
                                                         const int32_t *__restrict__ slot, int IM, int JM, TileMap tm,
                                                         int32_t nkeys, const int32_t *__restrict__ kstart,
-                                                        int32_t *__restrict__ idx) {
+                                                        int32_t *__restrict__ idx, const int64_t *__restrict__ pid,
+                                                        const R *__restrict__ P, SortRec<R> *__restrict__ rec) {
   int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n) return;
   const int32_t s = slot[p];
   if (s < 0) return;
   int32_t c = cell[p];
   if (c < 0 && guess) c = guess[p];
-  const int32_t b = bucket_of(c, status[p], IM, JM, tm, nkeys);
-  idx[kstart[b] + s] = (int32_t)p;
+  const int32_t st = status[p];
+  const int32_t b = bucket_of(c, st, IM, JM, tm, nkeys);
+  if constexpr (REC)
+    rec[kstart[b] + s] = SortRec<R>{(int32_t)p, c, pid[p], P[p], st};
+  else
+    idx[kstart[b] + s] = (int32_t)p;
 }
 
 // count: n, or *n_dev when n_dev is given (a count still on the device)
@@ -1976,7 +1984,8 @@ enum GatherMode : int { GATHER_ALL = 0, GATHER_STEP = 1, GATHER_LAST = 2 };
 constexpr int kGatherPer = 4;
 // (a template parameter: a run-time flag there made the FP32 gather 40 %
 // slower, its loads no longer issued ahead of the stores).
-template <typename R, bool MOVE_VW>
+// REC: in the order of rec, which holds the short fields (k_key_scatter).
+template <typename R, bool MOVE_VW, bool REC>
 __global__ __launch_bounds__(kBlock) void k_gather_swarm(int64_t m_max, const int32_t *__restrict__ m_dev, int mode,
                                                          const int32_t *__restrict__ idx,
                                                          const double *__restrict__ pos, const R *__restrict__ vel,
@@ -1987,13 +1996,20 @@ __global__ __launch_bounds__(kBlock) void k_gather_swarm(int64_t m_max, const in
                                                          R *__restrict__ w2, int32_t *__restrict__ cell2,
                                                          int32_t *__restrict__ status2, int64_t *__restrict__ pid2,
                                                          R *__restrict__ P2, const int32_t *__restrict__ pid32,
-                                                         int32_t *__restrict__ pid32_2) {
+                                                         int32_t *__restrict__ pid32_2,
+                                                         const SortRec<R> *__restrict__ rec) {
   constexpr int NP = kGatherPer;
   const int64_t m = dev_count(m_max, m_dev);
   const int64_t q0 = (int64_t)blockIdx.x * (kBlock * NP) + threadIdx.x;
   int64_t p[NP];
 #pragma unroll
-  for (int u = 0; u < NP; ++u) p[u] = q0 + u * kBlock < m ? idx[q0 + u * kBlock] : -1;
+  for (int u = 0; u < NP; ++u) {
+    const int64_t q = q0 + u * kBlock;
+    if constexpr (REC)
+      p[u] = q < m ? rec[q].p : -1;
+    else
+      p[u] = q < m ? idx[q] : -1;
+  }
   double x[NP][3];
   R v[NP][3], ww[NP][3], pp[NP];
   int32_t ce[NP], st[NP];
@@ -2009,10 +2025,18 @@ __global__ __launch_bounds__(kBlock) void k_gather_swarm(int64_t m_max, const in
         ww[u][c] = w[3 * p[u] + c];
       }
     }
-    ce[u] = cell[p[u]];
-    st[u] = mode == GATHER_ALL ? status[p[u]] : ST_LOCATED;
-    id[u] = pid[p[u]];
-    pp[u] = P[p[u]];
+    if constexpr (REC) {
+      const SortRec<R> r = rec[q0 + u * kBlock];
+      ce[u] = r.cell;
+      st[u] = r.status;
+      id[u] = r.pid;
+      pp[u] = r.P;
+    } else {
+      ce[u] = cell[p[u]];
+      st[u] = mode == GATHER_ALL ? status[p[u]] : ST_LOCATED;
+      id[u] = pid[p[u]];
+      pp[u] = P[p[u]];
+    }
   }
 #pragma unroll
   for (int u = 0; u < NP; ++u) {

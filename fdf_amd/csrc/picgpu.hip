@@ -573,7 +573,7 @@ static int ensure_filter(picgpu_ctx *c) {
   return PICGPU_OK;
 }
 
-static int build_key_index(picgpu_ctx *c, const int32_t *guess = nullptr);
+static int build_key_index(picgpu_ctx *c, const int32_t *guess = nullptr, bool rec = false);
 
 // An FP64 locate of at least this many particles from guessed start cells
 // visits them grouped by start cell (tile-major key), so that neighbouring
@@ -759,19 +759,16 @@ static int do_sort(picgpu_ctx *c) {
   }
   PG_CHECK(scan_exclusive_i32(c, c->cell_count.as<int32_t>(), c->cell_start.as<int32_t>(), c->ncell));
   if (n > 0) {
-    // the order under construction: kidx and pos0 hold nothing else here
-    DevBuf &sidx = c->kidx[c->kcur], &spid = c->pos0;
-    c->keyed = false;
-    PG_CHECK(sidx.ensure(sizeof(int32_t) * (size_t)n));
-    PG_CHECK(spid.ensure(sizeof(int64_t) * (size_t)n));
+    DevBuf &rec = c->pos0;  // the order under construction: pos0 holds nothing else here
+    PG_CHECK(rec.ensure(sizeof(SortRec<double>) * (size_t)n));
     const int32_t *start = c->cell_start.as<int32_t>();
-    PG_LAUNCH(c, "slot_scatter", nblocks(n), kBlock, k_slot_scatter, n, c->rank.as<int32_t>(), start,
-              c->sw.cell.as<int32_t>(), c->sw.pid.as<int64_t>(), sidx.as<int32_t>(), spid.as<int64_t>());
     int r = dispatch_real(c, [&](auto *tag) -> int {
       using R = std::remove_pointer_t<decltype(tag)>;
-      PG_LAUNCH(c, "sort_gather", nblocks(n), kBlock, k_sort_gather<R>, start + c->ncell, start, sidx.as<int32_t>(),
-                spid.as<int64_t>(), c->sw.pos.as<double>(), c->sw.vel.as<R>(), c->sw.w.as<R>(),
-                c->sw.cell.as<int32_t>(), c->sw.status.as<int32_t>(), c->sw.P.as<R>(), c->alt.pos.as<double>(),
+      PG_LAUNCH(c, "slot_scatter", nblocks(n), kBlock, k_slot_scatter<R>, n, c->rank.as<int32_t>(), start,
+                c->sw.cell.as<int32_t>(), c->sw.pid.as<int64_t>(), c->sw.P.as<R>(), c->sw.status.as<int32_t>(),
+                rec.as<SortRec<R>>());
+      PG_LAUNCH(c, "sort_gather", nblocks(n), kBlock, k_sort_gather<R>, start + c->ncell, start, rec.as<SortRec<R>>(),
+                c->sw.pos.as<double>(), c->sw.vel.as<R>(), c->sw.w.as<R>(), c->alt.pos.as<double>(),
                 c->alt.vel.as<R>(), c->alt.w.as<R>(), c->alt.cell.as<int32_t>(), c->alt.status.as<int32_t>(),
                 c->alt.pid.as<int64_t>(), c->alt.P.as<R>());
       return PICGPU_OK;
@@ -893,7 +890,8 @@ static constexpr int kCompactEvery = 16;
 // key, the live ones without a cell in the last bucket, removed ones left out.
 // With guess, a particle without a cell is keyed by its guessed start cell
 // instead (the order of a fresh locate; not an index of the swarm).
-static int build_key_index(picgpu_ctx *c, const int32_t *guess) {
+// rec: in pos0, with the particles' short fields, for compact_by_key.
+static int build_key_index(picgpu_ctx *c, const int32_t *guess, bool rec) {
   const TileMap tm = tile_map(c);
   const int64_t nkeys = ntiles(tm) * TS;
   const int64_t n = c->n;
@@ -910,9 +908,17 @@ static int build_key_index(picgpu_ctx *c, const int32_t *guess) {
               c->kslot.as<int32_t>());
   PG_CHECK(scan_exclusive_i32(c, c->kcount.as<int32_t>(), c->kstart[cur].as<int32_t>(), nkeys + 1));
   if (n > 0)
-    PG_LAUNCH(c, "key_scatter", nblocks(n), kBlock, k_key_scatter, n, c->sw.cell.as<int32_t>(),
-              c->sw.status.as<int32_t>(), guess, c->kslot.as<int32_t>(), c->IM, c->JM, tm, (int32_t)nkeys,
-              c->kstart[cur].as<int32_t>(), c->kidx[cur].as<int32_t>());
+    PG_CHECK(dispatch_real(c, [&](auto *tag) -> int {
+      using R = std::remove_pointer_t<decltype(tag)>;
+      auto launch = [&](auto to_rec) -> int {
+        PG_LAUNCH(c, "key_scatter", nblocks(n), kBlock, (k_key_scatter<R, decltype(to_rec)::value>), n,
+                  c->sw.cell.as<int32_t>(), c->sw.status.as<int32_t>(), guess, c->kslot.as<int32_t>(), c->IM, c->JM,
+                  tm, (int32_t)nkeys, c->kstart[cur].as<int32_t>(), c->kidx[cur].as<int32_t>(),
+                  c->sw.pid.as<int64_t>(), c->sw.P.as<R>(), c->pos0.as<SortRec<R>>());
+        return PICGPU_OK;
+      };
+      return rec ? launch(std::true_type{}) : launch(std::false_type{});
+    }));
   int32_t h[2] = {0, 0};
   PG_HIP(hipMemcpyAsync(h, c->kstart[cur].as<int32_t>() + nkeys, sizeof(h), hipMemcpyDeviceToHost, c->stream));
   PG_HIP(hipStreamSynchronize(c->stream));
@@ -927,24 +933,25 @@ static int build_key_index(picgpu_ctx *c, const int32_t *guess) {
 // index becomes the identity.  live_dev: the live count when it is still on
 // the device (live is then an upper bound, and c->n is set by the caller).
 static int compact_by_key(picgpu_ctx *c, int64_t live, int mode, const int32_t *live_dev = nullptr,
-                          bool move_vw = true) {
+                          bool move_vw = true, bool rec = false) {
   PG_CHECK(ensure_swarm(c, c->alt, c->n));
   int32_t *idx = c->kidx[c->kcur].as<int32_t>();
   const bool move32 = c->pid32_valid;  // the 32-bit PID copy moves with the swarm
   if (live > 0) {
     int r = dispatch_real(c, [&](auto *tag) -> int {
       using R = std::remove_pointer_t<decltype(tag)>;
-      auto gather = [&](auto vw_tag) -> int {
+      auto gather = [&](auto vw_tag, auto rec_tag) -> int {
         PG_LAUNCH(c, "gather_swarm", nblocks(live, kBlock * kGatherPer), kBlock,
-                  (k_gather_swarm<R, decltype(vw_tag)::value>), live, live_dev, mode, idx, c->sw.pos.as<double>(),
+                  (k_gather_swarm<R, decltype(vw_tag)::value, decltype(rec_tag)::value>), live, live_dev, mode, idx, c->sw.pos.as<double>(),
                   c->sw.vel.as<R>(), c->sw.w.as<R>(), c->sw.cell.as<int32_t>(), c->sw.status.as<int32_t>(),
                   c->sw.pid.as<int64_t>(), c->sw.P.as<R>(), c->alt.pos.as<double>(), c->alt.vel.as<R>(),
                   c->alt.w.as<R>(), c->alt.cell.as<int32_t>(), c->alt.status.as<int32_t>(), c->alt.pid.as<int64_t>(),
                   c->alt.P.as<R>(), move32 ? c->sw.pid32.as<int32_t>() : (const int32_t *)nullptr,
-                  c->alt.pid32.as<int32_t>());
+                  c->alt.pid32.as<int32_t>(), c->pos0.as<SortRec<R>>());
         return PICGPU_OK;
       };
-      return move_vw ? gather(std::true_type{}) : gather(std::false_type{});
+      if (rec) return gather(std::true_type{}, std::true_type{});
+      return move_vw ? gather(std::true_type{}, std::false_type{}) : gather(std::false_type{}, std::false_type{});
     });
     PG_CHECK(r);
     PG_LAUNCH(c, "iota", nblocks(live), kBlock, k_iota, live, live_dev, idx);
@@ -1074,10 +1081,15 @@ static int do_step_fused(picgpu_ctx *c, double dt, unsigned flags, int step, boo
   PG_CHECK(ensure_planes(c));
   const bool fresh = !c->keyed;  // index built here: statuses still to be read
   if (fresh) {
-    PG_CHECK(build_key_index(c));
     // a swarm in arbitrary order (fresh upload, stage-wise calls) is moved
-    // into key order first, so that the tiles read their particles coalesced
-    if (!c->key_ordered) PG_CHECK(compact_by_key(c, c->kend_unloc, GATHER_ALL));
+    // into key order first, so that the tiles read their particles coalesced:
+    // its short fields in records of 32 bytes, scattered with the order, where
+    // there is memory for them (16.8M particles, FP32: scatter and gather 0.54 +
+    // 2.54 -> KEYREC_A ms)
+    const bool rec = !c->key_ordered &&
+                     c->pos0.ensure(sizeof(SortRec<double>) * (size_t)(c->n > 0 ? c->n : 1)) == PICGPU_OK;
+    PG_CHECK(build_key_index(c, nullptr, rec));
+    if (!c->key_ordered) PG_CHECK(compact_by_key(c, c->kend_unloc, GATHER_ALL, nullptr, true, rec));
   }
   const TileMap tm = tile_map(c);
   const int64_t nt = ntiles(tm), nkeys = nt * TS;
