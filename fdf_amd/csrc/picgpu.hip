@@ -1027,6 +1027,7 @@ static void fill_step_args(picgpu_ctx *c, StepArgs<R> &a, double dt, unsigned lo
   a.status = c->sw.status.as<int32_t>();
   a.corner = c->corner.as<R>();
   a.planes = c->planes.ptr;
+  a.filter = c->have_filter ? c->filter.as<CellPlanes32>() : nullptr;
   a.dt = dt;
   a.max_traversal = c->opt.max_traversal;
   a.thresh_scale = c->opt.distance_threshold;
@@ -1136,12 +1137,13 @@ static int do_step_fused(picgpu_ctx *c, double dt, unsigned flags, int step, boo
       auto launch = [&](auto rk2_tag, auto wu_tag) -> int {
         constexpr bool RK = decltype(rk2_tag)::value, WU = decltype(wu_tag)::value;
         if (sparse) {
-          PG_LAUNCH(c, name, nblocks(n), kBlock, (k_step_list<R, EX, RK>), a, idx, (int64_t)0, (int64_t)0, m_dev);
+          PG_LAUNCH(c, name, nblocks(n), kBlock, (k_step_list<R, EX, RK, true>), a, idx, (int64_t)0, (int64_t)0,
+                    m_dev);
           return PICGPU_OK;
         }
         PG_LAUNCH(c, name, nt, kBlock, (k_step_tiled<R, EX, RK, WU>), a, idx, kstart, kbase);
         if (fresh && u1 > u0)
-          PG_LAUNCH(c, name_list, nblocks(u1 - u0), kBlock, (k_step_list<R, EX, RK>), a, idx, u0, u1,
+          PG_LAUNCH(c, name_list, nblocks(u1 - u0), kBlock, (k_step_list<R, EX, RK, false>), a, idx, u0, u1,
                     (const int32_t *)nullptr);
         const SeamCounts sc = dep ? seam_counts(c) : SeamCounts{0, 0, 0};
         if (dblocks + sc.total() > 0)
