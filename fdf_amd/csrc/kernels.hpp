@@ -251,7 +251,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_locate(LocateArgs<R> a) {
   int32_t lc = 0;  // ci + IM (cj + JM ck); used only inside the grid
   const int32_t sj = a.g.IM, sk = a.g.IM * a.g.JM;
   const CellPlanes32 *const recs = EXACT ? a.filter : static_cast<const CellPlanes32 *>(a.planes);
-  int32_t saved = -1;  // cell of the walk's last power-of-two iteration (CycleGuard's test)
+  int32_t saved = -1;  // the walk's cell at iteration 1, 3, 7, 15 ... (CycleGuard's test)
   int held = 0;        // full evaluations of the walk that took it on
   double x[3] = {0.0, 0.0, 0.0};
   float d[6];
@@ -278,7 +278,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_locate(LocateArgs<R> a) {
       ph = kLost;  // periodic walk: LOST at MAX_TRAVERSAL (:1206-1212)
       steps = a.max_traversal;
     } else {
-      if ((steps & (steps - 1)) == 0) saved = lc;
+      if ((steps & (steps + 1)) == 0) saved = lc;
       ph = kHold;
     }
   };
@@ -510,7 +510,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_locate_ahead(LocateArgs<R> a) {
         if (ph == kWalk) {
           // out of the domain, lc is no cell (the kind tells)
           periodic = lc == saved && !(len == 0 && (at & 3) == OUT);
-          if ((round & (round + 1)) == 0) saved = (len == 0 && (at & 3) == OUT) ? -1 : lc;
+          if (((round + 1) & (round + 2)) == 0) saved = (len == 0 && (at & 3) == OUT) ? -1 : lc;
           ++round;
           if (periodic || len >= a.max_traversal - steps) {
             steps = a.max_traversal;  // LOST there, and a periodic walk at once (:1206-1212)
