@@ -88,7 +88,7 @@ __global__ __launch_bounds__(kBlock) void k_reset_advect(int64_t n, double *__re
 // the latency of one load and its evaluation, and a large launch's is the
 // record lines it touches.  In FP64 the steps of a walk are therefore decided
 // on the 128-byte FP32 record (a.filter): where the filter certifies every
-// face (planes_fp32_distances), the reference's FP64 distances have those
+// face (planes_fp32_certified), the reference's FP64 distances have those
 // signs and lie outside the zero band, so the step is the reference's.  The
 // 304-byte FP64 record (3 or 4 lines) is read where the filter certifies the
 // owner, for the weights, and where it certifies nothing.  Lanes wait for that
@@ -154,10 +154,24 @@ constexpr int kStopped = 16;  // lanes without a walk at which a wavefront turns
 // and before both, 342, 265 and 60 at 10,000.
 constexpr int kLocateLong = 48;
 inline int locate_ahead(int64_t n) { return n <= kLocateWaves * 4 ? 16 : n <= kLocateWaves * 32 ? 4 : 1; }
-// From this many on, the records' lines through LDS (wave_records): 2,000,000 in
-// 128x128x192, 3.48 -> 3.12 ms in FP64, 4.20 -> 3.45 in FP32; 300,000 there 738
-// -> 728 us and 843 -> 771, in 63x47x129 453 -> 419; 100,000 there 271 -> 328.
+// From kLocateLines particles on, the records' lines through LDS (wave_records)
+// in the iterations that at least kLinesLanes lanes of the wavefront evaluate.
+// The staging costs a wavefront the same for one walk as for 64, so that a few
+// long walks among lanes that have ended (the bent pipe from cell (0,0,0): most
+// walks leave the grid after two or three iterations, the others take hundreds)
+// are better off with loads of their own.  The locate, us, own loads / all
+// iterations staged / those of 32 lanes:
+//   n            48x48x250 tube     63x47x129 cube     128x128x192 cube
+//   300,000 FP64  202 /  274 / 206   440 /  419 / 369   740 /  718 / 676
+//   300,000 FP32  274 /  341 / 287   461 /  428 / 379   839 /  756 / 722
+//   2M FP64       665 /  617 / 537  2107 / 1686 / 1574 3473 / 3026 / 2931
+//   2M FP32       640 /  629 / 576  2330 / 1772 / 1695 4180 / 3358 / 3170
+// 16.8M FP32 in a 128x128x1024 tube: 18.95 / 19.24 / 16.74 ms.  16 or 48 lanes in
+// place of 32 measure within 5 %.  Below the line the LDS gains less than it costs
+// where walks are short: 262,144 particles, own loads / 32 lanes, the tube 177 / 192
+// in FP32, the cubes 366 / 319 and 619 / 482; 140,000: 185 / 204, 297 / 308, 452 / 438.
 constexpr int64_t kLocateLines = 1 << 18;
+constexpr int kLinesLanes = 32;
 
 // The FP32 record of cell l for each lane of a wavefront (l < 0: none), all
 // lanes taking part; stage: 64 records of LDS, the wavefront's own.
@@ -328,7 +342,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_locate(LocateArgs<R> a) {
               ph = kOwner;
           }
         };
-        if constexpr (LINES) {
+        if (LINES && __popcll(__ballot(eval)) >= kLinesLanes) {
           const CellPlanes32 rec = wave_records(recs, eval ? lc : -1, my_stage, lane);
           if (eval) decide(rec);
         } else {
