@@ -1,0 +1,34 @@
+"""Checks of tests/test_gpu_alloc.py, each run in a process of its own with
+tests/alloc_shim.c between libpicgpu.so and the HIP runtime's allocations:
+alloc_child.py SHIM CHECK [ARGUMENT...]."""
+import ctypes as C
+import os
+import sys
+
+sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+shim = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)  # before the library
+shim.shim_limit.argtypes = [C.c_int64]
+for _f in ("shim_used", "shim_peak", "shim_host_calls"):
+    getattr(shim, _f).restype = C.c_int64
+shim.shim_host_flags.restype = C.c_uint
+
+import numpy as np  # noqa: E402
+
+from fdf_amd import _lib as L  # noqa: E402
+from fdf_amd import workloads as W  # noqa: E402
+from fdf_amd.swarm import PicGpu  # noqa: E402
+
+
+def coherent():
+    """The slots that kernels and host threads share are coherent by their own flag."""
+    with PicGpu(precision="fp64") as g:
+        g.upload_grid(4, 4, 4, W.uniform_grid(4, 4, 4))
+        g.upload_particles(np.full((100, 3), 0.5))
+        assert (g.download_particles()["pos"] == 0.5).all()
+    assert shim.shim_host_calls() >= 1
+    assert shim.shim_host_flags() & 0x40000000, hex(shim.shim_host_flags())  # hipHostMallocCoherent
+
+
+if __name__ == "__main__":
+    globals()[sys.argv[2]](*sys.argv[3:])
+    print("ok")
