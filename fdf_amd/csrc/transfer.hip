@@ -231,7 +231,7 @@ static int take_ring(void **out) {
   if (hipHostMalloc(out, kSlotBytes * kSlots, hipHostMallocPortable | hipHostMallocCoherent) == hipSuccess)
     return PICGPU_OK;
   (void)hipGetLastError();
-  set_error("hipHostMalloc(%zu) failed", kSlotBytes * kSlots);
+  *out = nullptr;
   return PICGPU_E_NOMEM;
 }
 static void give_ring(void *ring) {
@@ -420,6 +420,39 @@ static int move_host(picgpu_ctx *c, void *ring, const HostSeg *segs, int nsegs, 
   return PICGPU_OK;
 }
 
+// Without pinned memory (a limit of the process or the machine): the kernels
+// convert between the arrays and a slot of device memory, which the runtime
+// copies from and to the caller's pageable arrays, a chunk after another.
+static int move_pageable(picgpu_ctx *c, const HostSeg *segs, int nsegs, bool down) {
+  DevBuf slot;
+  PG_CHECK(slot.ensure(kSlotBytes));
+  hipError_t err = hipSuccess;
+  for (int s = 0; s < nsegs && err == hipSuccess; ++s) {
+    const size_t stride = segs[s].stride;
+    const int64_t w = (int64_t)(stride / 8), most = (int64_t)(kSlotBytes / stride);
+    for (int64_t e = 0; e < segs[s].n && err == hipSuccess; e += most) {
+      const int64_t m = segs[s].n - e < most ? segs[s].n - e : most;
+      const size_t bytes = (size_t)m * stride;
+      char *h = static_cast<char *>(segs[s].host) + (size_t)e * stride;
+      if (down) {
+        err = launch_pack(c, segs[s], e * w, m * w, slot.ptr);
+        if (err == hipSuccess) err = hipMemcpyAsync(h, slot.ptr, bytes, hipMemcpyDeviceToHost, c->stream);
+      } else {
+        err = hipMemcpyAsync(slot.ptr, h, bytes, hipMemcpyHostToDevice, c->stream);
+        if (err == hipSuccess) err = launch_unpack(c, segs[s], e, m, slot.ptr);
+      }
+      const hipError_t done = hipStreamSynchronize(c->stream);
+      if (err == hipSuccess) err = done;
+    }
+  }
+  slot.release();
+  if (err != hipSuccess) {
+    set_error("host transfer failed: %s", hipGetErrorString(err));
+    return PICGPU_E_HIP;
+  }
+  return PICGPU_OK;
+}
+
 static int host_transfer(picgpu_ctx *c, const HostSeg *segs, int nsegs, bool down) {
   size_t total = 0;
   for (int s = 0; s < nsegs; ++s) total += (size_t)segs[s].n * segs[s].stride;
@@ -427,7 +460,7 @@ static int host_transfer(picgpu_ctx *c, const HostSeg *segs, int nsegs, bool dow
   for (hipEvent_t &e : c->transfer.ev)
     if (!e) PG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   void *ring = nullptr;
-  PG_CHECK(take_ring(&ring));
+  if (take_ring(&ring) != PICGPU_OK) return move_pageable(c, segs, nsegs, down);
   const int r = move_host(c, ring, segs, nsegs, total, down);
   give_ring(ring);
   return r;

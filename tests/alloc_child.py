@@ -29,6 +29,39 @@ def coherent():
     assert shim.shim_host_flags() & 0x40000000, hex(shim.shim_host_flags())  # hipHostMallocCoherent
 
 
+def no_pinned(precision, n):
+    """Every kind of array, up and down, when pinned memory is refused: what a
+    context with pinned slots gives, bit for bit."""
+    n, (IM, JM, KM) = int(n), (23, 19, 31)
+    rng = np.random.default_rng(n)
+    coor = W.perturbed_cube(IM, JM, KM, seed=2)
+    a = {"vel": rng.standard_normal((n, 3)), "weight": rng.random((n, 3)),
+         "cell": rng.integers(-1, [IM + 1, JM + 1, KM + 1], (n, 3)), "status": rng.integers(0, 5, n),
+         "pid": rng.permutation(n) - n // 2, "P": rng.random(n)}
+    pos = rng.random((n, 3))
+    ucat = rng.standard_normal(3 * (IM + 1) * (JM + 1) * (KM + 1))
+    out = []
+    for refuse in (0, 1):
+        shim.shim_refuse_host(refuse)
+        with PicGpu(precision=precision) as g:
+            g.upload_grid(IM, JM, KM, coor)
+            g.upload_ucat(ucat)
+            g.upload_particles(pos, **a)
+            d = [g.download_particles()]
+            g.upload_particles(pos, pid=a["pid"])
+            g.LocateAllParticlesInGrid()
+            g.InterpolateAllFieldsToSwarm()
+            g.ScatterAllParticleFieldsToEulerFields()
+            g.DepositParticlesToFaces(1e-9)
+            d.append(g.download_particles())
+            d[1]["fields"] = np.concatenate([g.field(w).reshape(-1) for w in range(9)])
+            out.append(d)
+    assert shim.shim_host_calls() >= 2
+    for x, y in zip(*out):
+        for k in x:
+            assert x[k].tobytes() == y[k].tobytes(), k
+
+
 if __name__ == "__main__":
     globals()[sys.argv[2]](*sys.argv[3:])
     print("ok")

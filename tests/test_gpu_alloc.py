@@ -33,3 +33,9 @@ def _child(shim, *args):
 
 def test_pinned_slots_are_coherent(shim):
     _child(shim, "coherent")
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("n", [1, (1 << 20) // 24, (1 << 20) // 24 + 1, (1 << 20) // 8 + 1])  # around a chunk's end
+def test_transfers_without_pinned_memory(shim, precision, n):
+    _child(shim, "no_pinned", precision, n)
