@@ -29,11 +29,14 @@ namespace picgpu {
 // slot's time (kernels writing 1 MiB: 52 GB/s, 256 KiB 43, 128 KiB 35).  A
 // small transfer fills its slots less, so that the host's copies overlap too,
 // but not below 512 KiB: an event and its wait take about 10 us.
-constexpr int kSlots = TransferEvents::kSlots;
 constexpr size_t kSlotBytes = 1 << 20, kMinFill = 512 << 10;
-// one thread more for every 2 MiB, up to 7: memory copies reach 30 GB/s on one
-// thread, 81 on four, 124 on eight; starting 7 threads takes 0.1 ms
+// One thread more for every 2 MiB, up to 7: memory copies reach 30 GB/s on one
+// thread, 81 on four, 124 on eight; starting 7 threads takes 0.1 ms.
 constexpr size_t kBytesPerThread = 2 << 20;
+// Small transfers: by the calling thread alone, through three slots.  A helper
+// thread gains from 2 MiB down (positions of 2.4 MB: 125 -> 100 us) and costs up
+// to 4 MiB up (2.4 MB of FP32 swarm: 122 -> 136 us, 3.6 MB 155 -> 167).
+constexpr size_t kSmallDown = 2 << 20, kSmallUp = 4 << 20;
 constexpr int kMaxThreads = 7;
 // workgroups of a chunk's kernel: reads over the link lose where many
 // wavefronts issue them (1 MiB: 32 workgroups 50 GB/s, 512 38), writes do not
@@ -195,15 +198,25 @@ static hipError_t launch_unpack(picgpu_ctx *c, const HostSeg &s, int64_t e0, int
 // ---------------------------------------------------------------- the ring
 // The slots.  The host's first touch of pinned memory costs 0.38 ms a MiB (a
 // fault a page), so the rings of transfers that have ended are kept for the
-// next ones, at most kRingsKept of them, until the last context is destroyed.
+// next ones, at most kRingsKept of each size, until the last context is
+// destroyed.  A small transfer has a ring of its own size: the runtime hands
+// back an allocation below 2 MiB that it has seen before, already mapped, where
+// 8 MiB are new each time that a program's only context is made again
+// (20,000 particles, a context's first upload: 0.13 to 1.2 ms with the large
+// ring, by whether they were, 0.12 with the small one; steady state 0.09 both).
 // A transfer holds its ring alone; any device may use it.  The host rewrites a
 // slot while later kernels are queued, and reads one while earlier ones run, so
 // the memory is coherent by its own flag, whatever the environment asks of
 // unflagged allocations (same time a transfer: 200,000 particles down 596 and
 // 598 us, 2,000,000 up 6.11 and 6.11 ms).
+struct RingSize {
+  int slots;
+  size_t slot_bytes;
+};
+constexpr RingSize kSmallRing{3, kMinFill}, kLargeRing{TransferEvents::kSlots, kSlotBytes};
 constexpr int kRingsKept = 2;
 static std::mutex g_rings_mu;
-static void *g_rings[kRingsKept];
+static void *g_rings[2][kRingsKept];  // small, large
 static int g_ring_users;
 
 void rings_open() {
@@ -213,31 +226,33 @@ void rings_open() {
 void rings_close() {
   std::lock_guard<std::mutex> lock(g_rings_mu);
   if (--g_ring_users > 0) return;
-  for (void *&r : g_rings) {
-    if (r) (void)hipHostFree(r);
-    r = nullptr;
-  }
+  for (auto &size : g_rings)
+    for (void *&r : size) {
+      if (r) (void)hipHostFree(r);
+      r = nullptr;
+    }
 }
-static int take_ring(void **out) {
+static int take_ring(bool small, void **out) {
   {
     std::lock_guard<std::mutex> lock(g_rings_mu);
-    for (void *&r : g_rings)
+    for (void *&r : g_rings[small ? 0 : 1])
       if (r) {
         *out = r;
         r = nullptr;
         return PICGPU_OK;
       }
   }
-  if (hipHostMalloc(out, kSlotBytes * kSlots, hipHostMallocPortable | hipHostMallocCoherent) == hipSuccess)
+  const RingSize &s = small ? kSmallRing : kLargeRing;
+  if (hipHostMalloc(out, s.slot_bytes * s.slots, hipHostMallocPortable | hipHostMallocCoherent) == hipSuccess)
     return PICGPU_OK;
   (void)hipGetLastError();
   *out = nullptr;
   return PICGPU_E_NOMEM;
 }
-static void give_ring(void *ring) {
+static void give_ring(bool small, void *ring) {
   {
     std::lock_guard<std::mutex> lock(g_rings_mu);
-    for (void *&r : g_rings)
+    for (void *&r : g_rings[small ? 0 : 1])
       if (!r) {
         r = ring;
         return;
@@ -266,7 +281,7 @@ struct Group {
 };
 
 // One transfer, shared by the calling thread and its helpers.  Group k goes
-// through slot k % kSlots.
+// through slot k % size.slots.
 //  down: any thread may issue the next group's kernels (one thread at a time,
 //        in order, into a slot whose last group was copied out); threads claim
 //        issued groups, wait for the group's event and copy.
@@ -277,6 +292,7 @@ struct Group {
 struct Transfer {
   picgpu_ctx *c;
   char *ring;
+  RingSize size;
   const HostSeg *segs;
   const std::vector<Chunk> &chunks;
   const std::vector<Group> &groups;
@@ -286,8 +302,8 @@ struct Transfer {
   std::atomic_flag issuing = ATOMIC_FLAG_INIT;
   std::atomic<int> err{0};
 
-  char *slot(int64_t k) const { return ring + (size_t)(k % kSlots) * kSlotBytes; }
-  hipEvent_t event(int64_t k) const { return c->transfer.ev[k % kSlots]; }
+  char *slot(int64_t k) const { return ring + (size_t)(k % size.slots) * size.slot_bytes; }
+  hipEvent_t event(int64_t k) const { return c->transfer.ev[k % size.slots]; }
   void copy(int64_t k) const {
     for (size_t q = groups[(size_t)k].first; q < groups[(size_t)k].end; ++q) {
       const Chunk &ch = chunks[q];
@@ -320,7 +336,7 @@ struct Transfer {
     if (issuing.test_and_set(std::memory_order_acquire)) return;
     const int64_t N = (int64_t)groups.size();
     for (int64_t k = issued.load(); k < N && !err.load(); ++k) {
-      if (k >= kSlots && !done[k - kSlots].load(std::memory_order_acquire)) break;
+      if (k >= size.slots && !done[k - size.slots].load(std::memory_order_acquire)) break;
       if (!launch(k)) break;
       issued.store(k + 1, std::memory_order_release);
     }
@@ -346,8 +362,8 @@ struct Transfer {
     while (!err.load()) {
       const int64_t k = claimed.fetch_add(1);
       if (k >= N) return;
-      if (k >= kSlots) {
-        while (!done[k - kSlots].load(std::memory_order_acquire)) {
+      if (k >= size.slots) {
+        while (!done[k - size.slots].load(std::memory_order_acquire)) {
           if (err.load()) return;
           std::this_thread::yield();
         }
@@ -367,9 +383,9 @@ struct Transfer {
 };
 }  // namespace
 
-static int move_host(picgpu_ctx *c, void *ring, const HostSeg *segs, int nsegs, size_t total, bool down) {
-  size_t fill = total / kSlots;
-  fill = fill < kMinFill ? kMinFill : fill > kSlotBytes ? kSlotBytes : fill;
+static int move_host(picgpu_ctx *c, void *ring, bool small, const HostSeg *segs, int nsegs, size_t total, bool down) {
+  size_t fill = total / kLargeRing.slots;
+  fill = small || fill < kMinFill ? kMinFill : fill > kSlotBytes ? kSlotBytes : fill;
   std::vector<std::thread> helpers;
   try {
     std::vector<Chunk> chunks;
@@ -391,9 +407,10 @@ static int move_host(picgpu_ctx *c, void *ring, const HostSeg *segs, int nsegs, 
     }
     std::unique_ptr<std::atomic<unsigned char>[]> done(new std::atomic<unsigned char>[groups.size()]);
     for (size_t k = 0; k < groups.size(); ++k) done[k].store(0);
-    Transfer t{c, static_cast<char *>(ring), segs, chunks, groups, done.get(), down};
+    const RingSize size = small ? kSmallRing : kLargeRing;
+    Transfer t{c, static_cast<char *>(ring), size, segs, chunks, groups, done.get(), down};
     if (down) t.issue();
-    const size_t want = total / kBytesPerThread;
+    const size_t want = small ? 0 : total / kBytesPerThread;
     const int nth = want < (size_t)kMaxThreads ? (int)want : kMaxThreads;
     try {
       helpers.reserve((size_t)nth);
@@ -459,10 +476,11 @@ static int host_transfer(picgpu_ctx *c, const HostSeg *segs, int nsegs, bool dow
   if (total == 0) return PICGPU_OK;
   for (hipEvent_t &e : c->transfer.ev)
     if (!e) PG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  const bool small = total < (down ? kSmallDown : kSmallUp);
   void *ring = nullptr;
-  if (take_ring(&ring) != PICGPU_OK) return move_pageable(c, segs, nsegs, down);
-  const int r = move_host(c, ring, segs, nsegs, total, down);
-  give_ring(ring);
+  if (take_ring(small, &ring) != PICGPU_OK) return move_pageable(c, segs, nsegs, down);
+  const int r = move_host(c, ring, small, segs, nsegs, total, down);
+  give_ring(small, ring);
   return r;
 }
 
