@@ -797,7 +797,7 @@ int picgpu_compute_metrics(picgpu_ctx *c, int *orientation) {
     set_error("no grid uploaded");
     return PICGPU_E_STATE;
   }
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   const NodeDims d = node_dims(c);
   const int64_t nn = d.count();
   auto &e = c->eul;
@@ -891,7 +891,7 @@ int picgpu_boundary_create(picgpu_ctx *c, const picgpu_boundary_config *bc) {
       return PICGPU_E_UNSUPPORTED;
     }
   }
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   c->eul.bc = *bc;
   c->eul.have_bc = true;
   PG_CHECK(run_boundaries(c, true));
@@ -902,7 +902,7 @@ int picgpu_boundary_create(picgpu_ctx *c, const picgpu_boundary_config *bc) {
 int picgpu_upload_ucont(picgpu_ctx *c, const double *ucont) {
   if (!c || !ucont) return PICGPU_E_ARG;
   PG_CHECK(need_metrics(c));
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_HIP(hipMemcpy(c->eul.ucont.ptr, ucont, sizeof(double) * 3 * (size_t)c->nnode, hipMemcpyHostToDevice));
   return PICGPU_OK;
 }
@@ -910,7 +910,7 @@ int picgpu_upload_ucont(picgpu_ctx *c, const double *ucont) {
 int picgpu_upload_ucont_device(picgpu_ctx *c, const double *d_ucont) {
   if (!c || !d_ucont) return PICGPU_E_ARG;
   PG_CHECK(need_metrics(c));
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_HIP(hipMemcpyAsync(c->eul.ucont.ptr, d_ucont, sizeof(double) * 3 * (size_t)c->nnode, hipMemcpyDeviceToDevice,
                         c->stream));
   PG_HIP(hipStreamSynchronize(c->stream));
@@ -920,7 +920,7 @@ int picgpu_upload_ucont_device(picgpu_ctx *c, const double *d_ucont) {
 int picgpu_set_initial_ucont(picgpu_ctx *c, int finit, const double uin[3]) {
   if (!c) return PICGPU_E_ARG;
   PG_CHECK(need_metrics(c));
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(run_initial_ucont(c, finit, uin));
   PG_HIP(hipStreamSynchronize(c->stream));
   return PICGPU_OK;
@@ -929,7 +929,7 @@ int picgpu_set_initial_ucont(picgpu_ctx *c, int finit, const double uin[3]) {
 int picgpu_boundary_execute(picgpu_ctx *c) {
   if (!c) return PICGPU_E_ARG;
   PG_CHECK(need_bc(c));
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(run_boundaries(c, false));
   PG_HIP(hipStreamSynchronize(c->stream));
   return PICGPU_OK;
@@ -938,14 +938,14 @@ int picgpu_boundary_execute(picgpu_ctx *c) {
 int picgpu_contra2cart(picgpu_ctx *c) {
   if (!c) return PICGPU_E_ARG;
   PG_CHECK(need_metrics(c));
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   return run_contra2cart(c);
 }
 
 int picgpu_set_eulerian_fields(picgpu_ctx *c, int64_t step, int64_t start_step, int finit, const double uin[3]) {
   if (!c) return PICGPU_E_ARG;
   PG_CHECK(need_bc(c));
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   if (step == start_step && start_step > 0) return PICGPU_OK;  // restart: fields were read (simulation.c:53-58)
   if (step == 0) PG_CHECK(run_initial_ucont(c, finit, uin));
   PG_CHECK(run_boundaries(c, false));

@@ -266,7 +266,7 @@ int picgpu_write_output(picgpu_ctx *c, const char *dir, int64_t step) {
     set_error("no grid uploaded");
     return PICGPU_E_STATE;
   }
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(settle_swarm(c));
   const int64_t n = c->n, nn = c->nnode;
   std::vector<double> buf((size_t)std::max<int64_t>(3 * n, 3 * nn));
@@ -485,7 +485,7 @@ int picgpu_write_vtk(picgpu_ctx *c, const char *prefix, int64_t step) {
     set_error("no grid uploaded");
     return PICGPU_E_STATE;
   }
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(settle_swarm(c));
   const int64_t nn = c->nnode, n = c->n;
   std::vector<double> coor((size_t)(3 * nn)), f((size_t)(3 * nn));

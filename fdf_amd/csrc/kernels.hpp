@@ -988,6 +988,50 @@ __global__ __launch_bounds__(kBlock) void k_sort_gather(const int32_t *__restric
   P2[d] = own.P;
 }
 
+// The same sort without memory for the records: the swarm moved to its
+// provisional slots (start given), each slot's rank among its cell's PIDs, and
+// the swarm moved to the ranks (start null).  What lies from *located on stays.
+template <typename R>
+__global__ __launch_bounds__(kBlock) void k_move_swarm(
+    int64_t n, const int32_t *__restrict__ start, const int32_t *__restrict__ rank, const double *__restrict__ pos,
+    const R *__restrict__ vel, const R *__restrict__ w, const int32_t *__restrict__ cell,
+    const int32_t *__restrict__ status, const int64_t *__restrict__ pid, const R *__restrict__ P,
+    double *__restrict__ pos2, R *__restrict__ vel2, R *__restrict__ w2, int32_t *__restrict__ cell2,
+    int32_t *__restrict__ status2, int64_t *__restrict__ pid2, R *__restrict__ P2) {
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= n) return;
+  const int32_t c = cell[p];
+  if (start && c < 0) return;
+  const int64_t q = (start ? (int64_t)start[c] : 0) + rank[p];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    pos2[3 * q + k] = pos[3 * p + k];
+    vel2[3 * q + k] = vel[3 * p + k];
+    w2[3 * q + k] = w[3 * p + k];
+  }
+  cell2[q] = c;
+  status2[q] = status[p];
+  pid2[q] = pid[p];
+  P2[q] = P[p];
+}
+static __global__ __launch_bounds__(kBlock) void k_pid_rank(int64_t n, const int32_t *__restrict__ located,
+                                                            const int32_t *__restrict__ start,
+                                                            const int32_t *__restrict__ cell,
+                                                            const int64_t *__restrict__ pid,
+                                                            int32_t *__restrict__ rank) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= n) return;
+  if (q >= *located) {
+    rank[q] = (int32_t)q;
+    return;
+  }
+  const int64_t id = pid[q];
+  const int32_t c = cell[q], s = start[c], e = start[c + 1];
+  int32_t r = 0;
+  for (int32_t t = s; t < e; ++t) r += (pid[t] < id || (pid[t] == id && t < q)) ? 1 : 0;
+  rank[q] = s + r;
+}
+
 // Neumaier-compensated accumulator of the P averages in FP32 (a cell's sum of
 // equal P values stays exact at any count); plain sum in FP64.
 template <typename R>

@@ -672,7 +672,7 @@ int picgpu_mlp_enable(picgpu_ctx *c, int on) {
 
 int picgpu_mlp_set_params(picgpu_ctx *c, const float *params) {
   if (!c || !params) return PICGPU_E_ARG;
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(set_norm_from_grid(c));
   return upload_params(c, params);
 }
@@ -683,7 +683,7 @@ int picgpu_mlp_get_params(picgpu_ctx *c, float *params) {
     set_error("MLP parameters not set");
     return PICGPU_E_STATE;
   }
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_HIP(hipStreamSynchronize(c->stream));
   PG_HIP(hipMemcpy(params, c->mlp_master.ptr, sizeof(float) * NP, hipMemcpyDeviceToHost));
   return PICGPU_OK;
@@ -696,7 +696,7 @@ int picgpu_mlp_forward(picgpu_ctx *c, int64_t n, const float *x, float *y) {
     return PICGPU_E_STATE;
   }
   if (n == 0) return PICGPU_OK;
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(c->mlp_x.ensure(sizeof(float) * 3 * (size_t)n));
   PG_CHECK(c->mlp_y.ensure(sizeof(float) * 3 * (size_t)n));
   PG_HIP(hipMemcpy(c->mlp_x.ptr, x, sizeof(float) * 3 * (size_t)n, hipMemcpyHostToDevice));
@@ -714,7 +714,7 @@ int picgpu_mlp_loss_grad(picgpu_ctx *c, int64_t n, const float *x, const float *
     set_error("MLP parameters not set");
     return PICGPU_E_STATE;
   }
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(ensure_mlp_buffers(c));
   PG_CHECK(c->mlp_x.ensure(sizeof(float) * 3 * (size_t)n));
   PG_CHECK(c->mlp_t.ensure(sizeof(float) * 3 * (size_t)n));
@@ -733,13 +733,13 @@ int picgpu_mlp_train(picgpu_ctx *c, int64_t max_pairs, int batch, int iters, flo
     set_error("mlp_train: bad arguments (batch must be a positive multiple of 32)");
     return PICGPU_E_ARG;
   }
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(settle_swarm(c));
   if (!c->have_grid || c->n == 0) {
     set_error("mlp_train: needs a grid and a located swarm");
     return PICGPU_E_STATE;
   }
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(set_norm_from_grid(c));
   PG_CHECK(ensure_mlp_buffers(c));
   if (!c->have_mlp) {
@@ -816,7 +816,7 @@ int picgpu_mlp_train(picgpu_ctx *c, int64_t max_pairs, int batch, int iters, flo
 int picgpu_mlp_guess(picgpu_ctx *c, int64_t n, const double *pos, int64_t *cell) {
   if (!c || n < 0 || (n > 0 && (!pos || !cell))) return PICGPU_E_ARG;
   if (n == 0) return PICGPU_OK;
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   DevBuf dp, dg;
   PG_CHECK(dp.ensure(sizeof(double) * 3 * (size_t)n));
   PG_CHECK(dg.ensure(sizeof(int32_t) * (size_t)n));

@@ -23,6 +23,24 @@ void set_error(const char *fmt, ...) {
   va_end(ap);
 }
 
+static thread_local picgpu_ctx *t_entered = nullptr;
+
+int enter(picgpu_ctx *c) {
+  t_entered = c;
+  PG_HIP(hipSetDevice(c->device));
+  return PICGPU_OK;
+}
+
+bool release_spares() {
+  picgpu_ctx *const c = t_entered;
+  if (!c || (!c->filter.ptr && !c->rec.ptr)) return false;
+  c->filter.release();  // (hipFree waits for the kernels that use them)
+  c->rec.release();
+  c->have_filter = false;
+  c->no_spares = true;
+  return true;
+}
+
 hipEvent_t take_event(picgpu_ctx *c) {
   if (!c->event_pool.empty()) {
     hipEvent_t e = c->event_pool.back();
@@ -190,7 +208,7 @@ static int finish_grid(picgpu_ctx *c) {
     c->bmax[a] = c->bmax[a] + c->opt.bbox_tolerance;
   }
   c->have_grid = true;
-  c->have_planes = c->have_filter = c->filter_no_memory = false;
+  c->have_planes = c->have_filter = c->filter_no_memory = c->no_spares = false;
   c->have_ucat = false;
   c->eul.have_metrics = c->eul.have_bc = false;
   c->sorted = c->keyed = c->key_ordered = c->compact_pending = false;
@@ -272,6 +290,7 @@ int picgpu_create(picgpu_ctx **out, const picgpu_options *opt) {
 int picgpu_destroy(picgpu_ctx *c) {
   if (!c) return PICGPU_OK;
   (void)hipSetDevice(c->device);
+  if (t_entered == c) t_entered = nullptr;
   (void)hipStreamSynchronize(c->stream);
   for (auto &r : c->pending) {
     (void)hipEventDestroy(r.a);
@@ -282,7 +301,7 @@ int picgpu_destroy(picgpu_ctx *c) {
                     &c->vel0, &c->cell_count, &c->cell_start, &c->pavg, &c->face[0], &c->face[1], &c->face[2],
                     &c->scan_tmp, &c->counters, &c->mlp_master, &c->mlp_bf16, &c->mlp_adam_m, &c->mlp_adam_v,
                     &c->mlp_grad, &c->mlp_partial, &c->mlp_x, &c->mlp_t, &c->mlp_y, &c->kcount,
-                    &c->kstart[0], &c->kstart[1], &c->kidx[0], &c->kidx[1], &c->kslot, &c->kbase, &c->planes, &c->filter,
+                    &c->kstart[0], &c->kstart[1], &c->kidx[0], &c->kidx[1], &c->kslot, &c->kbase, &c->planes, &c->filter, &c->rec,
                     &c->defer, &c->walk_hist};
   for (DevBuf *b : bufs) b->release();
   c->step_counters.release();
@@ -321,13 +340,13 @@ int picgpu_upload_grid(picgpu_ctx *c, int64_t IM, int64_t JM, int64_t KM, const 
     set_error("upload_grid: bad arguments");
     return PICGPU_E_ARG;
   }
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   if (!c->swarm_invalid) PG_CHECK(settle_swarm(c));  // the particles stay; the new grid drops their index
   if (IM * JM * KM >= (int64_t)INT32_MAX - 2 || (IM + 1) * (JM + 1) * (KM + 1) >= ((int64_t)1 << 40)) {
     set_error("upload_grid: grid too large for 32-bit packed cell indices");
     return PICGPU_E_UNSUPPORTED;
   }
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   c->IM = (int)IM;
   c->JM = (int)JM;
   c->KM = (int)KM;
@@ -343,13 +362,13 @@ int picgpu_upload_grid_device(picgpu_ctx *c, int64_t IM, int64_t JM, int64_t KM,
     set_error("upload_grid_device: bad arguments");
     return PICGPU_E_ARG;
   }
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   if (!c->swarm_invalid) PG_CHECK(settle_swarm(c));  // the particles stay; the new grid drops their index
   if (IM * JM * KM >= (int64_t)INT32_MAX - 2) {
     set_error("upload_grid_device: grid too large for 32-bit packed cell indices");
     return PICGPU_E_UNSUPPORTED;
   }
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   c->IM = (int)IM;
   c->JM = (int)JM;
   c->KM = (int)KM;
@@ -364,7 +383,7 @@ int picgpu_upload_grid_device(picgpu_ctx *c, int64_t IM, int64_t JM, int64_t KM,
 int picgpu_upload_ucat_device(picgpu_ctx *c, const double *d_ucat) {
   if (!c || !d_ucat) return PICGPU_E_ARG;
   PG_CHECK(need_grid(c));
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(c->ucat.ensure(c->rsize * 3 * (size_t)c->ncell));
   PG_CHECK(c->corner.ensure(c->rsize * 3 * (size_t)c->nnode));
   int r = dispatch_real(c, [&](auto *tag) -> int {
@@ -386,7 +405,7 @@ int picgpu_init_particles_device(picgpu_ctx *c, int64_t n, const double *d_pos, 
     set_error("init_particles_device: more than 2^31-1 particles");
     return PICGPU_E_UNSUPPORTED;
   }
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(ensure_swarm(c, c->sw, n));
   c->n = n;
   c->sorted = c->keyed = c->key_ordered = c->compact_pending = false;
@@ -409,7 +428,7 @@ int picgpu_init_particles_device(picgpu_ctx *c, int64_t n, const double *d_pos, 
 int picgpu_upload_ucat(picgpu_ctx *c, const double *ucat) {
   if (!c || !ucat) return PICGPU_E_ARG;
   PG_CHECK(need_grid(c));
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   const int64_t nx = c->IM + 1, ny = c->JM + 1;
   PG_CHECK(c->ucat.ensure(c->rsize * 3 * (size_t)c->ncell));
   PG_CHECK(c->corner.ensure(c->rsize * 3 * (size_t)c->nnode));
@@ -445,7 +464,7 @@ int picgpu_upload_particles(picgpu_ctx *c, int64_t n, const double *pos, const d
     set_error("upload_particles: more than 2^31-1 particles");
     return PICGPU_E_UNSUPPORTED;
   }
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(ensure_swarm(c, c->sw, n));
   c->n = n;
   c->sorted = c->keyed = c->key_ordered = c->compact_pending = false;
@@ -488,7 +507,7 @@ int picgpu_num_particles(picgpu_ctx *c, int64_t *n) {
 int picgpu_download_particles(picgpu_ctx *c, double *pos, double *vel, int64_t *cell, double *weight,
                               int64_t *status, int64_t *pid) {
   if (!c) return PICGPU_E_ARG;
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(settle_swarm(c));
   const int64_t n = c->n;
   if (n == 0) {
@@ -512,7 +531,7 @@ int picgpu_download_particles(picgpu_ctx *c, double *pos, double *vel, int64_t *
 
 int picgpu_download_walk_steps(picgpu_ctx *c, int32_t *steps) {
   if (!c || !steps) return PICGPU_E_ARG;
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(settle_swarm(c));
   if (!c->opt.collect_walk_stats || !c->walk_steps.ptr || c->walk_steps.bytes < sizeof(int32_t) * (size_t)c->n) {
     set_error("walk statistics not collected (collect_walk_stats=0 or no locate yet)");
@@ -559,11 +578,13 @@ static int ensure_planes(picgpu_ctx *c) {
 }
 
 // FP64: the FP32 records on which a locate decides the steps of its walks
-// (128 B per cell beside the FP64 records' 304), once per grid.  Without
-// memory for them every evaluation is made in FP64.
+// (128 B per cell beside the FP64 records' 304), once per grid; after the
+// call's other allocations.  Without memory for them every evaluation is made
+// in FP64.
 static int ensure_filter(picgpu_ctx *c) {
-  if (c->opt.precision == PICGPU_FP32 || c->have_filter || c->filter_no_memory || c->ncell == 0) return PICGPU_OK;
-  if (c->filter.ensure(sizeof(CellPlanes32) * (size_t)c->ncell) != PICGPU_OK) {
+  if (c->opt.precision == PICGPU_FP32 || c->have_filter || c->filter_no_memory || c->no_spares || c->ncell == 0)
+    return PICGPU_OK;
+  if (c->filter.ensure(sizeof(CellPlanes32) * (size_t)c->ncell, true) != PICGPU_OK) {
     c->filter_no_memory = true;
     return PICGPU_OK;
   }
@@ -573,7 +594,12 @@ static int ensure_filter(picgpu_ctx *c) {
   return PICGPU_OK;
 }
 
-static int build_key_index(picgpu_ctx *c, const int32_t *guess = nullptr, bool rec = false);
+// The records of a sort of n particles, after the call's other allocations.
+static bool have_records(picgpu_ctx *c, int64_t n) {
+  return !c->no_spares && c->rec.ensure(sizeof(SortRec<double>) * (size_t)(n > 0 ? n : 1), true) == PICGPU_OK;
+}
+
+static int build_key_index(picgpu_ctx *c, const int32_t *guess = nullptr, bool *rec = nullptr);
 
 // An FP64 locate of at least this many particles from guessed start cells
 // visits them grouped by start cell (tile-major key), so that neighbouring
@@ -589,7 +615,6 @@ static int do_locate(picgpu_ctx *c, int skip_lost) {
   PG_CHECK(need_grid(c));
   PG_CHECK(settle_swarm(c));
   PG_CHECK(ensure_planes(c));
-  PG_CHECK(ensure_filter(c));
   PG_CHECK(counters_reset(c));
   const int64_t n = c->n;
   if (n > 0) {
@@ -616,11 +641,12 @@ static int do_locate(picgpu_ctx *c, int skip_lost) {
       PG_CHECK(build_key_index(c, guess));
       if (c->n_live == n) order = c->kidx[c->kcur].as<int32_t>();
     }
+    unsigned long long *hist = hist_reset(c);
+    PG_CHECK(ensure_filter(c));
     const bool records = c->opt.precision == PICGPU_FP32 || c->have_filter;
     const bool from_origin = records && c->cells_unset && !guess;
     const int ahead = from_origin && std::max(c->IM, std::max(c->JM, c->KM)) >= kLocateLong ? locate_ahead(n) : 1;
     const bool lines = from_origin && n >= kLocateLines;
-    unsigned long long *hist = hist_reset(c);
     int r = dispatch_real(c, [&](auto *tag) -> int {
       using R = std::remove_pointer_t<decltype(tag)>;
       LocateArgs<R> a;
@@ -742,7 +768,19 @@ static int do_interp(picgpu_ctx *c) {
   });
 }
 
-// Counting sort by cell; particles without a cell go to a last bucket.
+// particle p of `from` to start[cell] + rank[p] of `to` (located ones), or to rank[p]
+template <typename R>
+static int move_swarm(picgpu_ctx *c, SwarmBufs &from, SwarmBufs &to, const int32_t *start) {
+  PG_LAUNCH(c, "move_swarm", nblocks(c->n), kBlock, k_move_swarm<R>, c->n, start, c->rank.as<int32_t>(),
+            from.pos.as<double>(), from.vel.as<R>(), from.w.as<R>(), from.cell.as<int32_t>(),
+            from.status.as<int32_t>(), from.pid.as<int64_t>(), from.P.as<R>(), to.pos.as<double>(), to.vel.as<R>(),
+            to.w.as<R>(), to.cell.as<int32_t>(), to.status.as<int32_t>(), to.pid.as<int64_t>(), to.P.as<R>());
+  return PICGPU_OK;
+}
+
+// Counting sort by cell; particles without a cell go to a last bucket.  Without
+// memory for the records, in two moves of the whole swarm: into the cells'
+// segments, and to the PIDs' ranks there.
 static int do_sort(picgpu_ctx *c) {
   PG_CHECK(settle_swarm(c));
   const int64_t n = c->n;
@@ -759,18 +797,18 @@ static int do_sort(picgpu_ctx *c) {
   }
   PG_CHECK(scan_exclusive_i32(c, c->cell_count.as<int32_t>(), c->cell_start.as<int32_t>(), c->ncell));
   if (n > 0) {
-    DevBuf &rec = c->pos0;  // the order under construction: pos0 holds nothing else here
-    PG_CHECK(rec.ensure(sizeof(SortRec<double>) * (size_t)n));
     const int32_t *start = c->cell_start.as<int32_t>();
+    const bool rec = have_records(c, n);
     int r = dispatch_real(c, [&](auto *tag) -> int {
       using R = std::remove_pointer_t<decltype(tag)>;
+      if (!rec) return move_swarm<R>(c, c->sw, c->alt, start);
       PG_LAUNCH(c, "slot_scatter", nblocks(n), kBlock, k_slot_scatter<R>, n, c->rank.as<int32_t>(), start,
                 c->sw.cell.as<int32_t>(), c->sw.pid.as<int64_t>(), c->sw.P.as<R>(), c->sw.status.as<int32_t>(),
-                rec.as<SortRec<R>>());
-      PG_LAUNCH(c, "sort_gather", nblocks(n), kBlock, k_sort_gather<R>, start + c->ncell, start, rec.as<SortRec<R>>(),
-                c->sw.pos.as<double>(), c->sw.vel.as<R>(), c->sw.w.as<R>(), c->alt.pos.as<double>(),
-                c->alt.vel.as<R>(), c->alt.w.as<R>(), c->alt.cell.as<int32_t>(), c->alt.status.as<int32_t>(),
-                c->alt.pid.as<int64_t>(), c->alt.P.as<R>());
+                c->rec.as<SortRec<R>>());
+      PG_LAUNCH(c, "sort_gather", nblocks(n), kBlock, k_sort_gather<R>, start + c->ncell, start,
+                c->rec.as<SortRec<R>>(), c->sw.pos.as<double>(), c->sw.vel.as<R>(), c->sw.w.as<R>(),
+                c->alt.pos.as<double>(), c->alt.vel.as<R>(), c->alt.w.as<R>(), c->alt.cell.as<int32_t>(),
+                c->alt.status.as<int32_t>(), c->alt.pid.as<int64_t>(), c->alt.P.as<R>());
       return PICGPU_OK;
     });
     PG_CHECK(r);
@@ -797,7 +835,17 @@ static int do_sort(picgpu_ctx *c) {
       });
       PG_CHECK(r2);
     }
-    swap_swarm(c);
+    if (rec) {
+      swap_swarm(c);
+    } else {
+      // the particles are in their cells' segments; from there to their ranks, back in sw
+      PG_LAUNCH(c, "pid_rank", nblocks(n), kBlock, k_pid_rank, n, start + c->ncell, start, c->alt.cell.as<int32_t>(),
+                c->alt.pid.as<int64_t>(), c->rank.as<int32_t>());
+      PG_CHECK(dispatch_real(c, [&](auto *tag) -> int {
+        return move_swarm<std::remove_pointer_t<decltype(tag)>>(c, c->alt, c->sw, nullptr);
+      }));
+      c->pid32_valid = false;
+    }
   }
   c->sorted = true;
   c->keyed = c->key_ordered = false;
@@ -890,8 +938,9 @@ static constexpr int kCompactEvery = 16;
 // key, the live ones without a cell in the last bucket, removed ones left out.
 // With guess, a particle without a cell is keyed by its guessed start cell
 // instead (the order of a fresh locate; not an index of the swarm).
-// rec: in pos0, with the particles' short fields, for compact_by_key.
-static int build_key_index(picgpu_ctx *c, const int32_t *guess, bool rec) {
+// rec: in c->rec, with the particles' short fields, for compact_by_key, if there
+// is memory for it after what the two allocate (*rec tells).
+static int build_key_index(picgpu_ctx *c, const int32_t *guess, bool *rec) {
   const TileMap tm = tile_map(c);
   const int64_t nkeys = ntiles(tm) * TS;
   const int64_t n = c->n;
@@ -907,6 +956,10 @@ static int build_key_index(picgpu_ctx *c, const int32_t *guess, bool rec) {
               c->sw.status.as<int32_t>(), guess, c->IM, c->JM, tm, (int32_t)nkeys, c->kcount.as<int32_t>(),
               c->kslot.as<int32_t>());
   PG_CHECK(scan_exclusive_i32(c, c->kcount.as<int32_t>(), c->kstart[cur].as<int32_t>(), nkeys + 1));
+  if (rec) {
+    PG_CHECK(ensure_swarm(c, c->alt, n));
+    *rec = have_records(c, n);
+  }
   if (n > 0)
     PG_CHECK(dispatch_real(c, [&](auto *tag) -> int {
       using R = std::remove_pointer_t<decltype(tag)>;
@@ -914,10 +967,10 @@ static int build_key_index(picgpu_ctx *c, const int32_t *guess, bool rec) {
         PG_LAUNCH(c, "key_scatter", nblocks(n), kBlock, (k_key_scatter<R, decltype(to_rec)::value>), n,
                   c->sw.cell.as<int32_t>(), c->sw.status.as<int32_t>(), guess, c->kslot.as<int32_t>(), c->IM, c->JM,
                   tm, (int32_t)nkeys, c->kstart[cur].as<int32_t>(), c->kidx[cur].as<int32_t>(),
-                  c->sw.pid.as<int64_t>(), c->sw.P.as<R>(), c->pos0.as<SortRec<R>>());
+                  c->sw.pid.as<int64_t>(), c->sw.P.as<R>(), c->rec.as<SortRec<R>>());
         return PICGPU_OK;
       };
-      return rec ? launch(std::true_type{}) : launch(std::false_type{});
+      return rec && *rec ? launch(std::true_type{}) : launch(std::false_type{});
     }));
   int32_t h[2] = {0, 0};
   PG_HIP(hipMemcpyAsync(h, c->kstart[cur].as<int32_t>() + nkeys, sizeof(h), hipMemcpyDeviceToHost, c->stream));
@@ -947,7 +1000,7 @@ static int compact_by_key(picgpu_ctx *c, int64_t live, int mode, const int32_t *
                   c->sw.pid.as<int64_t>(), c->sw.P.as<R>(), c->alt.pos.as<double>(), c->alt.vel.as<R>(),
                   c->alt.w.as<R>(), c->alt.cell.as<int32_t>(), c->alt.status.as<int32_t>(), c->alt.pid.as<int64_t>(),
                   c->alt.P.as<R>(), move32 ? c->sw.pid32.as<int32_t>() : (const int32_t *)nullptr,
-                  c->alt.pid32.as<int32_t>(), c->pos0.as<SortRec<R>>());
+                  c->alt.pid32.as<int32_t>(), c->rec.as<SortRec<R>>());
         return PICGPU_OK;
       };
       if (rec) return gather(std::true_type{}, std::true_type{});
@@ -1087,9 +1140,8 @@ static int do_step_fused(picgpu_ctx *c, double dt, unsigned flags, int step, boo
     // its short fields in records of 32 bytes, scattered with the order, where
     // there is memory for them (16.8M particles, FP32: scatter and gather 0.54 +
     // 2.54 -> 0.70 + 1.52 ms)
-    const bool rec = !c->key_ordered &&
-                     c->pos0.ensure(sizeof(SortRec<double>) * (size_t)(c->n > 0 ? c->n : 1)) == PICGPU_OK;
-    PG_CHECK(build_key_index(c, nullptr, rec));
+    bool rec = false;
+    PG_CHECK(build_key_index(c, nullptr, c->key_ordered ? nullptr : &rec));
     if (!c->key_ordered) PG_CHECK(compact_by_key(c, c->kend_unloc, GATHER_ALL, nullptr, true, rec));
   }
   const TileMap tm = tile_map(c);
@@ -1344,25 +1396,25 @@ extern "C" {
 
 int picgpu_reset_statuses(picgpu_ctx *c) {
   if (!c) return PICGPU_E_ARG;
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   return do_reset_advect(c, 0.0, 1, 0);
 }
 
 int picgpu_advect(picgpu_ctx *c, double dt) {
   if (!c) return PICGPU_E_ARG;
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   return do_reset_advect(c, dt, 0, 1);
 }
 
 int picgpu_locate(picgpu_ctx *c) {
   if (!c) return PICGPU_E_ARG;
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   return do_locate(c, 0);
 }
 
 int picgpu_remove_lost(picgpu_ctx *c, int64_t *removed) {
   if (!c) return PICGPU_E_ARG;
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   int64_t rl = 0;
   PG_CHECK(do_remove(c, 1, 0, &rl, nullptr));
   c->stats.removed_lost = rl;
@@ -1372,7 +1424,7 @@ int picgpu_remove_lost(picgpu_ctx *c, int64_t *removed) {
 
 int picgpu_remove_out_of_bounds(picgpu_ctx *c, int64_t *removed) {
   if (!c) return PICGPU_E_ARG;
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(need_grid(c));
   int64_t ro = 0;
   PG_CHECK(do_remove(c, 0, 1, nullptr, &ro));
@@ -1383,7 +1435,7 @@ int picgpu_remove_out_of_bounds(picgpu_ctx *c, int64_t *removed) {
 
 int picgpu_interpolate(picgpu_ctx *c) {
   if (!c) return PICGPU_E_ARG;
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(need_grid(c));
   PG_CHECK(do_center_to_corner(c));
   PG_CHECK(do_interp(c));
@@ -1393,7 +1445,7 @@ int picgpu_interpolate(picgpu_ctx *c) {
 
 int picgpu_scatter(picgpu_ctx *c) {
   if (!c) return PICGPU_E_ARG;
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(need_grid(c));
   PG_CHECK(do_sort(c));
   PG_CHECK(do_scatter_P(c));
@@ -1403,7 +1455,7 @@ int picgpu_scatter(picgpu_ctx *c) {
 
 int picgpu_deposit_faces(picgpu_ctx *c, double particle_volume) {
   if (!c) return PICGPU_E_ARG;
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(need_grid(c));
   if (!c->sorted) PG_CHECK(do_sort(c));
   c->particle_volume = particle_volume;
@@ -1423,7 +1475,7 @@ int picgpu_set_particle_volume(picgpu_ctx *c, double particle_volume) {
 
 int picgpu_step(picgpu_ctx *c, double dt, int nsteps, unsigned flags) {
   if (!c || nsteps < 0) return PICGPU_E_ARG;
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(need_grid(c));
   if (!c->have_ucat) {
     set_error("ucat not uploaded");
@@ -1504,7 +1556,7 @@ static int ensure_cell_counts(picgpu_ctx *c) {
 
 int picgpu_particle_count_summary(picgpu_ctx *c, double *total, double *max_count, int64_t *max_index) {
   if (!c || !total || !max_count || !max_index) return PICGPU_E_ARG;
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(need_grid(c));
   PG_CHECK(ensure_cell_counts(c));
   PG_CHECK(c->count_summary.ensure(2 * sizeof(unsigned long long)));
@@ -1524,7 +1576,7 @@ int picgpu_particle_count_summary(picgpu_ctx *c, double *total, double *max_coun
 
 int picgpu_interpolation_error(picgpu_ctx *c, int finit, double *percent) {
   if (!c || !percent || (finit != 0 && finit != 1)) return PICGPU_E_ARG;
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(settle_swarm(c));
   const int64_t n = c->n;
   const int64_t nb = std::max<int64_t>(1, std::min<int64_t>(nblocks(3 * n), 1024));
@@ -1551,7 +1603,7 @@ int picgpu_interpolation_error(picgpu_ctx *c, int finit, double *percent) {
 
 int picgpu_download_grid_field(picgpu_ctx *c, int which, double *out) {
   if (!c || !out) return PICGPU_E_ARG;
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(need_grid(c));
   auto get = [&](HostKind kind, const void *dev, int64_t count, int dir = 0) {
     const HostSeg seg{kind, const_cast<void *>(dev), out, count, 8, dir};

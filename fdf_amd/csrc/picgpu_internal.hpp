@@ -29,18 +29,32 @@ void set_error(const char *fmt, ...);
     if (_r != PICGPU_OK) return _r; \
   } while (0)
 
+// Every entry point that may allocate: makes the context's device current, and
+// its spare buffers those that the calling thread's allocations may take back.
+int enter(picgpu_ctx *c);
+// Spare buffers (picgpu_ctx::filter, rec) only make a call faster: they are
+// taken when the call has the memory that it needs, and given back where a
+// later allocation fails without.  False: there was none to give back.
+bool release_spares();
+
 // A device buffer that grows on demand.
 struct DevBuf {
   void *ptr = nullptr;
   size_t bytes = 0;
-  int ensure(size_t want) {
+  int ensure(size_t want, bool spare = false) {
     if (want <= bytes && ptr) return PICGPU_OK;
     if (ptr) (void)hipFree(ptr);
     ptr = nullptr;
     bytes = 0;
     if (want == 0) want = 256;
-    if (hipMalloc(&ptr, want) != hipSuccess) {
+    bool ok = hipMalloc(&ptr, want) == hipSuccess;
+    if (!ok && !spare && release_spares()) {
       (void)hipGetLastError();
+      ok = hipMalloc(&ptr, want) == hipSuccess;
+    }
+    if (!ok) {
+      (void)hipGetLastError();
+      ptr = nullptr;
       set_error("hipMalloc(%zu) failed", want);
       return PICGPU_E_NOMEM;
     }
@@ -120,8 +134,9 @@ struct picgpu_ctx {
   double bmin[3] = {0, 0, 0}, bmax[3] = {0, 0, 0};
   picgpu::DevBuf planes;  // [ncell] CellPlanes64 (FP64) or CellPlanes32 (FP32)
   bool have_planes = false;
-  picgpu::DevBuf filter;  // FP64: [ncell] CellPlanes32 for the walk steps of a locate
+  picgpu::DevBuf filter;  // spare, FP64: [ncell] CellPlanes32 for the walk steps of a locate
   bool have_filter = false, filter_no_memory = false;
+  bool no_spares = false;  // memory ran out: no spare buffers until the next grid
 
   // Eulerian fields
   bool have_ucat = false;
@@ -151,6 +166,7 @@ struct picgpu_ctx {
   picgpu::DevBuf walk_hist; // uint64 [kCounterStripes][PICGPU_WALK_HIST_BINS]
   picgpu::DevBuf guess;     // int32 [n] MLP start cell
   picgpu::DevBuf pos0, vel0;// RK2 saved state
+  picgpu::DevBuf rec;       // spare: [n] SortRec, the order under construction of a sort
   bool sorted = false;      // particles sorted by cell, cell_start valid
   bool cells_unset = false; // the particles have no cells yet: the next locate's walks start in cell (0,0,0)
   int64_t n_live = 0;       // particles not removed (equals n outside picgpu_step)

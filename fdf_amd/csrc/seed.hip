@@ -158,7 +158,7 @@ int picgpu_seed_particles(picgpu_ctx *c, int64_t n, int mode, int inlet_face, in
     set_error("no grid uploaded");
     return PICGPU_E_STATE;
   }
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   DevBuf tmp;
   int r = seed_positions(c, n, mode, inlet_face, seed, tmp);
   if (r == PICGPU_OK) r = picgpu_init_particles_device(c, n, tmp.as<double>(), pid_base);
@@ -173,7 +173,7 @@ int picgpu_reinit_on_inlet(picgpu_ctx *c, int inlet_face, int64_t seed) {
     set_error("no grid uploaded");
     return PICGPU_E_STATE;
   }
-  PG_HIP(hipSetDevice(c->device));
+  PG_CHECK(enter(c));
   PG_CHECK(settle_swarm(c));
   const int64_t n = c->n;
   DevBuf tmp;

@@ -62,6 +62,62 @@ def no_pinned(precision, n):
             assert x[k].tobytes() == y[k].tobytes(), k
 
 
+def _swarm(g, n, IM, JM, KM, fused):
+    """A swarm through the sort's consumers (or the fused steps), some of it
+    outside the grid; what the sort returns in its order, the steps' by PID."""
+    rng = np.random.default_rng(n)
+    pos = rng.random((n, 3)) * 1.04 - 0.02
+    g.upload_particles(pos, pid=rng.permutation(n).astype(np.int64), P=rng.random(n))
+    g.LocateAllParticlesInGrid()
+    g.InterpolateAllFieldsToSwarm()
+    if fused:
+        g.AdvanceSimulation(2e-4, 3, rk2=True, deposit_cells=True, deposit_faces=True)
+    else:
+        g.ScatterAllParticleFieldsToEulerFields()
+        g.DepositParticlesToFaces(1e-9)
+    d = g.download_particles()
+    if fused:
+        o = np.argsort(d["pid"], kind="stable")
+        d = {k: v[o] for k, v in d.items()}
+    d["fields"] = np.concatenate([g.field(w).reshape(-1) for w in range(9)])
+    return d
+
+
+def tight(precision, fused):
+    """Calls that take the sort's records and the FP64 filter where there is
+    memory do with what they need: a small swarm, which leaves room for them,
+    then a large one, which needs it back; the results are the same bits."""
+    fused, (IM, JM, KM) = fused == "fused", (24, 24, 40)
+    small, large = 5_000, 90_000
+    coor = W.perturbed_cube(IM, JM, KM, seed=3)
+    ucat = W.ucat_random_fourier(coor, IM, JM, KM, seed=3, nmodes=4)
+    spares = 32 * large + (128 * IM * JM * KM if precision == "fp64" else 0)
+
+    def run():
+        shim.shim_peak_reset()
+        with PicGpu(precision=precision) as g:
+            g.upload_grid(IM, JM, KM, coor)
+            g.upload_ucat(ucat)
+            return [_swarm(g, n, IM, JM, KM, fused) for n in (small, large)]
+
+    used = shim.shim_used()
+    want = run()
+    need = shim.shim_peak() - used - spares
+    shim.shim_limit(used + need)
+    got = run()
+    for x, y in zip(want, got):
+        for k in x:
+            assert x[k].tobytes() == y[k].tobytes(), k
+    shim.shim_limit(used + need - 1)  # and without that, the error that it always was
+    try:
+        run()
+    except L.PicgpuError as e:
+        assert "NOMEM" in str(e), e
+    else:
+        raise AssertionError("ran in less than it needs")
+    assert shim.shim_used() == used
+
+
 if __name__ == "__main__":
     globals()[sys.argv[2]](*sys.argv[3:])
     print("ok")

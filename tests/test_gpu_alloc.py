@@ -39,3 +39,9 @@ def test_pinned_slots_are_coherent(shim):
 @pytest.mark.parametrize("n", [1, (1 << 20) // 24, (1 << 20) // 24 + 1, (1 << 20) // 8 + 1])  # around a chunk's end
 def test_transfers_without_pinned_memory(shim, precision, n):
     _child(shim, "no_pinned", precision, n)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("how", ["stages", "fused"])
+def test_without_memory_for_records_and_filter(shim, precision, how):
+    _child(shim, "tight", precision, how)
