@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -223,6 +224,7 @@ struct picgpu_ctx {
   bool timing = false;
   std::string timing_only;  // when not empty: only kernels whose name starts with it are timed
   std::vector<picgpu::TimerRec> pending;
+  std::mutex timing_mu;  // the threads of a transfer time their launches too
   std::vector<hipEvent_t> event_pool;
   std::map<std::string, std::pair<double, int64_t>> timing_acc;
 

@@ -146,6 +146,21 @@ __global__ __launch_bounds__(kBlock) void k_fill_real(int64_t n, R v, R *__restr
   if (q < n) out[q] = v;
 }
 
+// times a chunk's launch from whichever thread of the transfer makes it
+struct ChunkTimer {
+  picgpu_ctx *c;
+  std::unique_lock<std::mutex> lock;
+  TimerRec rec;
+  ChunkTimer(picgpu_ctx *ctx, const char *name) : c(ctx) {
+    rec.a = rec.b = nullptr;
+    if (!c->timing) return;
+    lock = std::unique_lock<std::mutex>(c->timing_mu);
+    c->pending.reserve(c->pending.size() + 1);
+    timer_begin(c, name, rec);
+  }
+  ~ChunkTimer() { timer_end(c, rec); }
+};
+
 static int chunk_blocks(int64_t m, int per_thread, int most) {
   const int64_t b = (m + (int64_t)kBlock * per_thread - 1) / ((int64_t)kBlock * per_thread);
   return (int)(b < most ? b : most);
@@ -153,6 +168,7 @@ static int chunk_blocks(int64_t m, int per_thread, int most) {
 
 static hipError_t launch_pack(picgpu_ctx *c, const HostSeg &s, int64_t e0, int64_t m, void *slot) {
   auto go = [&](auto f) {
+    ChunkTimer timer(c, s.kind == HostKind::Volfrac ? "face_volfrac" : "host_pack");
     hipLaunchKernelGGL(k_pack<decltype(f)>, dim3(chunk_blocks(m, 2, kDownBlocks)), dim3(kBlock), 0, c->stream, e0, m,
                        f, static_cast<unsigned long long *>(slot));
     return hipGetLastError();
@@ -180,6 +196,7 @@ static hipError_t launch_pack(picgpu_ctx *c, const HostSeg &s, int64_t e0, int64
 
 static hipError_t launch_unpack(picgpu_ctx *c, const HostSeg &s, int64_t e0, int64_t m, const void *slot) {
   auto go = [&](auto f) {
+    ChunkTimer timer(c, "host_unpack");
     hipLaunchKernelGGL(k_unpack<decltype(f)>, dim3(chunk_blocks(m, 1, kUpBlocks)), dim3(kBlock), 0, c->stream, e0, m,
                        f, static_cast<const unsigned long long *>(slot));
     return hipGetLastError();
@@ -375,10 +392,14 @@ struct Transfer {
     }
   }
   void run() {
-    if (down)
-      run_down();
-    else
-      run_up();
+    try {
+      if (down)
+        run_down();
+      else
+        run_up();
+    } catch (...) {
+      (void)ok(hipErrorOutOfMemory);
+    }
   }
 };
 }  // namespace
