@@ -26,7 +26,8 @@ def train_from_walk(ctx: PicGpu, d: dict, n_pairs: int | None = None, iters: int
     still-LOST particles from the current network's guess and trains again
     on the enlarged set of walk-produced pairs.  With kernel_timing the
     training kernels are timed with HIP events and the result holds their
-    totals under "kernels" ({name: (total ms, launches)})."""
+    totals under "kernels" ({name: (total ms, launches)}; Adam's step is part
+    of mlp_reduce)."""
     n_pairs = int(n_pairs or d.get("train_pairs") or min(2_097_152, d["n"]))
     tmp = PicGpu(precision=ctx.precision)
     hist = []
@@ -64,7 +65,7 @@ def train_from_walk(ctx: PicGpu, d: dict, n_pairs: int | None = None, iters: int
         params = tmp.mlp_get_params()
         if kernel_timing:
             tmp.synchronize()
-            for k in ("mlp_fwd_bwd", "mlp_reduce", "mlp_adam", "mlp_guess"):
+            for k in ("mlp_fwd_bwd", "mlp_reduce", "mlp_guess"):
                 kernels[k] = tmp.timing_query(k)
     finally:
         tmp.close()
