@@ -1305,25 +1305,34 @@ static int finish_step_call(picgpu_ctx *c, unsigned flags, bool stored, bool las
 // A tile's workgroup pays the same chain of loads for 5 particles as for 500,
 // and four of them fit on a CU.  Where a tile holds few particles a lane a
 // particle over the index (k_step_list) is faster: it writes weights and
-// velocities, and the previous step's faces are a pass of their own.  The line,
-// from 16-step calls (us a step, tiles -> list):
-//   particles a cell              0.08         0.36-0.38     0.51         0.73-0.75    0.95
-//   128x128x192 FP32 RK2          191 -> 106   257 -> 203    274 -> 233   309 -> 307   344 -> 387
-//                    with faces   246 -> 177   301 -> 275    316 -> 307   350 -> 384   383 -> 476
-//   128x128x192 FP64 RK2          307 -> 180   412 -> 367    453 -> 425   535 -> 551   617 -> 690
-//                    with faces   436 -> 327   537 -> 515    580 -> 577   667 -> 707   746 -> 851
-//   61x45x131 FP32 with faces      60 ->  51                 74 ->  61    78 ->  68
-//   61x45x131 FP64 with faces      79 ->  64                 91 ->  86    99 ->  99
-// In a grid of up to kFewTiles tiles (a few rounds on the chip) the line with
-// faces lies where it does without.  Up to kFewParticles the list is faster at
-// any density (24x24x24: 30,000 58 -> 49 in FP32 with faces, 100,000 111 -> 95).
+// velocities, and the previous step's faces are a pass of their own.  Time of an
+// RK2 step, lists / tiles, in 16-step calls, the mean (lowest-highest) over grids:
+//   particles a cell          0.30            0.55            0.65            0.75             0.85
+//   up to kFewTiles tiles: 64x64x96, 61x45x131, 96x80x60, 96x96x100
+//     FP32              0.68 (.67-.68)  0.73 (.70-.76)  0.76 (.73-.79)  0.77 (.75-.82)  0.81 (.79-.87)
+//          with faces   0.80 (.79-.81)  0.85 (.83-.86)  0.87 (.85-.90)  0.89 (.87-.94)  0.93 (.90-.99)
+//     FP64              0.80 (.75-.85)  0.89 (.83-.94)  0.91 (.89-.96)  0.93 (.91-.98)  0.95 (.91-1.00)
+//          with faces   0.91 (.87-.94)  0.98 (.93-1.02) 1.00 (.98-1.01) 1.01 (1.00-1.02) 1.03 (1.00-1.05)
+//   more: 128x128x96, 128x128x192, 200x180x160
+//     FP32              0.72 (.70-.74)  0.86 (.81-.89)  0.92 (.88-.94)  0.97 (.91-1.01) 1.04 (.97-1.09)
+//          with faces   0.85 (.82-.88)  0.96 (.92-.99)  1.01 (.96-1.04) 1.06 (1.00-1.09) 1.13 (1.06-1.17)
+//     FP64              0.84 (.82-.85)  0.95 (.94-.96)  0.99 (.97-1.00) 1.02 (1.00-1.04) 1.06 (1.03-1.09)
+//          with faces   0.93 (.93-.93)  1.01 (.99-1.02) 1.04 (1.02-1.05) 1.06 (1.05-1.08) 1.11 (1.09-1.12)
+// In tubes of 27,000 to 1,300,000 cells at 0.75: FP32 0.68-0.82, with faces
+// 0.80-0.93; FP64 0.80-0.94, with faces 0.91-1.00.  At 0.45 the large grids with
+// faces are at 0.92 and 0.99.  Euler steps lie within 0.05 of RK2 ones.  Up to
+// kFewParticles the list is faster at any density (24x24x24, 2 to 5 a cell:
+// 0.61-0.89 in both precisions) but in long thin grids with faces in FP64
+// (20x20x280: 0.99-1.05).
 static constexpr int64_t kFewTiles = 4096, kFewParticles = 65536;
 static bool sparse_steps(const picgpu_ctx *c, unsigned flags) {
   if (flags & PICGPU_STEP_FACES_OF_START) return false;  // the faces that the tiles' last launch leaves
-  const bool faces = (flags & PICGPU_STEP_DEPOSIT_FACES) != 0;
+  const bool faces = (flags & PICGPU_STEP_DEPOSIT_FACES) != 0, fp32 = c->opt.precision == PICGPU_FP32;
   const int64_t n = live_particles(c);
   if (n <= kFewParticles) return true;
-  return faces && ntiles(tile_map(c)) > kFewTiles ? 2 * n < c->ncell : 4 * n < 3 * c->ncell;
+  // particles a cell, in twentieths
+  const int64_t line = ntiles(tile_map(c)) <= kFewTiles ? 15 : faces ? 10 : fp32 ? 15 : 12;
+  return 20 * n < line * c->ncell;
 }
 
 // Fused steps s0 .. s0 + nb - 1 of a call of nsteps: queued, then one read of
