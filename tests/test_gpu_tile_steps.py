@@ -103,3 +103,100 @@ def test_line_in_large_grids(precision, faces, line):
                          staged=staged)
                 out.append(_result(g, faces))
         _same(*out)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_crowded_tiles_with_fast_particles(oracle, precision):
+    """Tiles of over ten thousand particles, most of which change cell in a step:
+    queues and staged results overflow, walks are handed over and go on.  FP64:
+    also the oracle's particles bit for bit."""
+    from fdf_amd.swarm import PicGpu
+
+    print("[gpu-case] crowded tiles", precision, flush=True)
+    dims, n, nsteps = (16, 16, 8), 110_000, 3
+    coor = W.perturbed_cube(*dims, seed=31, amp=0.15)
+    ucat = W.ucat_random_fourier(coor, *dims, seed=32)
+    pos = 0.05 + 0.9 * np.random.default_rng(33).random((n, 3))
+    dt = 1.5 / (np.abs(ucat).max() * max(dims))  # up to about 1.5 cells a step
+    out = []
+    for staged in (False, True):
+        with PicGpu(precision=precision) as g:
+            _start(g, dims, coor, ucat, pos)
+            _advance(g, dt, nsteps, None if staged else True, rk2=True, deposit_cells=True, deposit_faces=True,
+                     staged=staged)
+            out.append(_result(g, True))
+    _same(*out)
+    if precision == "fp64":
+        corner = oracle.center_to_corner(*dims, ucat)
+        c, w, st, _ = oracle.locate(*dims, coor, pos, status=np.full(n, 4, np.int64))
+        s = {"pos": pos.copy(), "vel": oracle.interp(*dims, corner, c, w), "cell": c, "weight": w, "status": st,
+             "pid": np.arange(n, dtype=np.int64), "P": np.full(n, 101325.0)}
+        for _ in range(nsteps):
+            oracle.step(*dims, coor, corner, s, dt, rk2=True)
+        for k in ("pid", "cell", "pos", "vel", "weight", "status"):
+            assert np.array_equal(out[0][k], s[k]), k
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_long_call_matches_staged(precision):
+    """Twenty steps in one call, which compacts in its middle: the staged path's
+    particles, deposits, processed particles and walk iterations."""
+    from fdf_amd.swarm import PicGpu
+
+    print("[gpu-case] long tile call", precision, flush=True)
+    dims, n = (24, 20, 40), 160_000
+    coor, ucat, pos, dt, _ = _workload(dims, n, 7, 0.5)
+    out, st = [], []
+    for staged in (False, True):
+        with PicGpu(precision=precision) as g:
+            _start(g, dims, coor, ucat, pos)
+            _advance(g, dt, 20, None if staged else True, rk2=True, deposit_cells=True, deposit_faces=True,
+                     staged=staged)
+            out.append(_result(g, True))
+            st.append(g.stats())
+    _same(*out)
+    assert st[0]["particle_steps"] == st[1]["particle_steps"]
+    assert st[0]["walk_iterations"] == st[1]["walk_iterations"]
+    assert 0 < len(out[0]["pid"]) < n
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_single_step_calls_match_one_call_twice(precision):
+    """Twenty one-step calls, the compaction falling inside the sequence, give
+    what one twenty-step call gives, and that gives it again, bit for bit."""
+    from fdf_amd.swarm import PicGpu
+
+    print("[gpu-case] single tile steps", precision, flush=True)
+    dims, n = (16, 16, 8), 200_000
+    coor, ucat, pos, dt, _ = _workload(dims, n, 71, 0.3)
+    out = []
+    for calls in ([20], [1] * 20, [20]):
+        with PicGpu(precision=precision) as g:
+            _start(g, dims, coor, ucat, pos)
+            for k in calls:
+                _advance(g, dt, k, True, rk2=True, deposit_cells=True, deposit_faces=True)
+            live = g.n
+            out.append(_result(g, True))
+            assert live == len(out[-1]["pid"])
+    _same(out[0], out[1])
+    _same(out[0], out[2])
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_faces_of_start_in_sparse_grids(precision):
+    """With the faces of the last step's start the steps stay with the tiles at
+    any number of particles: the end state of a call without that option, and
+    the faces of one that ends a step before."""
+    from fdf_amd.swarm import PicGpu
+
+    print("[gpu-case] faces of start", precision, flush=True)
+    dims, n = (20, 18, 16), 3_000
+    coor, ucat, pos, dt, _ = _workload(dims, n, 9, 0.5)
+    out = []
+    for steps, kw, tiles in ((5, dict(faces_of_start=True), True), (5, {}, False), (4, {}, False)):
+        with PicGpu(precision=precision) as g:
+            _start(g, dims, coor, ucat, pos)
+            _advance(g, dt, steps, tiles, rk2=True, deposit_cells=True, deposit_faces=True, **kw)
+            out.append(_result(g, True))
+    for k in out[1]:
+        assert np.array_equal(out[0][k], out[2][k] if k.startswith("face") else out[1][k]), k
