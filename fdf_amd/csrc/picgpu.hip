@@ -1120,9 +1120,11 @@ static constexpr size_t kStepCounterWords = (size_t)kCounterStripes * C_NUM;
 // and the compaction schedule (every kCompactEvery steps) carries on.
 //
 // step: the step's number in the call; the first reads each particle's start
-// velocity from vel, later ones recompute it (unless the field is prepared
-// every step) and deposit the start state onto the faces, which is the
-// previous step's deposition (finish_step_call deposits the last one).
+// velocity from vel, later ones recompute it and deposit the start state onto
+// the faces, which is the previous step's deposition (finish_step_call deposits
+// the last one).  Where the field is prepared every step, and in sparse steps
+// (sparse), weights and velocities are carried from step to step instead, and
+// the faces are a pass of their own.
 // last: the call's last step, which compacts with weights and statuses if the
 // schedule falls on it.  counters: this step's counter block.  *compacted:
 // set when this step compacted the swarm.
@@ -1197,6 +1199,7 @@ static int do_step_fused(picgpu_ctx *c, double dt, unsigned flags, int step, boo
         if (fresh && u1 > u0)
           PG_LAUNCH(c, name_list, nblocks(u1 - u0), kBlock, (k_step_list<R, EX, RK, false>), a, idx, u0, u1,
                     (const int32_t *)nullptr);
+        // one launch for both, under the name of the seams where it has them
         const SeamCounts sc = dep ? seam_counts(c) : SeamCounts{0, 0, 0};
         if (dblocks + sc.total() > 0)
           PG_LAUNCH(c, sc.total() ? "face_seams" : "step_deferred", dblocks + nblocks(sc.total()), kBlock,
@@ -1256,7 +1259,8 @@ static int do_step_fused(picgpu_ctx *c, double dt, unsigned flags, int step, boo
     // weights and statuses move too; the live count is the new index's total
     // the FP64 steps recompute every start state: between the steps of a
     // call (and before the call's last pass writes them) weights and
-    // velocities are not read, unless the per-step field path carries them
+    // velocities are not read, unless the per-step field path or sparse steps
+    // carry them
     const bool move_vw = wu || c->opt.precision == PICGPU_FP32;
     PG_CHECK(compact_by_key(c, n, last ? GATHER_LAST : GATHER_STEP, nstart + nkeys + 1, move_vw));
     c->steps_since_compact = 0;

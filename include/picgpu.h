@@ -191,7 +191,8 @@ int picgpu_set_particle_volume(picgpu_ctx *ctx, double particle_volume);
  * call makes no hipMalloc, hipFree or allocating library call.  Calls that
  * overlap on one device race on that array.  The grid's face-plane records
  * must already exist (any picgpu_locate or picgpu_step on the grid builds
- * them): else PICGPU_E_STATE.  n above PICGPU_NOALLOC_MAX_PARTICLES:
+ * them; in PICGPU_FP64 contexts a picgpu_locate also those on which the walks
+ * are fastest, memory allowing): else PICGPU_E_STATE.  n above PICGPU_NOALLOC_MAX_PARTICLES:
  * PICGPU_E_ARG.  st NULL: the call returns once the kernels are queued on the
  * context's stream (picgpu_synchronize waits); st given: it waits and fills
  * located, lost, walk_iterations, walk_max, fp64_fallbacks, n_particles = n
