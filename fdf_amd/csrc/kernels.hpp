@@ -947,6 +947,17 @@ __global__ __launch_bounds__(kBlock) void k_slot_scatter(int64_t n, const int32_
   rec[(int64_t)start[c] + rank[p]] = SortRec<R>{(int32_t)p, c, pid[p], P[p], status[p]};
 }
 
+// lane t's value in every lane (t the same in all)
+template <typename V>
+__device__ __forceinline__ V lane_value(V v, int t) {
+  if constexpr (sizeof(V) == 4) {
+    return __builtin_bit_cast(V, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), t));
+  } else {
+    const int2 w = __builtin_bit_cast(int2, v);
+    return __builtin_bit_cast(V, make_int2(__builtin_amdgcn_readlane(w.x, t), __builtin_amdgcn_readlane(w.y, t)));
+  }
+}
+
 template <typename R>
 __global__ __launch_bounds__(kBlock) void k_sort_gather(const int32_t *__restrict__ located,
                                                         const int32_t *__restrict__ start,
