@@ -140,6 +140,14 @@ inline int64_t locate_blocks(int64_t n, int64_t chunk) {
   return (waves * 64 + kBlock - 1) / kBlock;
 }
 constexpr int kExactGroup = 24;
+// FP32: the lanes at a face that is not certified for which a wavefront leaves its
+// iterations.  They are few, and a lane that waits for others of its kind holds up
+// its own walk: of 24, as in FP64, and with the last ones left to the end of the
+// wavefront's walks, 16.8M out of cell (0,0,0) of a 128x128x1024 tube, the lines
+// in LDS 16.8 ms, without 19.0; of 2, 15.3 and 17.5 (17.6 with fallbacks in
+// place).  One at a time: 14.2 and 16.3, but 300,000 in a 48x48x250 tube 293 ->
+// 328 us and 2M in 24x24x24 cells 413 -> 456.
+constexpr int kFallbacks = 2;
 constexpr int kHeld = 2;      // full evaluations that took a walk on before it is taken on by them alone
 constexpr int kStopped = 16;  // lanes without a walk at which a wavefront turns to them
 
@@ -349,11 +357,11 @@ __global__ __launch_bounds__(kBlock, 4) void k_locate(LocateArgs<R> a) {
           if (eval && (!EXACT || recs)) decide(recs[lc]);
         }
         walking = __ballot(ph == kWalk);
-      } while (__popcll(walking) > least);
+      } while (__popcll(walking) > least && (EXACT || __popcll(__ballot(ph == kHold)) < kFallbacks));
     }
     const unsigned long long waiting = __ballot(ph == kHold);
     if ((walking | waiting) == 0ull && __ballot(ph != kIdle) == 0ull && cursor >= end) break;
-    if (waiting != 0ull && (walking == 0ull || __popcll(waiting) >= kExactGroup)) {
+    if (waiting != 0ull && (walking == 0ull || __popcll(waiting) >= (EXACT ? kExactGroup : kFallbacks))) {
       // the last walks of a wavefront that are certified nowhere (a point within
       // the filter's bound of a plane along the grid) stay here to their end
       const bool last = walking == 0ull && cursor >= end;
