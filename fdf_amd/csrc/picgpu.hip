@@ -1325,15 +1325,24 @@ static int finish_step_call(picgpu_ctx *c, unsigned flags, bool stored, bool las
 // In tubes of 27,000 to 1,300,000 cells at 0.75: FP32 0.68-0.82, with faces
 // 0.80-0.93; FP64 0.80-0.94, with faces 0.91-1.00.  At 0.45 the large grids with
 // faces are at 0.92 and 0.99.  Euler steps lie within 0.05 of RK2 ones.  Up to
-// kFewParticles the list is faster at any density (24x24x24, 2 to 5 a cell:
-// 0.61-0.89 in both precisions) but in long thin grids with faces in FP64
-// (20x20x280: 0.99-1.05).
-static constexpr int64_t kFewTiles = 4096, kFewParticles = 65536;
+// kFewParticles the list is faster at any density without faces, in grids of 8 to
+// 8,000 cells 0.25-0.99.  All keys of a one-cell grid count up one address: in
+// FP32 1.16-1.94 from 1,000 particles on, which leaves it to the tiles (FP64 0.80-0.92
+// with RK2, 1.01-1.18 with Euler steps).  With faces the list deposits from memory
+// what a tile sums in its LDS; lists / tiles (FP64, FP32):
+//   particles a cell    5             7             9             12            16
+//     4x4x40        0.95, 0.99    0.96, 1.02    0.99, 1.06    1.05, 1.13    1.09, 1.14
+//     8x8x8         0.87, 0.86    0.86, 1.01    0.99, 1.09    1.09, 1.25    1.08, 1.24
+//     12x12x12      0.78, 0.83    0.84, 0.96    0.90, 1.05    0.98, 1.23    1.01, 1.19
+//     16x16x16      0.82, 0.89    0.84, 0.97    0.98, 1.11    0.98, 1.12    0.95, 1.11
+// (24x24x24, 2 to 5 a cell: 0.61-0.89; 20x20x280 in FP64: 0.99-1.05; 6x6x6 with 300:
+// 1.20, 1.54; one cell with 65,000: 2.2, 2.4), hence up to kFewInCell.
+static constexpr int64_t kFewTiles = 4096, kFewParticles = 65536, kFewInCell = 7;
 static bool sparse_steps(const picgpu_ctx *c, unsigned flags) {
   if (flags & PICGPU_STEP_FACES_OF_START) return false;  // the faces that the tiles' last launch leaves
   const bool faces = (flags & PICGPU_STEP_DEPOSIT_FACES) != 0, fp32 = c->opt.precision == PICGPU_FP32;
   const int64_t n = live_particles(c);
-  if (n <= kFewParticles) return true;
+  if (n <= kFewParticles) return faces ? n <= kFewInCell * c->ncell : c->ncell > 1 || !fp32;
   // particles a cell, in twentieths
   const int64_t line = ntiles(tile_map(c)) <= kFewTiles ? 15 : faces ? 10 : fp32 ? 15 : 12;
   return 20 * n < line * c->ncell;

@@ -106,6 +106,30 @@ def test_line_in_large_grids(precision, faces, line):
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("dims,n,faces,tiles", [
+    ((5, 4, 3), 420, True, False), ((5, 4, 3), 421, True, True), ((5, 4, 3), 20_000, False, False),
+    ((24, 23, 17), 65_536, True, False), ((24, 23, 15), 65_536, True, True), ((1, 1, 1), 7, True, False),
+    ((1, 1, 1), 8, True, True), ((1, 1, 1), 3_000, False, None), ((2, 1, 1), 3_000, False, False)])
+def test_line_for_few_particles(precision, dims, n, faces, tiles):
+    """Up to 65,536 particles: the list with faces up to seven a cell, without
+    them always but in a single cell in FP32; the staged path's results."""
+    from fdf_amd.swarm import PicGpu
+
+    print("[gpu-case] few particles", precision, dims, n, faces, flush=True)
+    tiles = precision == "fp32" if tiles is None else tiles
+    coor, ucat, _, dt, _ = _workload(dims, 1, 4, 0.01)
+    pos = 0.1 + 0.8 * np.random.default_rng(n).random((n, 3))
+    out = []
+    for staged in (False, True):
+        with PicGpu(precision=precision) as g:
+            _start(g, dims, coor, ucat, pos)
+            _advance(g, dt, 2, None if staged else tiles, rk2=True, deposit_cells=True, deposit_faces=faces,
+                     staged=staged)
+            out.append(_result(g, faces))
+    _same(*out)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
 def test_crowded_tiles_with_fast_particles(oracle, precision):
     """Tiles of over ten thousand particles, most of which change cell in a step:
     queues and staged results overflow, walks are handed over and go on.  FP64:
