@@ -174,8 +174,9 @@ inline int locate_ahead(int64_t n) { return n <= kLocateWaves * 4 ? 16 : n <= kL
 //   300,000 FP32  274 /  341 / 287   461 /  428 / 379   839 /  756 / 722
 //   2M FP64       665 /  617 / 537  2107 / 1686 / 1574 3473 / 3026 / 2931
 //   2M FP32       640 /  629 / 576  2330 / 1772 / 1695 4180 / 3358 / 3170
-// 16.8M FP32 in a 128x128x1024 tube: 18.95 / 19.24 / 16.74 ms.  16 or 48 lanes in
-// place of 32 measure within 5 %.  Below the line the LDS gains less than it costs
+// 16.8M FP32 in a 128x128x1024 tube: 18.95 / 19.24 / 16.74 ms.  (FP32 with lanes that
+// wait for 24 uncertified faces; kFallbacks takes off up to 7 %, here 17.4 / - / 15.3.)
+// 16 or 48 lanes in place of 32 measure within 5 %.  Below the line the LDS gains less than it costs
 // where walks are short: 262,144 particles, own loads / 32 lanes, the tube 177 / 192
 // in FP32, the cubes 366 / 319 and 619 / 482; 140,000: 185 / 204, 297 / 308, 452 / 438.
 constexpr int64_t kLocateLines = 1 << 18;
